@@ -6,6 +6,7 @@
 // recorded for a fused "stream + boundaries + collide" pass.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <limits>
 #include <cstdarg>
@@ -91,10 +92,6 @@ struct lbm_context {
     int device = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev[8] = {};
-    // second stream (default priority) for 3D smoothed nodes run concurrently with the fused pass,
-    // forked from and joined back to `stream` by events
-    hipStream_t side_stream = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     bool concurrent_smoothing = true;  // lbm_context_set_concurrent_smoothing
     lbm_program *recording = nullptr;
     lbm_batch *batching = nullptr;  // between lbm_batch_begin and lbm_batch_end
@@ -136,7 +133,7 @@ struct lbm_lattice {
     std::vector<lbm_program *> hs_retired;  // earlier heat-source tables: graphs may still read them
     std::vector<int> hs_mask;
     std::vector<double> hs_qn;
-    Grid grid() const { return Grid{lx, ly, lz, N}; }
+    Grid grid() const { return lbm::make_grid(lx, ly, lz, N); }
 };
 
 struct HostOp {
@@ -159,24 +156,26 @@ struct lbm_program {
     // device tables
     bool uploaded = false;
     bool dev_used = false;  // device copies exist (a launch may still read them)
-    DevBuf d_slot_entry, d_entry_node, d_entry_ops, d_ops, d_sops, d_slot_list;
-    DevBuf d_side_of_slot, d_smoothed, d_side, d_side_nodes;  // corner smoothing from side states
-    DevBuf d_self;  // 3D smoothed nodes with face node indices (k_collide_smoothed_self)
-    int nentry = 0, nslot = 0, maxops = 0, n_smoothed = 0, smooth_stride = 1, n_side = 0, n_self = 0;
-    bool corner_block_ok = false;  // the corners may be done by the fused pass's last workgroup
+    DevBuf d_slot_entry, d_entry_node, d_entry_ops, d_ops, d_form_ops, d_list_ops, d_slot_list, d_place_list;
+    unsigned shared_places = 0, slot_places = 0;  // ProgView::shared, by_slot
+    DevBuf d_side_of_slot, d_smoothed, d_side;  // smoothing after the pass, from side states
+    DevBuf d_smooth_lanes;                      // 3D smoothing inside the pass (ProgView::smooth_lanes)
+    int nentry = 0, nslot = 0, maxops = 0, n_smoothed = 0, smooth_stride = 1, n_smooth_lanes = 0;
+    bool smooth_in_pass_ok = false;  // the smoothed nodes may be done by the fused pass's first workgroups
     bool owned_by_ctx = false;  // eager scratch program
     ~lbm_program() {
         d_slot_entry.release();
         d_entry_node.release();
         d_entry_ops.release();
         d_ops.release();
-        d_sops.release();
+        d_form_ops.release();
+        d_list_ops.release();
         d_slot_list.release();
+        d_place_list.release();
         d_side_of_slot.release();
         d_smoothed.release();
-        d_self.release();
         d_side.release();
-        d_side_nodes.release();
+        d_smooth_lanes.release();
     }
 };
 
@@ -348,6 +347,54 @@ int prog_record_smooth(lbm_program *P, lbm_lattice *L) {
     return LBM_OK;
 }
 
+// The words of a node's operators, and the values they read (program.h): an operator takes its
+// values from the list's first or second set where they agree with what is there, else from the
+// recorded operator.
+lbm::ListVals pack_list(const Op *o, int count, uint32_t *words) {
+    lbm::ListVals v{};
+    bool have_a[4] = {}, have_b[2][2] = {};
+    for (int t = 0; t < count; ++t) {
+        const lbm::OpIn in = lbm::op_in(o[t]);
+        const int code = o[t].code;
+        bool a[4] = {}, b[2] = {};  // the values this operator reads
+        uint32_t arg = 0, src = lbm::kFromList;
+        switch (code) {
+        case lbm::OP_NS_SET_U:
+        case lbm::OP_NS_SET_RHO: a[0] = a[1] = a[2] = true; break;
+        case lbm::OP_ANS_ISET_U: a[0] = a[1] = a[2] = a[3] = true; arg = o[t].arg ? 1 : 0; break;
+        case lbm::OP_AD_SET_T: b[0] = true; break;
+        case lbm::OP_AD_SET_Q: b[0] = b[1] = true; break;
+        case lbm::OP_AAD_ISET_Q: b[1] = true; break;
+        case lbm::OP_AAD_ISET_RHO: b[1] = true; arg = o[t].arg & 3u; break;
+        case lbm::OP_BOUNCE:
+        case lbm::OP_IBOUNCE: arg = o[t].arg & 3u; break;
+        default: break;
+        }
+        auto same = [](double x, double y) { return memcmp(&x, &y, sizeof x) == 0; };
+        bool fits = true;
+        for (int c = 0; c < 4; ++c) fits &= !a[c] || !have_a[c] || same(v.a[c], in.a[c]);
+        for (uint32_t k = 0; k < 2 && src == lbm::kFromList; ++k) {
+            bool ok = fits;
+            for (int c = 0; c < 2; ++c) ok &= !b[c] || !have_b[k][c] || same(v.b[k][c], in.b[c]);
+            if (!ok) continue;
+            for (int c = 0; c < 2; ++c)
+                if (b[c]) {
+                    v.b[k][c] = in.b[c];
+                    have_b[k][c] = true;
+                }
+            src = k;
+        }
+        if (src != lbm::kFromList)
+            for (int c = 0; c < 4; ++c)
+                if (a[c]) {
+                    v.a[c] = in.a[c];
+                    have_a[c] = true;
+                }
+        words[t] = lbm::op_word((uint32_t)code, o[t].face, o[t].lat, o[t].fset, arg, src);
+    }
+    return v;
+}
+
 int prog_upload(lbm_program *P) {
     if (P->uploaded) return LBM_OK;
     lbm_lattice *L = P->lat[0];
@@ -357,15 +404,20 @@ int prog_upload(lbm_program *P) {
     if (cap != hipStreamCaptureStatusNone)
         return fail(LBM_ERR_STATE, "a program's first use is inside a graph capture: use it once before capturing");
     // group operators by node, keeping record order within a node
-    std::map<int, std::vector<int>> by_node;
-    for (size_t t = 0; t < P->ops.size(); ++t) by_node[P->ops[t].node].push_back((int)t);
+    std::vector<int> order(P->ops.size());
+    for (size_t t = 0; t < order.size(); ++t) order[t] = (int)t;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return P->ops[x].node < P->ops[y].node; });
     std::vector<int> entry_node;
     std::vector<int2> entry_ops;
     std::vector<Op> ops;
-    for (auto &kv : by_node) {
-        entry_node.push_back(kv.first);
-        entry_ops.push_back(make_int2((int)ops.size(), (int)kv.second.size()));
-        for (int t : kv.second) ops.push_back(P->ops[t].op);
+    ops.reserve(order.size());
+    for (int t : order) {
+        if (entry_node.empty() || entry_node.back() != P->ops[t].node) {
+            entry_node.push_back(P->ops[t].node);
+            entry_ops.push_back(make_int2((int)ops.size(), 0));
+        }
+        ops.push_back(P->ops[t].op);
+        entry_ops.back().y++;
     }
     P->nentry = (int)entry_node.size();
     P->nslot = lbm::boundary_slot_count(L->lx, L->ly, L->lz, L->nd);
@@ -377,38 +429,73 @@ int prog_upload(lbm_program *P) {
         if (s < 0) return fail(LBM_ERR_STATE, "boundary operator on an interior node");
         slot_entry[s] = e;
     }
-    // operator lists for the fused kernels: each boundary slot's operators, OP_NONE-padded to maxops,
-    // stored once per distinct list (a face's nodes mostly share theirs), slot -> list index
+    // operator lists for the fused kernels: lists are stored once per distinct one (a face's nodes
+    // mostly share theirs), forms once per distinct sequence of operator words
     int most = 0;
     for (const int2 &r : entry_ops) most = std::max(most, r.y);
-    P->maxops = (most + lbm::kOpBatch - 1) / lbm::kOpBatch * lbm::kOpBatch;
-    std::vector<Op> sops;
-    std::vector<int> slot_list(P->nslot, -1);
-    std::map<std::string, int> list_of;
+    P->maxops = most;
+    std::vector<Op> list_ops;
+    std::vector<uint32_t> form_ops;
+    std::vector<lbm::NodeList> slot_list(P->nslot, lbm::NodeList{-1, -1, 0, 0, {0, 0}, {}});
+    std::map<std::string, int> form_of, list_of;
     std::vector<Op> one(P->maxops);
+    std::vector<uint32_t> words(P->maxops);
+    auto key_of = [](const auto &v) { return std::string(reinterpret_cast<const char *>(v.data()), v.size() * sizeof v[0]); };
+    int last = -1;  // the slot before with operators: a face's nodes follow each other and mostly share theirs
     for (int s = 0; s < P->nslot; ++s) {
         int e = slot_entry[s];
         if (e < 0) continue;
-        std::fill(one.begin(), one.end(), Op{});
-        for (int t = 0; t < entry_ops[e].y; ++t) one[t] = ops[entry_ops[e].x + t];
-        // the list's operator count rides in its first operator, so a node stops after its own
-        // batches (0 when it does not fit a byte: the kernels then walk all maxops)
-        one[0].pad[0] = entry_ops[e].y <= 255 ? (uint8_t)entry_ops[e].y : 0;
-        std::string key(reinterpret_cast<const char *>(one.data()), one.size() * sizeof(Op));
-        auto it = list_of.find(key);
-        if (it == list_of.end()) {
-            it = list_of.emplace(std::move(key), (int)(sops.size() / P->maxops)).first;
-            sops.insert(sops.end(), one.begin(), one.end());
+        const int before = last;
+        last = s;
+        if (before >= 0) {
+            const int2 x = entry_ops[slot_entry[before]], y = entry_ops[e];
+            if (x.y == y.y && !memcmp(&ops[x.x], &ops[y.x], y.y * sizeof(Op))) {
+                slot_list[s] = slot_list[before];
+                continue;
+            }
         }
-        slot_list[s] = it->second;
+        std::fill(one.begin(), one.end(), Op{});
+        std::fill(words.begin(), words.end(), 0u);
+        const int count = entry_ops[e].y;
+        for (int t = 0; t < count; ++t) one[t] = ops[entry_ops[e].x + t];
+        const lbm::ListVals vals = pack_list(one.data(), count, words.data());
+        auto l = list_of.emplace(key_of(one), (int)list_of.size());
+        if (l.second) list_ops.insert(list_ops.end(), one.begin(), one.end());
+        auto f = form_of.emplace(key_of(words), (int)form_of.size());
+        if (f.second) form_ops.insert(form_ops.end(), words.begin(), words.end());
+        lbm::NodeList so{l.first->second, f.first->second, count, 0, {0, 0}, vals};
+        for (int t = 0; t < std::min(count, lbm::kWordOps); ++t) so.w[t / 4] |= (uint64_t)words[t] << (16 * (t % 4));
+        slot_list[s] = so;
     }
-    // Smoothed nodes are done from their inward face neighbours' post-boundary states.  2D corners:
-    // by the fused pass's last workgroup or, when the boundary operators read arrays the collide
-    // saves, by a kernel after the pass from states the pass stores in a side buffer.  3D edges and
-    // corners: always by that kernel after the pass (k_collide_smoothed, two int4 per node).
-    std::vector<int> side_of_slot, side_nodes;
-    std::vector<int4> sm_ents, self_ents;
-    P->corner_block_ok = false;
+    // places whose nodes share one list (or have none), and places that have several
+    std::vector<lbm::NodeList> place_list(lbm::kPlaces, lbm::NodeList{-1, -1, 0, 0, {0, 0}, {}});
+    unsigned seen = 0;
+    P->shared_places = P->slot_places = 0;
+    for (int k = 0; k < L->lz; ++k)
+        for (int j = 0; j < L->ly; ++j) {
+            const bool whole = j == 0 || j == L->ly - 1 || (L->nd == 3 && (k == 0 || k == L->lz - 1));
+            for (int i = 0; i < L->lx; i += (whole || i == L->lx - 1) ? 1 : L->lx - 1) {
+                const int s = lbm::boundary_slot(i, j, k, L->lx, L->ly, L->lz, L->nd);
+                if (s < 0 || s >= P->nslot) continue;
+                const int at = lbm::place_of(i, j, k, L->lx, L->ly, L->lz, L->nd);
+                if (!(seen >> at & 1u)) {
+                    seen |= 1u << at;
+                    place_list[at] = slot_list[s];
+                    if (slot_list[s].list >= 0) P->shared_places |= 1u << at;
+                } else if (slot_list[s].list != place_list[at].list) {
+                    P->slot_places |= 1u << at;
+                }
+            }
+        }
+    P->shared_places &= ~P->slot_places;
+    // Smoothed nodes are done from their inward face neighbours' post-boundary states: by the fused
+    // pass's first workgroups or, when the boundary operators read arrays the collide saves, by a
+    // kernel after the pass from states the pass stores in a side buffer (k_collide_smoothed, one
+    // int4 per 2D corner, two per 3D node).
+    std::vector<int> side_of_slot;
+    std::vector<int4> sm_ents;
+    std::vector<int2> lanes;
+    P->smooth_in_pass_ok = false;
     P->smooth_stride = L->nd == 3 ? 2 : 1;
     const bool any_smoothed = P->smoothed[0] || P->smoothed[1];
     std::map<int, int> side;
@@ -420,36 +507,19 @@ int prog_upload(lbm_program *P) {
         return id;
     };
     if (any_smoothed && L->nd == 3) {
-        // edge node -> side states of its two inward face neighbours (axis order)
-        std::map<int, int2> edge_sides;
+        // edge node -> its two inward face neighbours (axis order), and their side states
+        std::map<int, int2> edge_nodes, edge_sides;
         for (const int4 &e : L->sm_edge) {
             if (e.x < 0 || e.x >= L->N || e.y < 0 || e.y >= L->N || e.z < 0 || e.z >= L->N ||
                 nboundary(L, e.y) != 1 || nboundary(L, e.z) != 1)
                 return fail(LBM_ERR_STATE, "a smoothed edge node's neighbour is not a face node");
             int2 ab = make_int2(side_id(e.y), side_id(e.z));
             edge_sides[e.x] = ab;
+            edge_nodes[e.x] = make_int2(e.y, e.z);
             sm_ents.push_back(make_int4(e.x, ab.x, ab.y, -1));
             sm_ents.push_back(make_int4(-1, -1, -1, -1));
         }
-        // Concurrent form (k_collide_smoothed_self): the edge nodes beside a corner publish their
-        // smoothed state in an LDS slot of workgroup 0, where the corners read it; they and the
-        // corners come first, the other edge nodes after them.
-        std::map<int, int> edge_slot;
-        for (const int4 &e : L->sm_corner)
-            for (int nb : {e.y, e.z, e.w})
-                if (edge_slot.find(nb) == edge_slot.end()) {
-                    const int id = (int)edge_slot.size();
-                    edge_slot[nb] = id;
-                }
-        if ((int)edge_slot.size() > lbm::kCornerEdgeSlots)
-            return fail(LBM_ERR_STATE, "too many edge nodes beside the corners");
-        std::vector<int4> rest;
-        for (const int4 &e : L->sm_edge) {
-            auto it = edge_slot.find(e.x);
-            std::vector<int4> &dst = it != edge_slot.end() ? self_ents : rest;
-            dst.push_back(make_int4(e.x, e.y, e.z, it != edge_slot.end() ? it->second : -1));
-            dst.push_back(make_int4(-1, -1, -1, -1));
-        }
+        // lanes of the pass's smoothing workgroups: a wavefront per corner (8 lanes of it), then 4 per edge node
         for (const int4 &e : L->sm_corner) {  // (corner, x-, y-, z-neighbour): three edge nodes
             auto ex = edge_sides.find(e.y), ey = edge_sides.find(e.z), ez = edge_sides.find(e.w);
             if (e.x < 0 || e.x >= L->N || e.w < 0 || ex == edge_sides.end() || ey == edge_sides.end() ||
@@ -457,27 +527,45 @@ int prog_upload(lbm_program *P) {
                 return fail(LBM_ERR_STATE, "a smoothed corner's neighbour is not an edge node");
             sm_ents.push_back(make_int4(e.x, ex->second.x, ex->second.y, -1));
             sm_ents.push_back(make_int4(ey->second.x, ey->second.y, ez->second.x, ez->second.y));
-            self_ents.push_back(make_int4(e.x, -1, -1, -1));
-            self_ents.push_back(make_int4(edge_slot.at(e.y), edge_slot.at(e.z), edge_slot.at(e.w), 1));
+            for (int nb : {e.y, e.z, e.w}) {
+                lanes.push_back(make_int2(edge_nodes.at(nb).x, -1));
+                lanes.push_back(make_int2(edge_nodes.at(nb).y, -1));
+            }
+            lanes.push_back(make_int2(e.x, e.x));
+            lanes.push_back(make_int2(e.x, -1));
+            lanes.resize((lanes.size() + 63) / 64 * 64, make_int2(-1, -1));
         }
-        if (self_ents.size() / 2 > (size_t)lbm::kSmoothedGroup)
-            return fail(LBM_ERR_STATE, "the corners and their edge nodes do not fit one workgroup");
-        self_ents.insert(self_ents.end(), rest.begin(), rest.end());
+        if (lanes.size() != (size_t)lbm::kCornerLanes) return fail(LBM_ERR_STATE, "a 3D grid has eight corners");
+        // edge line by edge line: a wavefront's lanes then have few different operator lists
+        std::vector<int4> edges = L->sm_edge;
+        auto line_of = [&](const int4 &e) {
+            int c[3], n[3] = {L->lx, L->ly, L->lz}, key = 0;
+            node_coords(L, e.x, c[0], c[1], c[2]);
+            for (int ax = 0; ax < 3; ++ax) key = 3 * key + (c[ax] == 0 ? 0 : (c[ax] == n[ax] - 1 ? 1 : 2));
+            return key;
+        };
+        std::stable_sort(edges.begin(), edges.end(),
+                         [&](const int4 &x, const int4 &y) { return line_of(x) < line_of(y); });
+        for (const int4 &e : edges) {
+            lanes.push_back(make_int2(e.y, -1));
+            lanes.push_back(make_int2(e.z, -1));
+            lanes.push_back(make_int2(e.x, e.x));
+            lanes.push_back(make_int2(e.x, -1));
+        }
+        P->smooth_in_pass_ok = true;
     } else if (any_smoothed && L->nd == 2) {
         const int smoothed_bits = (P->smoothed[0] ? 1 : 0) | (P->smoothed[1] ? 2 : 0);
         for (const int4 &e : L->sm_corner) {
             int a = side_id(e.y), b = side_id(e.z);
             sm_ents.push_back(make_int4(e.x, a, b, smoothed_bits));
         }
-        side_nodes.assign(side.size(), 0);
-        for (auto &kv : side) side_nodes[kv.second] = kv.first;
-        // The corner workgroup gives a corner, per lattice, either the neighbours' mean (smoothed)
-        // or its own pull + operators: exact when no operator at a corner reads the other lattice.
+        // A smoothing lane gives a corner, per lattice, either the neighbours' mean (smoothed) or its
+        // own pull + operators: exact when no operator at a corner reads the other lattice.
         bool cross = false;
         for (const int4 &e : L->sm_corner)
             for (const HostOp &h : P->ops)
                 if (h.node == e.x && h.op.code == lbm::OP_AAD_ISET_RHO) cross = true;
-        P->corner_block_ok = !cross && (int)side.size() <= lbm::kMaxSide && sm_ents.size() + side.size() <= 256;
+        P->smooth_in_pass_ok = !cross && L->sm_corner.size() == 4;
     }
     if (any_smoothed) {
         side_of_slot.assign(P->nslot, -1);
@@ -502,14 +590,14 @@ int prog_upload(lbm_program *P) {
     if ((rc = up(P->d_entry_node, entry_node.data(), entry_node.size() * sizeof(int)))) return rc;
     if ((rc = up(P->d_entry_ops, entry_ops.data(), entry_ops.size() * sizeof(int2)))) return rc;
     if ((rc = up(P->d_ops, ops.data(), ops.size() * sizeof(Op)))) return rc;
-    if ((rc = up(P->d_sops, sops.data(), sops.size() * sizeof(Op)))) return rc;
-    if ((rc = up(P->d_slot_list, slot_list.data(), slot_list.size() * sizeof(int)))) return rc;
+    if ((rc = up(P->d_form_ops, form_ops.data(), form_ops.size() * sizeof(uint32_t)))) return rc;
+    if ((rc = up(P->d_place_list, place_list.data(), place_list.size() * sizeof(lbm::NodeList)))) return rc;
+    if ((rc = up(P->d_list_ops, list_ops.data(), list_ops.size() * sizeof(Op)))) return rc;
+    if ((rc = up(P->d_slot_list, slot_list.data(), slot_list.size() * sizeof(lbm::NodeList)))) return rc;
     if ((rc = up(P->d_side_of_slot, side_of_slot.data(), side_of_slot.size() * sizeof(int)))) return rc;
     if ((rc = up(P->d_smoothed, sm_ents.data(), sm_ents.size() * sizeof(int4)))) return rc;
-    if ((rc = up(P->d_self, self_ents.data(), self_ents.size() * sizeof(int4)))) return rc;
-    P->n_self = (int)self_ents.size() / 2;
-    if ((rc = up(P->d_side_nodes, side_nodes.data(), side_nodes.size() * sizeof(int)))) return rc;
-    P->n_side = (int)side_nodes.size();
+    if ((rc = up(P->d_smooth_lanes, lanes.data(), lanes.size() * sizeof(int2)))) return rc;
+    P->n_smooth_lanes = (int)lanes.size();
     P->uploaded = true;
     P->dev_used = true;
     return LBM_OK;
@@ -521,14 +609,32 @@ ProgView prog_view(const lbm_program *P) {
     v.entry_node = (const int *)P->d_entry_node.p;
     v.entry_ops = (const int2 *)P->d_entry_ops.p;
     v.ops = (const Op *)P->d_ops.p;
-    v.sops = (const Op *)P->d_sops.p;
-    v.slot_list = (const int *)P->d_slot_list.p;
+    v.place_list = (const lbm::NodeList *)P->d_place_list.p;
+    v.shared = P->shared_places;
+    v.by_slot = P->slot_places;
+    v.slot_list = (const lbm::NodeList *)P->d_slot_list.p;
+    v.list_ops = (const Op *)P->d_list_ops.p;
+    v.form_ops = (const uint32_t *)P->d_form_ops.p;
     v.maxops = P->maxops;
     v.side_of_slot = P->n_smoothed > 0 ? (const int *)P->d_side_of_slot.p : nullptr;
     v.side = P->n_smoothed > 0 ? (double *)P->d_side.p : nullptr;
     v.nentry = P->nentry;
     v.nslot = P->nslot;
-    for (size_t k = 0; k < P->fsets.size() && k < (size_t)lbm::kMaxFieldSets; ++k) v.fs[k] = P->fsets[k];
+    // merge the sets that do not contradict each other (bindings may have changed since the last launch)
+    const double *FieldSet::*const names[] = {&FieldSet::rho, &FieldSet::ux,  &FieldSet::uy,
+                                              &FieldSet::uz,  &FieldSet::tem, &FieldSet::diff};
+    for (size_t k = 0; k < P->fsets.size() && k < (size_t)lbm::kMaxFieldSets; ++k) {
+        const FieldSet &f = v.fs[k] = P->fsets[k];
+        bool agree = true;
+        for (auto m : names) agree &= !(f.*m && v.fm.*m && f.*m != v.fm.*m);
+        if (agree) {
+            for (auto m : names)
+                if (f.*m) v.fm.*m = f.*m;
+            v.fmerged |= 1u << k;
+        }
+        if (f.diff) v.has_diff |= 1u << k;
+    }
+    if (P->fsets.empty()) v.fmerged = 1u;  // operators that read no field carry set 0
     return v;
 }
 
@@ -662,35 +768,22 @@ int collide_call(lbm_program *P, lbm_lattice *p, lbm_lattice *q, std::initialize
     cl.smoothed = (const int4 *)P->d_smoothed.p;
     cl.n_smoothed = P->n_smoothed;
     cl.smooth_stride = P->smooth_stride;
-    // The smoothed nodes may be done concurrently with the pass (2D: its corner workgroup; 3D: a
-    // kernel on the second stream) only when no field an operator reads is one the collide writes:
-    // both rebuild the neighbours' post-boundary states while the pass collides those neighbours.
+    // The smoothed nodes may be done inside the pass only when no field an operator reads is one the
+    // collide writes: their lanes rebuild the neighbours' post-boundary states while other lanes
+    // collide those neighbours.
     bool alias = false;
     if (P->n_smoothed > 0)
         for (const FieldSet &fs : P->fsets)
             for (const double *r : {fs.rho, fs.ux, fs.uy, fs.uz, fs.tem, fs.diff})
                 for (const double *w : saved) alias |= (r != nullptr && r == w);
-    if (P->n_self > 0 && !alias && !sink && P->ctx->concurrent_smoothing) {
-        cl.self_ents = (const int4 *)P->d_self.p;
-        cl.n_self = P->n_self;
-        cl.self_stream = P->ctx->side_stream;
-        cl.ev_fork = P->ctx->ev_fork;
-        cl.ev_join = P->ctx->ev_join;
+    const bool wanted = p->nd == 2 || (!sink && P->ctx->concurrent_smoothing);
+    if (P->n_smoothed > 0 && P->smooth_in_pass_ok && !alias && wanted) {
+        v.smooth_bits = (P->smoothed[0] ? 1 : 0) | (P->smoothed[1] ? 2 : 0);
+        v.nsmooth = p->nd == 2 ? 4 * 64 : P->n_smooth_lanes;
+        v.smooth_lanes = (const int2 *)P->d_smooth_lanes.p;
         v.side_of_slot = nullptr;
         v.side = nullptr;
         cl.n_smoothed = 0;
-    }
-    if (P->corner_block_ok && P->n_smoothed > 0) {
-        if (!alias) {
-            v.corner_block = 1;
-            v.nside = P->n_side;
-            v.ncorner = P->n_smoothed;
-            v.side_nodes = (const int *)P->d_side_nodes.p;
-            v.corners = (const int4 *)P->d_smoothed.p;
-            v.side_of_slot = nullptr;
-            v.side = nullptr;
-            cl.n_smoothed = 0;
-        }
     }
     cl.any_smooth = (P->smoothed[0] || P->smoothed[1]) ? 1 : 0;
     if (sink) {
@@ -783,9 +876,6 @@ int lbm_context_create(int device, lbm_context **out) {
         return fail(LBM_ERR_HIP, "hipStreamCreate: %s", hipGetErrorString(e));
     }
     for (auto &ev : C->ev) HIPCHK(hipEventCreate(&ev));
-    HIPCHK(hipStreamCreateWithFlags(&C->side_stream, hipStreamNonBlocking));
-    HIPCHK(hipEventCreateWithFlags(&C->ev_fork, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&C->ev_join, hipEventDisableTiming));
     HIPCHK(hipMalloc(&C->d_part, sizeof(double) * 2 * lbm::reduction_blocks()));
     HIPCHK(hipMalloc(&C->d_out, sizeof(double) * 4));
     HIPCHK(hipHostMalloc(&C->h_out, sizeof(double) * 4, hipHostMallocDefault));
@@ -807,10 +897,6 @@ int lbm_context_destroy(lbm_context *C) {
     (void)hipSetDevice(C->device);
     (void)hipStreamSynchronize(C->stream);
     for (auto &ev : C->ev) (void)hipEventDestroy(ev);
-    if (C->side_stream) (void)hipStreamSynchronize(C->side_stream);
-    if (C->ev_fork) (void)hipEventDestroy(C->ev_fork);
-    if (C->ev_join) (void)hipEventDestroy(C->ev_join);
-    if (C->side_stream) (void)hipStreamDestroy(C->side_stream);
     (void)hipFree(C->d_part);
     (void)hipFree(C->d_out);
     (void)hipHostFree(C->h_out);
@@ -1767,10 +1853,11 @@ static int batch_retile(lbm_batch *B) {
         if (B->rows > 1) {  // tiles of (block / rows) x rows nodes per (x, y) plane, as fused_block maps them
             const int4 d = k.dims[i];
             const int tw = B->block / B->rows;
-            nb = ((d.x + tw - 1) / tw) * ((d.y + B->rows - 1) / B->rows) * d.z + k.corner[i];
+            nb = ((d.x + tw - 1) / tw) * ((d.y + B->rows - 1) / B->rows) * d.z;
         } else {
-            nb = (k.nodes[i] + B->block - 1) / B->block + k.corner[i];
+            nb = (k.nodes[i] + B->block - 1) / B->block;
         }
+        nb += (k.smooth[i] + B->block - 1) / B->block;
         t[i] = make_int2(start, nb);
         start += (nb + 7) & ~7;  // instances start on multiples of 8 workgroups (one per XCD)
     }

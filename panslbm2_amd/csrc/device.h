@@ -10,13 +10,13 @@
 namespace lbm {
 
 // Fused steps collected for one batched launch (k_collide_batch): the items' bytes, per item its
-// node count and corner workgroup, and the launcher of the one kernel instantiation they share.
+// node count and smoothing lanes, and the launcher of the one kernel instantiation they share.
 struct BatchSink {
     using LaunchFn = hipError_t (*)(const void *items, const int2 *tiles, const int *active, int nitem,
                                     int nblocks_total, int block, int xcd, int rows, hipStream_t s);
     std::vector<unsigned char> bytes;
     size_t item_size = 0;
-    std::vector<int> nodes, corner;
+    std::vector<int> nodes, smooth;
     std::vector<int4> dims;  // (nx, ny, nz) of each instance
     LaunchFn launch = nullptr;
 };
@@ -33,10 +33,6 @@ struct CollideLaunch {
     const int4 *smoothed;      // smoothed nodes done after the fused pass from the side states it saved:
     int n_smoothed;            // smooth_stride int4 per node (2D corners 1, 3D edges and corners 2;
     int smooth_stride;         // layout at k_collide_smoothed)
-    const int4 *self_ents;     // 3D smoothed nodes run concurrently with the pass on self_stream
-    int n_self;                // (k_collide_smoothed_self; 0: not used), forked and joined with
-    hipStream_t self_stream;   // ev_fork / ev_join
-    hipEvent_t ev_fork, ev_join;
     int any_smooth;
     BatchSink *batch;          // non-null: collect the fused step instead of launching it
 };
@@ -79,6 +75,14 @@ hipError_t launch_stream(int kind, int prec, const void *src, void *dst, Grid g,
 hipError_t launch_smooth(int kind, int prec, void *f, int N, const int4 *list, int count, const Enc &e, hipStream_t s);
 hipError_t launch_program_apply(int ka, int kb, int prec, void *a, void *b, int N, const ProgView &pv, int seg,
                                 const Enc &ea, const Enc &eb, hipStream_t s);
+struct ApplyLaunch {  // launch_program_apply's arguments, for the instantiations in apply_*.hip
+    int ka, kb;
+    void *a, *b;
+    int N, seg;
+    Enc ea, eb;
+    hipStream_t stream;
+};
+template <int ND, int P> hipError_t program_apply_nd(const ApplyLaunch &al, const ProgView &pv);
 template <int ND, int P> hipError_t ns_collide_nd(const CollideLaunch &cl, const NSArgs &a);
 template <int ND, int P> hipError_t ad_collide_nd(const CollideLaunch &cl, const ADArgs &a);
 template <int ND, int P> hipError_t ans_collide_nd(const CollideLaunch &cl, const ANSArgs &a);

@@ -1,7 +1,7 @@
 // panslbm2_amd/csrc/device.hip -- HIP kernels for gfx950 other than the collides (streaming,
 // eager boundary programs, corner smoothing, initial conditions, sensitivities, reductions,
 // filters) and their typed launchers.  The collide kernels live in collide.h and are launched
-// from collide_{ns,ad,ans,aad}.hip.
+// from collide_{ns,ad,ans,aad}.hip; the eager boundary programs live in apply.h (apply_*.hip).
 #include "collide.h"
 
 namespace lbm {
@@ -21,28 +21,6 @@ __global__ void __launch_bounds__(kBlock) k_stream(const S *__restrict__ src, S 
     double f[L::nc];
     load_pull<L>(src, g, i, j, k, n, pull, f, e);
     store_node<L>(dst, g.N, n, f, e);
-}
-
-// ------------------------------------------------------------------------------------------
-// Boundary program, applied in place: one thread per boundary node runs that node's operators of
-// segment `seg` in call order (segments are separated by SmoothCorner calls).
-// ------------------------------------------------------------------------------------------
-template <class LA, class LB, class S>
-__global__ void __launch_bounds__(kBlock) k_program_apply(S *a, S *b, int N, ProgView pv, int seg, Enc ea, Enc eb) {
-    int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= pv.nentry) return;
-    int n = pv.entry_node[e];
-    int2 r = pv.entry_ops[e];
-    double fa[LA::nc], fb[LB::nc > 0 ? LB::nc : 1];
-    load_node<LA>(a, N, n, fa, ea);
-    load_node<LB>(b, N, n, fb, eb);
-    NodeFieldCache fc = prefetch_fields(pv, n);
-    for (int t = r.x; t < r.x + r.y; ++t) {
-        Op op = pv.ops[t];
-        if (op.code != OP_SMOOTH && (int)op.seg == seg) apply_op<LA, LB>(op, fa, fb, pv, n, fc);
-    }
-    store_node<LA>(a, N, n, fa, ea);
-    store_node<LB>(b, N, n, fb, eb);
 }
 
 // Corner / edge smoothing in place, d2q9.h:577-587, d3q15.h:1241-1303.  Entry = (node, nb0,
@@ -521,30 +499,20 @@ hipError_t launch_smooth(int kind, int prec, void *f, int N, const int4 *list, i
     });
 }
 
+static bool is_3d_kind(int k) { return k == kD3Q15 || k == kD3Q7 || k == kD3Q27; }
 hipError_t launch_program_apply(int ka, int kb, int prec, void *a, void *b, int N, const ProgView &pv, int seg,
                                 const Enc &ea, const Enc &eb, hipStream_t s) {
     if (pv.nentry == 0) return hipSuccess;
-    return dispatch_pair(ka, kb, [&](auto la, auto lb) {
-        using LA = decltype(la);
-        using LB = decltype(lb);
-        if (prec == kF64)
-            LBM_LAUNCH((k_program_apply<LA, LB, double>), nblocks(pv.nentry), s, static_cast<double *>(a),
-                       static_cast<double *>(b), N, pv, seg, ea, eb);
-        else if (prec == kF32)
-            LBM_LAUNCH((k_program_apply<LA, LB, float>), nblocks(pv.nentry), s, static_cast<float *>(a),
-                       static_cast<float *>(b), N, pv, seg, ea, eb);
-        else if (prec == kF16)
-            LBM_LAUNCH((k_program_apply<LA, LB, _Float16>), nblocks(pv.nentry), s, static_cast<_Float16 *>(a),
-                       static_cast<_Float16 *>(b), N, pv, seg, ea, eb);
-        else
-            return hipErrorInvalidValue;
-        return hipGetLastError();
-    });
+    const ApplyLaunch al{ka, kb, a, b, N, seg, ea, eb, s};
+    const bool d3 = is_3d_kind(ka);
+    if (prec == kF64) return d3 ? program_apply_nd<3, kF64>(al, pv) : program_apply_nd<2, kF64>(al, pv);
+    if (prec == kF32) return d3 ? program_apply_nd<3, kF32>(al, pv) : program_apply_nd<2, kF32>(al, pv);
+    if (prec == kF16) return d3 ? program_apply_nd<3, kF16>(al, pv) : program_apply_nd<2, kF16>(al, pv);
+    return hipErrorInvalidValue;
 }
 
 // collides: by the dimension of the first lattice (kinds D2Q9/D2Q5 are 2D, D3Q15/D3Q7/D3Q27 3D)
 // and the storage precision
-static bool is_3d_kind(int k) { return k == kD3Q15 || k == kD3Q7 || k == kD3Q27; }
 #define LBM_COLLIDE_DISPATCH(eq, cl, a)                                                                          \
     (cl.prec == kF64   ? (is_3d_kind(cl.ka) ? eq##_collide_nd<3, kF64>(cl, a) : eq##_collide_nd<2, kF64>(cl, a)) \
      : cl.prec == kF32 ? (is_3d_kind(cl.ka) ? eq##_collide_nd<3, kF32>(cl, a) : eq##_collide_nd<2, kF32>(cl, a)) \

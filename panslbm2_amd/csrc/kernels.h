@@ -2,7 +2,7 @@
 // corner-smoothing and collide kernels.
 //
 // A node's post-stream state is pulled from the source buffer (periodic wrap as in d2q9.h:80-84),
-// then the node's boundary operators run in call order.  Kernels that own smoothed nodes
+// then the node's boundary operators run in call order.  The lanes that own smoothed nodes
 // (SmoothCorner) rebuild the neighbours' states the same way and average them.
 #pragma once
 #include "bc2d.h"
@@ -81,12 +81,12 @@ struct NodeFields {
 };
 __device__ __forceinline__ NodeFields load_fields(const FieldSet &s, int n) {
     NodeFields v;
-    v.rho = s.rho ? s.rho[n] : 0.0;
-    v.ux = s.ux ? s.ux[n] : 0.0;
-    v.uy = s.uy ? s.uy[n] : 0.0;
-    v.uz = s.uz ? s.uz[n] : 0.0;
-    v.tem = s.tem ? s.tem[n] : 0.0;
-    v.diff = s.diff ? s.diff[n] : 0.0;
+    v.rho = s.rho ? gat(s.rho, n) : 0.0;
+    v.ux = s.ux ? gat(s.ux, n) : 0.0;
+    v.uy = s.uy ? gat(s.uy, n) : 0.0;
+    v.uz = s.uz ? gat(s.uz, n) : 0.0;
+    v.tem = s.tem ? gat(s.tem, n) : 0.0;
+    v.diff = s.diff ? gat(s.diff, n) : 0.0;
     v.has_diff = s.diff != nullptr;
     return v;
 }
@@ -94,51 +94,53 @@ __device__ __forceinline__ NodeFields load_fields(const FieldSet &s, int n) {
 // Apply one boundary operator to lattice L's populations `f`; `o` holds the other lattice's
 // populations (lattice LO), read by the coupled adjoint pressure operator.
 template <class L, class LO>
-__device__ __forceinline__ void apply_on(const Op &op, double *f, const double *o, const NodeFields &s) {
+__device__ __forceinline__ void apply_on(const OpWord &op, const OpIn &q, double *f, const double *o,
+                                         const NodeFields &s) {
+    const int face = (int)op.face, arg = (int)op.arg;
     switch (op.code) {
-    case OP_BOUNCE: bounce<L, false>(f, op.face, op.arg); break;
-    case OP_IBOUNCE: bounce<L, true>(f, op.face, op.arg); break;
+    case OP_BOUNCE: bounce<L, false>(f, face, arg); break;
+    case OP_IBOUNCE: bounce<L, true>(f, face, arg); break;
     case OP_NS_SET_U:
-        if constexpr (L::kind == kD2Q9) ns_set_u_2d(f, op.face, op.v[0], op.v[1]);
+        if constexpr (L::kind == kD2Q9) ns_set_u_2d(f, face, q.a[0], q.a[1]);
         else if constexpr (L::kind == kD3Q15 || L::kind == kD3Q27)
-            ns_set_u_3d<L>(f, op.face, op.v[0], op.v[1], op.v[2]);
+            ns_set_u_3d<L>(f, face, q.a[0], q.a[1], q.a[2]);
         break;
     case OP_NS_SET_RHO:
-        if constexpr (L::kind == kD2Q9) ns_set_rho_2d(f, op.face, op.v[0], op.v[1]);
+        if constexpr (L::kind == kD2Q9) ns_set_rho_2d(f, face, q.a[0], q.a[1]);
         else if constexpr (L::kind == kD3Q15 || L::kind == kD3Q27)
-            ns_set_rho_3d<L>(f, op.face, op.v[0], op.v[1], op.v[2]);
+            ns_set_rho_3d<L>(f, face, q.a[0], q.a[1], q.a[2]);
         break;
     case OP_AD_SET_T:  // (the host rejects advection-diffusion operators on D3Q27)
-        if constexpr (L::nd == 2) ad_set_t_2d<L>(f, op.face, op.v[0], s.ux, s.uy);
-        else if constexpr (L::nd == 3 && L::kind != kD3Q27) ad_set_t_3d<L>(f, op.face, op.v[0], s.ux, s.uy, s.uz);
+        if constexpr (L::nd == 2) ad_set_t_2d<L>(f, face, q.b[0], s.ux, s.uy);
+        else if constexpr (L::nd == 3 && L::kind != kD3Q27) ad_set_t_3d<L>(f, face, q.b[0], s.ux, s.uy, s.uz);
         break;
     case OP_AD_SET_Q: {
-        double d = s.has_diff ? s.diff : op.v[1];
-        if constexpr (L::nd == 2) ad_set_q_2d<L>(f, op.face, op.v[0], s.ux, s.uy, d);
-        else if constexpr (L::nd == 3 && L::kind != kD3Q27) ad_set_q_3d<L>(f, op.face, op.v[0], s.ux, s.uy, s.uz, d);
+        double d = s.has_diff ? s.diff : q.b[1];
+        if constexpr (L::nd == 2) ad_set_q_2d<L>(f, face, q.b[0], s.ux, s.uy, d);
+        else if constexpr (L::nd == 3 && L::kind != kD3Q27) ad_set_q_3d<L>(f, face, q.b[0], s.ux, s.uy, s.uz, d);
     } break;
     case OP_ANS_ISET_U:
-        if constexpr (L::kind == kD2Q9) ans_iset_u_2d(f, op.face, op.v[0], op.v[1], op.v3, op.arg);
+        if constexpr (L::kind == kD2Q9) ans_iset_u_2d(f, face, q.a[0], q.a[1], q.a[3], arg);
         else if constexpr (L::kind == kD3Q15 || L::kind == kD3Q27)
-            ans_iset_u_3d<L>(f, op.face, op.v[0], op.v[1], op.v[2], op.v3);
+            ans_iset_u_3d<L>(f, face, q.a[0], q.a[1], q.a[2], q.a[3]);
         break;
     case OP_ANS_ISET_RHO:
-        if constexpr (L::kind == kD2Q9) ans_iset_rho_2d(f, op.face);
-        else if constexpr (L::kind == kD3Q15 || L::kind == kD3Q27) ans_iset_rho_3d<L>(f, op.face);
+        if constexpr (L::kind == kD2Q9) ans_iset_rho_2d(f, face);
+        else if constexpr (L::kind == kD3Q15 || L::kind == kD3Q27) ans_iset_rho_3d<L>(f, face);
         break;
     case OP_AAD_ISET_T:
-        if constexpr (L::nd == 2) aad_iset_t_2d<L>(f, op.face, s.ux, s.uy);
-        else if constexpr (L::nd == 3 && L::kind != kD3Q27) aad_iset_t_3d<L>(f, op.face, s.ux, s.uy, s.uz);
+        if constexpr (L::nd == 2) aad_iset_t_2d<L>(f, face, s.ux, s.uy);
+        else if constexpr (L::nd == 3 && L::kind != kD3Q27) aad_iset_t_3d<L>(f, face, s.ux, s.uy, s.uz);
         break;
     case OP_AAD_ISET_Q:
-        if constexpr (L::nd == 2) aad_iset_q_2d<L>(f, op.face, s.ux, s.uy, op.v3);
-        else if constexpr (L::nd == 3 && L::kind != kD3Q27) aad_iset_q_3d<L>(f, op.face, s.ux, s.uy, s.uz, op.v3);
+        if constexpr (L::nd == 2) aad_iset_q_2d<L>(f, face, s.ux, s.uy, q.b[1]);
+        else if constexpr (L::nd == 3 && L::kind != kD3Q27) aad_iset_q_3d<L>(f, face, s.ux, s.uy, s.uz, q.b[1]);
         break;
     case OP_AAD_ISET_RHO:
         if constexpr (L::kind == kD2Q9 && LO::nd == 2)
-            aad_iset_rho_2d<LO>(f, o, op.face, op.arg, s.rho, s.ux, s.uy, s.tem, op.v3);
+            aad_iset_rho_2d<LO>(f, o, face, arg, s.rho, s.ux, s.uy, s.tem, q.b[1]);
         else if constexpr (L::kind == kD3Q15 && LO::nd == 3)
-            aad_iset_rho_3d<LO>(f, o, op.face, op.arg, s.rho, s.ux, s.uy, s.uz, s.tem, op.v3);
+            aad_iset_rho_3d<LO>(f, o, face, arg, s.rho, s.ux, s.uy, s.uz, s.tem, q.b[1]);
         break;
     default: break;
     }
@@ -151,53 +153,103 @@ __device__ __forceinline__ FieldSet field_set(const ProgView &pv, int k) {
     return k == 0 ? pv.fs[0] : (k == 1 ? pv.fs[1] : (k == 2 ? pv.fs[2] : pv.fs[3]));
 }
 
-// The field sets a node's operators read most often (0 and 1) are loaded once per node, with the
-// operators; operators on sets 2 and 3 load theirs at use.
-struct NodeFieldCache {
-    NodeFields f0, f1;
+// pre: the merged set's fields (pv.fm) at node n; a set outside it is loaded at use.
+template <class LA, class LB>
+__device__ __forceinline__ void apply_op(const OpWord &op, const OpIn &q, double *a, double *b, const ProgView &pv,
+                                         int n, const NodeFields &pre) {
+    NodeFields s = pre;
+    if (!((pv.fmerged >> op.fset) & 1u)) s = load_fields(field_set(pv, (int)op.fset), n);
+    s.has_diff = (pv.has_diff >> op.fset) & 1u;
+    if (((int)op.lat ^ pv.latswap) == 0) apply_on<LA, LB>(op, q, a, b, s);
+    else if constexpr (LB::nc > 0) apply_on<LB, LA>(op, q, b, a, s);
+}
+// What node n needs for its boundary operators: its list with the values, and the fields of the merged
+// set.  The fused kernels load it before the node's pull, so that the operators wait for no memory
+// of their own.
+struct NodeOps {
+    NodeList o;
+    NodeFields f;
 };
-__device__ __forceinline__ NodeFieldCache prefetch_fields(const ProgView &pv, int n) {
-    return NodeFieldCache{load_fields(pv.fs[0], n), load_fields(pv.fs[1], n)};
-}
-
-template <class LA, class LB>
-__device__ __forceinline__ void apply_op(const Op &op, double *a, double *b, const ProgView &pv, int n,
-                                         const NodeFieldCache &fc) {
-    NodeFields s = op.fset == 0 ? fc.f0 : (op.fset == 1 ? fc.f1 : load_fields(field_set(pv, op.fset), n));
-    if ((op.lat ^ pv.latswap) == 0) apply_on<LA, LB>(op, a, b, s);
-    else if constexpr (LB::nc > 0) apply_on<LB, LA>(op, b, a, s);
-}
-
-// Run the operators of boundary slot `slot` (node n) except SMOOTH, in record order.  The slot's
-// operator list (shared by every slot with the same operators) sits at sops[list * maxops ...],
-// padded with OP_NONE to a multiple of kOpBatch, its count in the first operator; a batch is
-// fetched with independent loads together with the node's fields.
-template <class LA, class LB>
-__device__ __forceinline__ void run_list_ops(const ProgView &pv, int li, int n, double *a, double *b) {
-    if (li < 0) return;
-    const Op *p = pv.sops + (size_t)li * pv.maxops;
-    NodeFieldCache fc = prefetch_fields(pv, n);
-    int count = pv.maxops;  // the list's own count arrives with its first batch
-    for (int base = 0; base < count; base += kOpBatch) {
-        Op o[kOpBatch];
-        sfor<0, kOpBatch>([&](auto q) { o[decltype(q)::value] = p[base + decltype(q)::value]; });
-        if (base == 0 && o[0].pad[0] != 0) count = o[0].pad[0];
-        sfor<0, kOpBatch>([&](auto q) {
-            const Op &op = o[decltype(q)::value];
-            if (op.code != OP_NONE && op.code != OP_SMOOTH) apply_op<LA, LB>(op, a, b, pv, n, fc);
-        });
+__device__ __forceinline__ NodeOps ops_of_node(const ProgView &pv, const Grid &g, int i, int j, int k, int n, int nd,
+                                               bool wanted = true) {
+    const int place = place_of(i, j, k, g.nx, g.ny, g.nz, nd);
+    NodeOps no{{-1, -1, 0, 0, {0, 0}, {}}, {}};
+    if (wanted && ((pv.shared | pv.by_slot) >> place & 1u)) {
+        const NodeList *e = pv.place_list + place;
+        if (pv.by_slot >> place & 1u) e = pv.slot_list + boundary_slot(i, j, k, g.nx, g.ny, g.nz, nd);
+        const uint64_t *p = reinterpret_cast<const uint64_t *>(e);
+        const uint64_t lf = gat(p, 0);
+        no.o.list = (int)(uint32_t)lf;
+        no.o.form = (int)(uint32_t)(lf >> 32);
+        no.o.count = (int)(uint32_t)gat(p, 1);
+        no.o.w[0] = gat(p, 2);
+        no.o.w[1] = gat(p, 3);
+        const double *v = reinterpret_cast<const double *>(e) + 4;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) no.o.vals.a[c] = gat(v, c);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) no.o.vals.b[c >> 1][c & 1] = gat(v, 4 + c);
+        no.f = load_fields(pv.fm, n);
     }
+    return no;
 }
 
-template <class LA, class LB>
-__device__ __forceinline__ void run_slot_ops(const ProgView &pv, int slot, int n, double *a, double *b) {
-    run_list_ops<LA, LB>(pv, pv.slot_list[slot], n, a, b);
+__device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+    return (uint64_t)hi << 32 | lo;
 }
-// Operator list of node (i, j, k), or -1 (no boundary slot, or a slot without operators).  The
-// fused kernels load it before the node's pull so that its latency overlaps the pull's.
-__device__ __forceinline__ int list_of_node(const ProgView &pv, const Grid &g, int i, int j, int k, int nd) {
-    const int slot = boundary_slot(i, j, k, g.nx, g.ny, g.nz, nd);
-    return (slot >= 0 && slot < pv.nslot) ? pv.slot_list[slot] : -1;
+// One register for each population, whichever operator wrote it (without it the register allocator
+// has spilled the single-lattice kernels: up to 2.6 kB per lane).
+template <class L>
+__device__ __forceinline__ void settle(double *f) {
+#pragma unroll
+    for (int c = 0; c < L::nc; ++c) asm volatile("" : "+v"(f[c]));
+}
+// Run a node's operators in record order; smooth(kernel lattice 0 / 1) stands for a SMOOTH operator.
+// Called with the boundary lanes (and any others: form -1) active.
+//
+// What bounds it is latency and instruction fetch, not arithmetic: a wavefront of 64 consecutive
+// nodes holds one or two x-face nodes, which it all waits for, and with each lane deciding for
+// itself which operator and which face to run, the wavefront walked every branch of a decision
+// tree per operator, in four inlined copies, after three dependent memory round trips.  Here the
+// wavefront takes the forms its lanes have one after the other (nearly always one or two); a form's
+// words are uniform, so the choice of operator and face is scalar branches over one copy.
+template <class LA, class LB, class Smooth>
+__device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, int n, double *a, double *b,
+                                        Smooth &&smooth) {
+    const NodeList &o = no.o;
+    unsigned long long todo = __ballot(o.form >= 0);
+    if (todo == 0) return;
+    do {
+        const int lead = __builtin_ctzll(todo);
+        const int form = __builtin_amdgcn_readlane(o.form, lead);
+        const int count = __builtin_amdgcn_readlane(o.count, lead);
+        uint64_t w0 = readlane64(o.w[0], lead), w1 = readlane64(o.w[1], lead);
+        const bool mine = o.form == form;
+        todo &= ~__ballot(mine);
+        for (int t = 0; t < count; ++t) {
+            uint32_t w = (uint32_t)w0 & 0xffffu;
+            w0 = w0 >> 16 | w1 << 48;
+            w1 >>= 16;
+            if (t >= kWordOps)
+                w = (uint32_t)__builtin_amdgcn_readfirstlane((int)pv.form_ops[(size_t)form * pv.maxops + t]);
+            const OpWord op = op_fields(w);
+            if (mine) {
+                OpIn q{{o.vals.a[0], o.vals.a[1], o.vals.a[2], o.vals.a[3]}, {o.vals.b[0][0], o.vals.b[0][1]}};
+                if (op.src == kFromSecond) {
+                    q.b[0] = o.vals.b[1][0];
+                    q.b[1] = o.vals.b[1][1];
+                } else if (op.src == kFromList) {
+                    q = op_in(pv.list_ops[(size_t)o.list * pv.maxops + t]);
+                }
+                if (op.code == OP_SMOOTH) smooth((int)op.lat ^ pv.latswap);
+                else if (op.code != OP_NONE) apply_op<LA, LB>(op, q, a, b, pv, n, no.f);
+                settle<LA>(a);
+                settle<LB>(b);
+            }
+        }
+    } while (todo);
 }
 
 // E_c of a shift, in FP64
@@ -217,30 +269,40 @@ __device__ __forceinline__ S enc(double v, const Enc &e) {
     else return S(v - shift_c<L, C>(e));
 }
 
-// One pulled value, loaded non-temporal with NT (see node_state).
+// One value at a byte offset of a plane, loaded non-temporal with NT (see pull_pair).
 template <bool NT, class S>
-__device__ __forceinline__ S pull_load(const S *p) {
-    if constexpr (NT) return __builtin_nontemporal_load(p);
-    else return *p;
+__device__ __forceinline__ S pull_load(const S *plane, uint32_t off) {
+    if constexpr (NT) return gload_nt(plane, off);
+    else return gload(plane, off);
 }
 
 // Pull node n's populations: pull = +1 from x - c (Stream), -1 from x + c (iStream), 0 in place.
-// S: storage type; values are decoded with the source node's shift.
+// S: storage type; values are decoded with the source node's shift.  The byte offsets of the three
+// columns, rows and planes a pull can come from are formed once; each population then costs one
+// three-way add beside its load (64-bit addresses per population took about 300 of the 1,200
+// vector instructions of a D3Q15 + D3Q7 step).
 template <class L, bool NT = false, class S, class R>
-__device__ __forceinline__ void load_pull(const S *__restrict__ src, const Grid &g, int i, int j, int k, int n,
+__device__ __forceinline__ void load_pull(const S *src, const Grid &g, int i, int j, int k, int n,
                                           int pull, R *f, const Enc &e = Enc{}) {
     if constexpr (L::nc > 0) {
-        f[0] = R(dec<L, 0>(pull_load<NT>(&src[n]), e));
+        // its own value of the pointer, or the two forms' loads are merged into plain ones
+        if constexpr (NT) asm volatile("" : "+s"(src));
+        constexpr uint32_t E = sizeof(S);
+        const uint32_t row = (uint32_t)g.nx * E, lay = row * (uint32_t)g.ny;
+        const int lo = pull, hi = -pull;  // displacement of the source for c = -1 and c = +1
+        const uint32_t x[3] = {(uint32_t)wrap(i, lo, g.nx) * E, (uint32_t)i * E, (uint32_t)wrap(i, hi, g.nx) * E};
+        const uint32_t y[3] = {(uint32_t)wrap(j, lo, g.ny) * row, (uint32_t)j * row, (uint32_t)wrap(j, hi, g.ny) * row};
+        uint32_t z[3] = {0u, 0u, 0u};
+        if constexpr (L::nd == 3) {
+            z[0] = (uint32_t)wrap(k, lo, g.nz) * lay;
+            z[1] = (uint32_t)k * lay;
+            z[2] = (uint32_t)wrap(k, hi, g.nz) * lay;
+        }
+        f[0] = R(dec<L, 0>(pull_load<NT>(src, (uint32_t)n * E), e));
         sfor<1, L::nc>([&](auto c) {
             constexpr int C = decltype(c)::value;
-            int s = n;
-            if (pull != 0) {
-                int ii = wrap(i, -pull * L::cx[C], g.nx);
-                int jj = wrap(j, -pull * L::cy[C], g.ny);
-                int kk = L::nd == 3 ? wrap(k, -pull * L::cz[C], g.nz) : 0;
-                s = ii + g.nx * (jj + g.ny * kk);
-            }
-            f[C] = R(dec<L, C>(pull_load<NT>(&src[(size_t)C * g.N + s]), e));
+            const uint32_t off = x[L::cx[C] + 1] + y[L::cy[C] + 1] + z[L::cz[C] + 1];
+            f[C] = R(dec<L, C>(pull_load<NT>(src + (size_t)C * g.N, off), e));
         });
     }
 }
@@ -248,14 +310,14 @@ template <class L, class S>
 __device__ __forceinline__ void load_node(const S *__restrict__ src, int N, int n, double *f, const Enc &e = Enc{}) {
     sfor<0, L::nc>([&](auto c) {
         constexpr int C = decltype(c)::value;
-        f[C] = dec<L, C>(src[(size_t)C * N + n], e);
+        f[C] = dec<L, C>(gat(src + (size_t)C * N, n), e);
     });
 }
 template <class L, class S>
 __device__ __forceinline__ void store_node(S *__restrict__ dst, int N, int n, const double *f, const Enc &e = Enc{}) {
     sfor<0, L::nc>([&](auto c) {
         constexpr int C = decltype(c)::value;
-        dst[(size_t)C * N + n] = enc<L, C, S>(f[C], e);
+        gput(dst + (size_t)C * N, n, enc<L, C, S>(f[C], e));
     });
 }
 
@@ -270,11 +332,16 @@ __device__ __forceinline__ Sh4 own_shift(const Enc &e) {
 // Values as stored, without decoding (the hot path keeps FP32 deviations of the node's own shift).
 template <class L, class S, class R>
 __device__ __forceinline__ void load_raw(const S *__restrict__ src, int N, int n, R *f) {
-    sfor<0, L::nc>([&](auto c) { f[decltype(c)::value] = R(src[(size_t)decltype(c)::value * N + n]); });
+    sfor<0, L::nc>([&](auto c) { f[decltype(c)::value] = R(gat(src + (size_t)decltype(c)::value * N, n)); });
 }
-template <class L, class S, class R>
-__device__ __forceinline__ void store_raw(S *__restrict__ dst, int N, int n, const R *f) {
-    sfor<0, L::nc>([&](auto c) { dst[(size_t)decltype(c)::value * N + n] = S(f[decltype(c)::value]); });
+template <class L, bool NT = false, class S, class R>
+__device__ __forceinline__ void store_raw(S *dst, int N, int n, const R *f) {
+    if constexpr (L::nc > 0 && NT) asm volatile("" : "+s"(dst));  // as in load_pull
+    sfor<0, L::nc>([&](auto c) {
+        constexpr int C = decltype(c)::value;
+        if constexpr (NT) gstore_nt(dst + (size_t)C * N, (uint32_t)n * (uint32_t)sizeof(S), S(f[C]));
+        else gput(dst + (size_t)C * N, n, S(f[C]));
+    });
 }
 // Register state <-> FP64 populations (identity in FP64; deviations of shift o in FP32)
 template <class L>
@@ -289,22 +356,6 @@ __device__ __forceinline__ void get_state(double *v, const double *src, const En
 }
 template <class L>
 __device__ __forceinline__ void get_state(float *v, const double *src, const Enc &e, const Sh4 &o);
-// d2q9.h:577-587: the mean of two FP64 states
-template <class L>
-__device__ __forceinline__ void mean_state(double *v, const double *a, const double *b, const Enc &, const Sh4 &) {
-    sfor<0, L::nc>([&](auto c) {
-        constexpr int C = decltype(c)::value;
-        v[C] = 0.5 * (a[C] + b[C]);
-    });
-}
-template <class L>
-__device__ __forceinline__ void mean_state(float *v, const double *a, const double *b, const Enc &e, const Sh4 &) {
-    sfor<0, L::nc>([&](auto c) {
-        constexpr int C = decltype(c)::value;
-        v[C] = float(0.5 * (a[C] + b[C]) - shift_c<L, C>(e));
-    });
-}
-
 // FP32 deviations <-> FP64 populations, for the boundary operators and smoothing
 template <class L>
 __device__ __forceinline__ void dev_to_f64(const float *d, double *f, const Enc &e, const Sh4 &) {
@@ -329,11 +380,33 @@ __device__ __forceinline__ void get_state(float *v, const double *src, const Enc
     f64_to_dev<L>(src, v, e, o);
 }
 
+// Smoothed states (d2q9.h:577-587, d3q15.h:1241-1303) across the lanes of a wavefront.  Lanes come in
+// groups: 4 per 2D corner or 3D edge node (two face neighbours' states, then the node's own, then a
+// spare), 8 per 3D corner (the neighbours of its three edge nodes in x, y, z order, then its own,
+// then a spare).  Lane 2 of a group of 4 gets 0.5 (a + b); lane 6 of a group of 8 the mean of the
+// three edge means.  The means are of FP64 populations.
+template <class L, class R>
+__device__ __forceinline__ void smooth_lanes_mean(R *f, const Enc &e, bool corner3) {
+    const int base = (int)(threadIdx.x & 56u);
+    sfor<0, L::nc>([&](auto c) {
+        constexpr int C = decltype(c)::value;
+        double v;
+        if constexpr (is_f64<R>) v = f[C];
+        else v = double(f[C]) + shift_c<L, C>(e);
+        const double m = 0.5 * (v + __shfl_xor(v, 1));
+        double s;
+        if (corner3) s = (__shfl(m, base) + __shfl(m, base + 2) + __shfl(m, base + 4)) / 3.0;
+        else s = __shfl_xor(m, 2);
+        if constexpr (is_f64<R>) f[C] = s;
+        else f[C] = float(s - shift_c<L, C>(e));
+    });
+}
+
 __device__ __forceinline__ void coords(int n, const Grid &g, int &i, int &j, int &k) {
-    i = n % g.nx;
-    int t = n / g.nx;
-    j = t % g.ny;
-    k = t / g.ny;
+    const int t = (int)div_by((uint32_t)n, g.by_nx);
+    i = n - t * g.nx;
+    k = (int)div_by((uint32_t)t, g.by_ny);
+    j = t - k * g.ny;
 }
 __device__ __forceinline__ int nboundary(int i, int j, int k, const Grid &g, int nd) {
     int c = (i == 0 || i == g.nx - 1) + (j == 0 || j == g.ny - 1);
@@ -342,11 +415,12 @@ __device__ __forceinline__ int nboundary(int i, int j, int k, const Grid &g, int
 }
 
 // Both lattices' pulls of node n.  With g.nt (3D launches whose populations do not fit the
-// Infinity Cache, set by the host) the loads are non-temporal: a step reads each source population
-// once, and streaming them keeps the caches for the populations the step writes, which the next
-// step reads (128x128x64 duct step 98 -> 82 us).  Where the step fits the cache (96x96x48: 3.44 ->
-// 3.58 s per design iteration with the hint) or reuses a source row from L2 for the rows beside it
-// (2D, 4096^2 step 773 -> 837 us with the hint) the loads stay normal.
+// Infinity Cache, set by the host) the pulled loads and the stores are non-temporal: a step reads
+// each source population once and writes each once, in an order the next step repeats, so lines
+// kept behind only displace each other.  D3Q15 + D3Q7 FP64 forward step: 128x128x64 (369 MB) 89 us
+// with plain accesses, 82 with the loads non-temporal, 79 with the stores too; at 96x96x48 (156 MB,
+// cache-resident) non-temporal stores cost 32 -> 39 us.  In 2D a source row is reused from L2 for the
+// rows beside it (4096^2 step 773 -> 837 us with the loads non-temporal), so 2D stays plain.
 template <class LA, class LB, class S, class R>
 __device__ __forceinline__ void pull_pair(const S *sa, const S *sb, const Grid &g, int i, int j, int k, int n,
                                           const ProgView &pv, R *a, R *b, const Enc &, const Enc &) {
@@ -360,30 +434,31 @@ __device__ __forceinline__ void pull_pair(const S *sa, const S *sb, const Grid &
 }
 
 // Post-stream, post-boundary state of node n; SMOOTH operators are skipped (callers that own
-// smoothed nodes apply them).  FP64: the populations.  FP32: their deviations from node n's shift
+// smoothed nodes apply them), and all are without ops.  FP64: the populations.  FP32: their deviations from node n's shift
 // (oa, ob); the boundary operators run on FP64 populations.
 template <class LA, class LB>
 __device__ __forceinline__ void node_state(const double *sa, const double *sb, const Grid &g, const ProgView &pv, int n,
-                                           double *a, double *b, const Enc &, const Enc &, const Sh4 &, const Sh4 &) {
+                                           double *a, double *b, const Enc &, const Enc &, const Sh4 &, const Sh4 &,
+                                           bool ops = true) {
     int i, j, k;
     coords(n, g, i, j, k);
-    const int li = list_of_node(pv, g, i, j, k, LA::nd);
+    const NodeOps no = ops_of_node(pv, g, i, j, k, n, LA::nd, ops);
     pull_pair<LA, LB>(sa, sb, g, i, j, k, n, pv, a, b, Enc{}, Enc{});
-    run_list_ops<LA, LB>(pv, li, n, a, b);
+    run_ops<LA, LB>(pv, no, n, a, b, [](int) {});
 }
 template <class LA, class LB, class S, std::enable_if_t<!std::is_same_v<S, double>, int> = 0>
 __device__ __forceinline__ void node_state(const S *sa, const S *sb, const Grid &g, const ProgView &pv, int n,
                                            float *a, float *b, const Enc &ea, const Enc &eb, const Sh4 &oa,
-                                           const Sh4 &ob) {
+                                           const Sh4 &ob, bool ops = true) {
     int i, j, k;
     coords(n, g, i, j, k);
-    const int li = list_of_node(pv, g, i, j, k, LA::nd);
+    const NodeOps no = ops_of_node(pv, g, i, j, k, n, LA::nd, ops);
     pull_pair<LA, LB>(sa, sb, g, i, j, k, n, pv, a, b, Enc{}, Enc{});
-    if (li >= 0) {
+    if (no.o.form >= 0) {
         double xa[LA::nc], xb[LB::nc > 0 ? LB::nc : 1];
         dev_to_f64<LA>(a, xa, ea, oa);
         if constexpr (LB::nc > 0) dev_to_f64<LB>(b, xb, eb, ob);
-        run_list_ops<LA, LB>(pv, li, n, xa, xb);
+        run_ops<LA, LB>(pv, no, n, xa, xb, [](int) {});
         f64_to_dev<LA>(xa, a, ea, oa);
         if constexpr (LB::nc > 0) f64_to_dev<LB>(xb, b, eb, ob);
     }

@@ -99,6 +99,42 @@ struct D3Q7 {
     static constexpr double w[7] = {0.0, 1.0 / 6.0, 1.0 / 6.0, 1.0 / 6.0, 1.0 / 6.0, 1.0 / 6.0, 1.0 / 6.0};
 };
 
+// ---- device memory as global memory ---------------------------------------------------------
+// Pointers that reach a kernel inside a struct in memory (batched steps) would be accessed as flat
+// addresses; these helpers name them global, and take a uniform base with a 32-bit byte offset per
+// lane, which is the addressing form that needs no 64-bit address per lane.  A plane's byte offsets
+// fit 32 bits: a lattice holds at most 2^31 populations, and has at least 5 of them per node.
+#define LBM_GLOBAL __attribute__((address_space(1)))
+template <class T>
+__device__ __forceinline__ T gload(const T *base, uint32_t off) {
+    return *(const LBM_GLOBAL T *)((const LBM_GLOBAL char *)base + off);
+}
+template <class T>
+__device__ __forceinline__ T gload_nt(const T *base, uint32_t off) {
+    return __builtin_nontemporal_load((const LBM_GLOBAL T *)((const LBM_GLOBAL char *)base + off));
+}
+template <class T>
+__device__ __forceinline__ void gstore(T *base, uint32_t off, T v) {
+    *(LBM_GLOBAL T *)((LBM_GLOBAL char *)base + off) = v;
+}
+template <class T>
+__device__ __forceinline__ void gstore_nt(T *base, uint32_t off, T v) {
+    __builtin_nontemporal_store(v, (LBM_GLOBAL T *)((LBM_GLOBAL char *)base + off));
+}
+// element n of a node field
+template <class T>
+__device__ __forceinline__ T gat(const T *p, int n) {
+    return gload(p, (uint32_t)n * (uint32_t)sizeof(T));
+}
+__device__ __forceinline__ int2 gat(const int2 *p, int n) {
+    const uint64_t w = gat(reinterpret_cast<const uint64_t *>(p), n);
+    return make_int2((int)(uint32_t)w, (int)(uint32_t)(w >> 32));
+}
+template <class T, class V>
+__device__ __forceinline__ void gput(T *p, int n, V v) {
+    gstore(p, (uint32_t)n * (uint32_t)sizeof(T), T(v));
+}
+
 // ---- compile-time loop ------------------------------------------------------------------
 template <class F, int... Is>
 __host__ __device__ __forceinline__ void sfor_impl(F &&f, std::integer_sequence<int, Is...>) {
@@ -128,10 +164,30 @@ __device__ __forceinline__ R cmul(R v) {
 }
 
 // ---- grid geometry ------------------------------------------------------------------------
+// n / d for 0 <= n < 2^31, d >= 1 as one high multiply, one add and one shift: with s = ceil(log2 d)
+// and m = floor(2^32 (2^s - d) / d) + 1 the quotient is (mulhi(m, n) + n) >> s (Granlund and
+// Montgomery 1994, the round-up form; the sum stays below 2^32 because n < 2^31).  A division by a
+// run-time nx costs about 20 vector instructions; every lane makes up to two to find its node.
+struct FastDiv {
+    uint32_t m, s;
+};
+__host__ inline FastDiv fast_div(uint32_t d) {
+    uint32_t s = 0;
+    while ((uint64_t(1) << s) < d) ++s;
+    return FastDiv{uint32_t((((uint64_t(1) << s) - d) << 32) / d + 1), s};
+}
+__host__ __device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv &f) {
+    return (uint32_t((uint64_t(f.m) * n) >> 32) + n) >> f.s;
+}
+
 struct Grid {
     int nx, ny, nz, N;
     int nt;  // 1: the fused kernels load the pulled populations non-temporal (set per launch)
+    FastDiv by_nx, by_ny;
 };
+inline Grid make_grid(int nx, int ny, int nz, int N) {
+    return Grid{nx, ny, nz, N, 0, fast_div((uint32_t)nx), fast_div((uint32_t)ny)};
+}
 
 // Periodic neighbour of (i, j, k) shifted by (dx, dy, dz) in {-1, 0, 1}: d2q9.h:80-84.
 __device__ __forceinline__ int wrap(int a, int d, int n) {
@@ -141,10 +197,12 @@ __device__ __forceinline__ int wrap(int a, int d, int n) {
 
 // Workgroup -> tile order that keeps consecutive tiles on one XCD: the hardware deals
 // workgroups round-robin over the 8 XCDs, so workgroup b runs on XCD b % 8.  Tiles of XCD x are
-// made contiguous, which keeps a tile's +-1 row neighbours in the same L2.
+// made contiguous, which keeps a tile's +-1 row neighbours in the same L2.  The upper four XCDs walk
+// their tiles downwards: the grid's last plane (3D) or row, whose nodes all run boundary operators,
+// is then begun first instead of being what the other XCDs wait for.
 __device__ __forceinline__ int xcd_tile(int b, int nb) {
-    int q = nb >> 3, r = nb & 7, x = b & 7;
-    return x * q + (x < r ? x : r) + (b >> 3);
+    const int q = nb >> 3, r = nb & 7, x = b & 7, t = b >> 3, size = q + (x < r);
+    return x * q + (x < r ? x : r) + (x < 4 ? t : size - 1 - t);
 }
 
 }  // namespace lbm

@@ -29,7 +29,7 @@ enum OpCode : uint8_t {
     OP_SMOOTH = 12,       // d2q9.h:577-587, d3q15.h:1241-1303 (fix-up kernels only)
 };
 
-// One operator at one node.  40 bytes, naturally aligned for 8-byte loads.
+// One operator at one node, as recorded.
 struct Op {
     uint8_t code;
     uint8_t face;  // 0 xmin, 1 xmax, 2 ymin, 3 ymax, 4 zmin, 5 zmax
@@ -37,7 +37,7 @@ struct Op {
     uint8_t arg;
     uint8_t fset;  // index of the field set the operator reads
     uint8_t seg;   // number of SmoothCorner calls recorded before this operator
-    uint8_t pad[2];  // operator lists (sops): pad[0] of a list's first operator = its operator count
+    uint8_t pad[2];
     double v[3];
     double v3;     // eps where used
 };
@@ -49,7 +49,53 @@ struct FieldSet {
 };
 constexpr int kMaxFieldSets = 4;
 constexpr size_t kXcdRemapMaxBytes = size_t(640) << 20;  // population bytes read + written per step
-constexpr int kOpBatch = 4;  // operators fetched per batch by the fused kernels
+
+
+// The fused kernels' form of an operator: 16 bits, and its values among the few its node's list holds
+// (OpIn: a for the Navier-Stokes operators, b for the advection-diffusion ones), so that a boundary
+// node learns all it has to do with one load and has every operand with the next ones.
+enum OpSource : uint32_t { kFromFirst = 0, kFromSecond = 1, kFromList = 2 };
+constexpr int kWordOps = 8;  // operators in a SlotOps; a longer list's further words sit in form_ops
+__host__ __device__ constexpr uint32_t op_word(uint32_t code, uint32_t face, uint32_t lat, uint32_t fset, uint32_t arg,
+                                               uint32_t src) {
+    return code | face << 4 | lat << 7 | fset << 8 | arg << 10 | src << 12;
+}
+struct OpWord {
+    uint32_t code, face, lat, fset, arg, src;
+};
+__host__ __device__ inline OpWord op_fields(uint32_t w) {
+    return OpWord{w & 15u, w >> 4 & 7u, w >> 7 & 1u, w >> 8 & 3u, w >> 10 & 3u, w >> 12 & 3u};
+}
+// An operator's values: a = (v[0], v[1], v[2], v3); b = (v[0], v[1]) of OP_AD_SET_Q, (v[0], -) of
+// OP_AD_SET_T, (-, v3) of the adjoint ones.
+struct OpIn {
+    double a[4], b[2];
+};
+// The values of a recorded operator.
+__host__ __device__ inline OpIn op_in(const Op &o) {
+    return OpIn{{o.v[0], o.v[1], o.v[2], o.v3}, {o.v[0], o.code == OP_AD_SET_Q ? o.v[1] : o.v3}};
+}
+struct alignas(16) ListVals {  // a list's values: one a, two b
+    double a[4], b[2][2];
+};
+
+// A boundary node's operators and their values.  Lists that differ in their values only share a form
+// (the sequence of words): a wavefront runs one form at a time on all lanes that have it.
+struct alignas(16) NodeList {
+    int list, form, count, pad;  // list, form: -1 without operators
+    uint64_t w[2];               // the first kWordOps operators, 16 bits each
+    ListVals vals;
+};
+// The nodes of a grid fall into 27 places: on the low side, between or on the high side of each axis
+// (2D: always between in z); 13 is the interior.  Where all nodes of a place share one list, as those
+// of a wall or of a uniform inlet do, the fused kernels take it from a table of places, which stays
+// in the nearest cache; the nodes of other places look theirs up by slot.
+constexpr int kPlaces = 27, kInterior = 13;
+__host__ __device__ inline int place_of(int i, int j, int k, int nx, int ny, int nz, int nd) {
+    const int x = i == 0 ? 0 : (i == nx - 1 ? 2 : 1), y = j == 0 ? 0 : (j == ny - 1 ? 2 : 1);
+    const int z = nd == 2 ? 1 : (k == 0 ? 0 : (k == nz - 1 ? 2 : 1));
+    return x + 3 * y + 9 * z;
+}
 
 // Device view of a program.
 struct ProgView {
@@ -57,32 +103,37 @@ struct ProgView {
     const int *entry_node;  // entry -> node index
     const int2 *entry_ops;  // entry -> (first op, op count)
     const Op *ops;
-    const Op *sops;         // distinct operator lists, maxops each, OP_NONE-padded
-    const int *slot_list;   // boundary slot -> its list in sops, or -1 (size nslot)
-    int maxops;             // operators per list in sops, a multiple of kOpBatch (0: no operators)
+    const NodeList *place_list;  // place -> its nodes' list, where they share one
+    const NodeList *slot_list;   // boundary slot -> its list (size nslot)
+    unsigned shared, by_slot;    // bit p: place p's nodes share a list of operators / have several lists
+    const Op *list_ops;         // list -> maxops operators (for values outside a NodeList)
+    const uint32_t *form_ops;   // form -> maxops words
+    int maxops;             // operators per list (0: no operators)
     int nentry;
     int nslot;
     FieldSet fs[kMaxFieldSets];
+    // The field sets that agree wherever two of them name the same field, as one: a boundary node's
+    // fields are loaded once for all of them (bit k of fmerged: set k is in fm; bit k of has_diff:
+    // set k has a diffusivity field).
+    FieldSet fm;
+    unsigned fmerged, has_diff;
     int pull[2];            // per kernel lattice: +1 stream (pull from x - c), -1 iStream (x + c), 0 none
     int latswap;            // 1 when the program's lattice 0 is the kernel's second lattice
     int xcd;                // 1: workgroup -> tile remap that keeps consecutive tiles on one XCD
-    // Corner smoothing after the pass: the fused pass saves the post-boundary state of each
+    // Smoothing after the pass: the fused pass saves the post-boundary state of each
     // smoothed node's inward face neighbours here (kSideStride doubles each: the kernel's first
     // lattice, then its second) and a kernel launched after it averages them (2D corners; 3D edges
     // and corners).  nullptr when unused.
     const int *side_of_slot;  // boundary slot -> side-state index or -1
     double *side;
-    // 2D corner smoothing inside the fused pass, used when the boundary operators read no array the
-    // collide saves: the grid's last workgroup rebuilds the corners' inward neighbours' states, swaps
-    // them through LDS and finishes the corners, concurrently with the rest of the pass.
-    int corner_block;         // 1: the last workgroup does the corners
-    int nside, ncorner;       // neighbour states (<= kMaxSide) and corners
-    const int *side_nodes;    // node of each neighbour state
-    const int4 *corners;      // (node, state of x-neighbour, state of y-neighbour, smoothed-lattice bits)
+    // Smoothing inside the fused pass, used when the boundary operators read no array the collide
+    // saves: the grid's first lanes rebuild the states of the smoothed nodes' inward neighbours and
+    // finish the smoothed nodes, concurrently with the rest of the pass.
+    int nsmooth;                // lanes (2D: a wavefront per corner; 3D: the length of smooth_lanes); 0: none
+    int smooth_bits;            // bit k: the program's lattice k is smoothed
+    const int2 *smooth_lanes;   // 3D: per lane (node whose state it rebuilds, node it finishes or -1)
 };
-constexpr int kMaxSide = 8;
-constexpr int kCornerEdgeSlots = 24;  // 3D edge nodes beside a corner (k_collide_smoothed_self's LDS)
-constexpr int kSmoothedGroup = 256;   // lanes of k_collide_smoothed_self's workgroup 0 (its block size)
+constexpr int kCornerLanes = 512;  // 3D: the first lanes of smooth_lanes, a wavefront per corner
 constexpr int kSideStride = 40;  // >= nc(first) + nc(second) of any lattice pair (D3Q27 + D3Q7: 34)
 
 // Boundary slot of node (i, j, k) on an nx*ny*nz grid, -1 for interior nodes.  Surface nodes are
