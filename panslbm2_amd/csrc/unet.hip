@@ -8,13 +8,13 @@
 //   * convolutions are implicit GEMMs on the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16):
 //     bfloat16 weights and activations, FP32 accumulation.  Activations are channels-last
 //     ([voxel][channel], voxel = x + nx (y + ny z)), so the 8 consecutive K values one lane feeds
-//     the matrix core (8 channels of one tap) are one 16-byte load;
+//     the matrix core (8 channels of one tap) are one 16-byte load, of a brick staged in LDS;
 //   * the input gradient of a convolution is the same kernel run on the output gradient with the
 //     weights transposed and the taps mirrored;
-//   * the weight gradient reduces over voxels: 32-voxel tiles of the output gradient and of the
-//     shifted input are staged through LDS in [channel][voxel] order, so the matrix-core operands
-//     are again 16-byte reads; partial sums per voxel range are reduced in a fixed order, so the
-//     gradient is deterministic;
+//   * the weight gradient reduces over voxels: tiles of the output gradient and of the shifted input
+//     are staged through LDS in [channel][voxel] order, so the matrix-core operands are again
+//     16-byte reads; partial sums per voxel range are reduced in a fixed order, so the gradient is
+//     deterministic;
 //   * Adam keeps FP32 master weights and repacks the bfloat16 copies after each update.
 //
 // The fields the solver uses are FP64 arrays; the network reads and writes them directly
@@ -26,6 +26,7 @@
 // the reference starts every solve from rest.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -44,7 +45,7 @@ typedef __attribute__((ext_vector_type(4))) float f4;
 constexpr int kMaxFields = 16;
 constexpr int kMaxCg = 64;   // widest output gradient a weight-gradient launch stages
 constexpr int kMaxCx = 96;   // widest input it stages
-constexpr int kTileV = 64;   // voxels per LDS tile (two matrix-core K steps of 32)
+constexpr int kTileV = 64;   // voxel ranges of the weight gradient are multiples of this
 
 __host__ __device__ inline bf16_t f2bf(float f) {
     uint32_t u;
@@ -66,154 +67,320 @@ __host__ __device__ inline int tap_dy(int t, int taps) { return taps == 27 ? (t 
 __host__ __device__ inline int tap_dz(int t, int taps) { return taps == 27 ? t / 9 - 1 : 0; }
 
 // ---- convolution (forward, and input gradient with transposed weights) ----------------------------
-// y[v][o] = bias[o] + sum_k w[o][k] x[v + off(tap)][ci], k = tap cin + ci.  One wave computes
-// 16 MT output channels x 64 voxels (4 tiles of 16); a workgroup is 4 waves along the voxels.
+// y[v][o] = bias[o] + sum_k w[o][k] x[v + off(tap)][ci], k = tap cin + ci.
 // The matrix core sums A[m][k] B[k][n] over k: A = weights (row m = lane % 16), B = shifted input
 // (column n = lane % 16); both operands give slot j of lane group q the same k = 8q + j, so the
 // sum is the same whatever order the hardware pairs slots in.  D[m = 4q + j][n = lane % 16].
-template <int MT>
-__global__ void __launch_bounds__(256) k_conv(const bf16_t *__restrict__ x, int cin, int taps,
-                                              const bf16_t *__restrict__ w, int kpad,
-                                              const float *__restrict__ bias, bf16_t *__restrict__ y,
-                                              float *__restrict__ y32, int cstore, int creal, int relu, int nx,
-                                              int ny, int nz) {
+
+// Four output channels of one voxel: bias, ReLU, or the mask of a ReLU's input gradient (act: the
+// activation the ReLU gave; y = act > 0 ? value : 0), stored as 8 bytes of bfloat16 or 16 of FP32.
+struct ConvOut {
+    const float *bias;
+    bf16_t *y;
+    float *y32;
+    const bf16_t *act;
+    int cstore, creal, relu;
+};
+__device__ __forceinline__ void conv_store(const ConvOut &o, size_t v, int co, f4 a) {
+    float val[4];
+    uint2 on = {0u, 0u};
+    if (o.act) on = *(const uint2 *)(o.act + v * o.cstore + co);
+    const uint32_t m[4] = {on.x & 0xffffu, on.x >> 16, on.y & 0xffffu, on.y >> 16};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        val[j] = a[j] + (o.bias ? o.bias[co + j] : 0.f);
+        if (o.relu) val[j] = fmaxf(val[j], 0.f);
+        if (co + j >= o.creal) val[j] = 0.f;  // padded channels stay zero
+        if (o.act && !(bf2f((bf16_t)m[j]) > 0.f)) val[j] = 0.f;
+    }
+    if (o.y) {
+        uint2 p;
+        p.x = (uint32_t)f2bf(val[0]) | (uint32_t)f2bf(val[1]) << 16;
+        p.y = (uint32_t)f2bf(val[2]) | (uint32_t)f2bf(val[3]) << 16;
+        *(uint2 *)(o.y + v * o.cstore + co) = p;
+    }
+    if (o.y32) *(f4 *)(o.y32 + v * o.cstore + co) = f4{val[0], val[1], val[2], val[3]};
+}
+
+// 1x1x1 convolution to 16 output channels (the head and its input gradient): one wave computes 16
+// channels x 64 voxels; every input is read once, straight from memory.
+__global__ void __launch_bounds__(256) k_conv1(const bf16_t *__restrict__ x, int cin, const bf16_t *__restrict__ w,
+                                               int kpad, ConvOut out, int V) {
     constexpr int NT = 4;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-    const int V = nx * ny * nz;
-    const int v0 = (blockIdx.x * 4 + wv) * (16 * NT);
-    const int co0 = blockIdx.y * 16 * MT;
-    int px[NT], py[NT], pz[NT];
-    bool pin[NT];
+    const int v0 = (blockIdx.x * 4 + wv) * (16 * NT), co0 = blockIdx.y * 16;
+    f4 acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int kc = 0; kc < kpad; kc += 32) {
+        const int k = kc + 8 * q;
+        const bf16x8 a = ld8(w + (size_t)(co0 + r) * kpad + k);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int v = v0 + nt * 16 + r;
+            bf16x8 b = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
+            if (k < cin && v < V) b = ld8(x + (size_t)v * cin + k);
+            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nt], 0, 0, 0);
+        }
+    }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const int v = v0 + nt * 16 + r;
-        pin[nt] = v < V;
-        const int vv = pin[nt] ? v : 0;
-        px[nt] = vv % nx;
-        py[nt] = (vv / nx) % ny;
-        pz[nt] = vv / (nx * ny);
+        if (v < V) conv_store(out, (size_t)v, co0 + 4 * q, acc[nt]);
+    }
+}
+
+// 3x3x3 convolution.  A workgroup of WM x WN waves stages a brick of 18 x 6 x (WN + 2) voxels (its 16
+// x 4 x WN outputs and their halo, zero outside the grid) with all CIN channels in LDS once; wave
+// (m, n) computes 16 MT output channels of z layer n, 4 rows of 16 voxels.  Read from global memory
+// per tap, as it was, every input came through L1 27 times and each of those reads cost an address
+// and three bounds checks: at 96x96x48 and 16 -> 16 channels 58 us (109 TFLOP/s), bound by vector
+// instructions and L1.  Here a K step of 32 costs one LDS read of 16 bytes per lane and row at an
+// address the compiler knows up to a per-lane base, and its weights; all K steps are unrolled.
+// A voxel's row in LDS is 16 bytes longer than its channels (CIN = 8: not), so that the 16 lanes of a
+// row fall into different banks.  The products are summed in the order k = 0, 32, ... as before.
+template <int CIN>
+struct Brick {
+    static constexpr int VS = CIN * 2 + (CIN == 8 ? 0 : 16);  // bytes of a voxel in LDS
+    static constexpr int KS = (27 * CIN + 31) / 32;           // K steps
+    // byte offset of K unit u = 4 step + q (8 values of k) from the voxel at the output's corner (-1, -1, -1)
+    static constexpr int off(int u) {
+        const int k = 8 * u < 27 * CIN ? 8 * u : 0, t = k / CIN;  // past the end: any voxel of the brick
+        return (((t / 9) * 6 + (t / 3) % 3) * 18 + t % 3) * VS + (k % CIN) * 2;
+    }
+};
+template <int CIN, int MT, int WM, int WN>
+__global__ void __launch_bounds__(64 * WM * WN) k_conv3(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w,
+                                                        ConvOut out, int nx, int ny, int nz, int ntx, int nty) {
+    using B = Brick<CIN>;
+    constexpr int NT = 4, VS = B::VS, KS = B::KS, KPAD = 32 * KS, NV = 18 * 6 * (WN + 2), THREADS = 64 * WM * WN;
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 15, q = lane >> 4;
+    const int wm = wv % WM, wn = wv / WM;
+    const int bx = blockIdx.x % ntx, by = (blockIdx.x / ntx) % nty, bz = blockIdx.x / (ntx * nty);
+    const int x0 = bx * 16, y0 = by * 4, z0 = bz * WN;
+    constexpr int CU = CIN / 8;
+    for (int u = tid; u < NV * CU; u += THREADS) {
+        const int vox = u / CU, c = u - vox * CU;
+        const int px = vox % 18, py = (vox / 18) % 6, pz = vox / 108;
+        const int xx = x0 + px - 1, yy = y0 + py - 1, zz = z0 + pz - 1;
+        uint4 d = {0u, 0u, 0u, 0u};
+        if ((unsigned)xx < (unsigned)nx && (unsigned)yy < (unsigned)ny && (unsigned)zz < (unsigned)nz)
+            d = *(const uint4 *)(x + (size_t)(xx + nx * (yy + ny * zz)) * CIN + 8 * c);
+        *(uint4 *)(lds + vox * VS + 16 * c) = d;
     }
     f4 acc[MT][NT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
-    const int K = taps * cin;
-    for (int kc = 0; kc < kpad; kc += 32) {
-        const int k = kc + 8 * q;
+    __syncthreads();
+    const int co0 = (blockIdx.y * WM + wm) * 16 * MT;
+    const bf16_t *wr = w + (size_t)(co0 + r) * KPAD + 8 * q;
+    const unsigned char *base = lds + (wn * 108 + r) * VS;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
         bf16x8 a[MT];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) a[mt] = ld8(w + (size_t)(co0 + mt * 16 + r) * kpad + k);
-        const int tap = k / cin, ci = k - tap * cin;
-        const int dx = tap_dx(tap, taps), dy = tap_dy(tap, taps), dz = tap_dz(tap, taps);
-        const bool kin = k < K;
+        for (int mt = 0; mt < MT; ++mt) a[mt] = ld8(wr + (size_t)mt * 16 * KPAD + 32 * s);
+        // the four lane groups' units: one tap with the next channels, or taps of their own
+        const int o0 = B::off(4 * s), o1 = B::off(4 * s + 1), o2 = B::off(4 * s + 2), o3 = B::off(4 * s + 3);
+        const int at = (o1 == o0 + 16 && o2 == o0 + 32 && o3 == o0 + 48)
+                           ? o0 + 16 * q
+                           : (q < 2 ? (q == 0 ? o0 : o1) : (q == 2 ? o2 : o3));
+        const bool past = 32 * s + 8 * q >= 27 * CIN;  // the padding of the last step
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const int xx = px[nt] + dx, yy = py[nt] + dy, zz = pz[nt] + dz;
-            const bool ok = kin && pin[nt] && (unsigned)xx < (unsigned)nx && (unsigned)yy < (unsigned)ny &&
-                            (unsigned)zz < (unsigned)nz;
-            bf16x8 b = __builtin_bit_cast(bf16x8, uint4{0u, 0u, 0u, 0u});
-            if (ok) b = ld8(x + (size_t)(xx + nx * (yy + ny * zz)) * cin + ci);
+            uint4 d = *(const uint4 *)(base + at + nt * 18 * VS);
+            if (32 * s + 32 > 27 * CIN && past) d = uint4{0u, 0u, 0u, 0u};
+            const bf16x8 b = __builtin_bit_cast(bf16x8, d);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
                 acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], b, acc[mt][nt], 0, 0, 0);
         }
     }
+    const int vx = x0 + r, vz = z0 + wn;
+    if (vx >= nx || vz >= nz) return;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        const int v = v0 + nt * 16 + r;
-        if (v >= V) continue;
+        const int vy = y0 + nt;
+        if (vy >= ny) continue;
+        const size_t v = (size_t)vx + (size_t)nx * (vy + (size_t)ny * vz);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int co = co0 + mt * 16 + 4 * q + j;
-                if (co >= cstore) continue;
-                float val = acc[mt][nt][j] + (bias ? bias[co] : 0.f);
-                if (relu) val = fmaxf(val, 0.f);
-                if (co >= creal) val = 0.f;  // padded channels stay zero
-                if (y) y[(size_t)v * cstore + co] = f2bf(val);
-                if (y32) y32[(size_t)v * cstore + co] = val;
-            }
+        for (int mt = 0; mt < MT; ++mt) conv_store(out, v, co0 + mt * 16 + 4 * q, acc[mt][nt]);
     }
 }
 
 // ---- weight gradient ----------------------------------------------------------------------------
 // part[split][tap][o][i] = sum over the split's voxels v of g[v][o] x[v + off(tap)][i].
-// Matrix core: A[m = o][k = v], B[k = v][n = i], two K steps of 32 voxels per LDS tile.
-// The tap-0 workgroups also sum the staged g tiles: bpart[split][o] = sum over the split of g[v][o].
+// Matrix core: A[m = o][k = v], B[k = v][n = i], K steps of 32 voxels in ascending order.
+// The first tap's workgroups also sum the staged g: bpart[split][o] = sum over the split of g[v][o],
+// as four sums over every fourth 16-voxel run.
+//
+// A workgroup takes the TX taps along x of one (dy, dz) (3, or 1 for the 1x1x1 head) over one split.
+// Per tile of kt voxels a thread loads 8 channels of the 8 (or, shifted, 10) voxels it owns, transposes
+// them in registers (v_perm) and writes 8-voxel rows of 16 bytes to LDS, once per tap: the operands
+// then are 16-byte LDS reads.  The next tile's loads are issued before the products of this one.
+// One tap per workgroup, element-wise LDS writes and no prefetch, as it was, read g and x 27 times:
+// 178 us on average over the layers at 96x96x48.  LDS rows are kt + 8 voxels, so that the 16 rows of an
+// operand fall into different banks.
+__device__ __forceinline__ void transpose8(const uint4 (&d)[8], uint4 (&o)[8]) {
+    const uint32_t *s = reinterpret_cast<const uint32_t *>(d);  // s[4 voxel + p]: channels 2p, 2p + 1
+    uint32_t *t = reinterpret_cast<uint32_t *>(o);              // t[4 channel + m]: voxels 2m, 2m + 1
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            t[4 * (2 * p) + m] = __builtin_amdgcn_perm(s[4 * (2 * m + 1) + p], s[4 * (2 * m) + p], 0x05040100u);
+            t[4 * (2 * p + 1) + m] = __builtin_amdgcn_perm(s[4 * (2 * m + 1) + p], s[4 * (2 * m) + p], 0x07060302u);
+        }
+}
+template <int TX>
 __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g, int cg,
-                                                    const bf16_t *__restrict__ x, int cx, int taps, int nx, int ny,
-                                                    int nz, int chunk, float *__restrict__ part,
+                                                    const bf16_t *__restrict__ x, int cx, int nx, int ny, int nz,
+                                                    int chunk, int kt, float *__restrict__ part,
                                                     float *__restrict__ bpart) {
-    __shared__ __align__(16) bf16_t sg[kMaxCg][kTileV + 8];
-    __shared__ __align__(16) bf16_t sx[kMaxCx][kTileV + 8];
+    constexpr int NA = TX == 3 ? 12 : 4;  // products a wave owns at most: TX (cg / 16) (cxp / 16) / 4
+    constexpr int NL = TX == 3 ? 10 : 8;  // voxels a thread of x loads: its 8 and their x neighbours
+    extern __shared__ __align__(16) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 15, q = lane >> 4;
-    const int split = blockIdx.x, tap = blockIdx.y;
+    const int split = blockIdx.x, yz = blockIdx.y, taps = TX * gridDim.y;
     const int V = nx * ny * nz;
-    const int dx = tap_dx(tap, taps), dy = tap_dy(tap, taps), dz = tap_dz(tap, taps);
+    const int dy = TX == 3 ? yz % 3 - 1 : 0, dz = TX == 3 ? yz / 3 - 1 : 0;
     const int vbeg = split * chunk, vend = min(V, vbeg + chunk);
     const int cxp = (cx + 15) & ~15;
     const int nmt = cg / 16, nnt = cxp / 16, tiles = nmt * nnt;
-    f4 acc[6];
+    const int row = (kt + 8) * 2;  // bytes of an LDS row
+    unsigned char *sg = lds, *sx = lds + cg * row;
+    f4 acc[NA];
 #pragma unroll
-    for (int s = 0; s < 6; ++s) acc[s] = f4{0.f, 0.f, 0.f, 0.f};
-    const int gu = cg / 8, xu = cxp / 8;
-    // bias: in tap-0 workgroups thread (o, quarter) = (tid / 4, tid % 4) sums a quarter of row o
-    const bool bias = tap == 0 && tid < 4 * cg;
+    for (int s = 0; s < NA; ++s) acc[s] = f4{0.f, 0.f, 0.f, 0.f};
+    // the thread's unit: 8 voxels x 8 channels of g, or of x
+    const int groups = kt / 8, gunits = groups * (cg / 8), units = gunits + groups * (cxp / 8);
+    const bool is_g = tid < gunits, is_x = !is_g && tid < units;
+    const int un = is_g ? tid : tid - gunits, vg = un % groups, c8 = (un / groups) * 8;
+    const bool bias = yz == 0 && tid < 4 * cg;
     const int bo = tid >> 2, bq = tid & 3;
     float bsum = 0.f;
-    for (int vb = vbeg; vb < vend; vb += kTileV) {
-        for (int u = tid; u < kTileV * gu; u += 256) {
-            const int vl = u / gu, c8 = (u - vl * gu) * 8, v = vb + vl;
-            uint4 d = {0u, 0u, 0u, 0u};
-            if (v < vend) d = *(const uint4 *)(g + (size_t)v * cg + c8);
-            const bf16_t *e = (const bf16_t *)&d;
+    uint4 d[NL];
+    uint32_t edge = 0;  // bit i: the thread's voxel i is at x = 0; bit 8 + i: at x = nx - 1
+    auto load = [&](int vb) {
+        const int v0 = vb + 8 * vg;
+        edge = 0;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) sg[c8 + j][vl] = e[j];
-        }
-        for (int u = tid; u < kTileV * xu; u += 256) {
-            const int vl = u / xu, c8 = (u - vl * xu) * 8, v = vb + vl;
-            uint4 d = {0u, 0u, 0u, 0u};
-            if (v < vend && c8 < cx) {
-                const int xx = v % nx + dx, yy = (v / nx) % ny + dy, zz = v / (nx * ny) + dz;
-                if ((unsigned)xx < (unsigned)nx && (unsigned)yy < (unsigned)ny && (unsigned)zz < (unsigned)nz)
-                    d = *(const uint4 *)(x + (size_t)(xx + nx * (yy + ny * zz)) * cx + c8);
+        for (int i = 0; i < NL; ++i) d[i] = uint4{0u, 0u, 0u, 0u};
+        if (is_g) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (v0 + i < vend) d[i] = *(const uint4 *)(g + (size_t)(v0 + i) * cg + c8);
+        } else if (is_x && c8 < cx) {
+            if constexpr (TX == 1) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (v0 + i < vend) d[i] = *(const uint4 *)(x + (size_t)(v0 + i) * cx + c8);
+            } else {
+                // voxel v0 + i of the row at (dy, dz), and the x neighbours of the first and last
+                int xx = v0 % nx, yy = (v0 / nx) % ny, zz = v0 / (nx * ny);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int v = v0 + i;
+                    const bool in = v < vend && (unsigned)(yy + dy) < (unsigned)ny && (unsigned)(zz + dz) < (unsigned)nz;
+                    const bf16_t *p = x + ((size_t)v + (size_t)((dy + ny * dz) * nx)) * cx + c8;
+                    if (in) d[i + 1] = *(const uint4 *)p;
+                    if (i == 0 && in && xx > 0) d[0] = *(const uint4 *)(p - cx);
+                    if (i == 7 && in && xx < nx - 1) d[9] = *(const uint4 *)(p + cx);
+                    // a neighbour is also wanted where its own voxel lies past the split
+                    if (i < 7 && in && xx < nx - 1 && v + 1 >= vend) d[i + 2] = *(const uint4 *)(p + cx);
+                    edge |= (uint32_t)(xx == 0) << i | (uint32_t)(xx == nx - 1) << (8 + i);
+                    edge |= (uint32_t)in << (16 + i);
+                    if (++xx == nx) {
+                        xx = 0;
+                        if (++yy == ny) {
+                            yy = 0;
+                            ++zz;
+                        }
+                    }
+                }
             }
-            const bf16_t *e = (const bf16_t *)&d;
+        }
+    };
+    auto put = [&](unsigned char *rows, const uint4 (&v)[8]) {
+        uint4 o[8];
+        transpose8(v, o);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) sx[c8 + j][vl] = e[j];
+        for (int j = 0; j < 8; ++j) *(uint4 *)(rows + (c8 + j) * row + vg * 16) = o[j];
+    };
+    load(vbeg);
+    for (int vb = vbeg; vb < vend; vb += kt) {
+        if (is_g) {
+            uint4 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = d[i];
+            put(sg, v);
+        } else if (is_x) {
+            if constexpr (TX == 1) {
+                uint4 v[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = d[i];
+                put(sx, v);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    uint4 v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const bool off = !(edge >> (16 + i) & 1u) || (t == 0 && (edge >> i & 1u)) ||
+                                         (t == 2 && (edge >> (8 + i) & 1u));
+                        v[i] = off ? uint4{0u, 0u, 0u, 0u} : d[i + t];
+                    }
+                    put(sx + t * cxp * row, v);
+                }
+            }
         }
         __syncthreads();
+        if (vb + kt < vend) load(vb + kt);
         if (bias)
+            for (int v64 = 0; v64 < kt; v64 += 64) {
+                const uint4 *e = (const uint4 *)(sg + bo * row + (v64 + bq * 16) * 2);
 #pragma unroll
-            for (int vl = 0; vl < kTileV / 4; ++vl) bsum += bf2f(sg[bo][bq * (kTileV / 4) + vl]);
+                for (int h = 0; h < 2; ++h) {
+                    const uint4 w = e[h];
+                    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-        for (int s = 0; s < 6; ++s) {
-            const int t = wv + 4 * s;
-            if (t < tiles) {
-                const int mt = t / nnt, nt = t - mt * nnt;
+                    for (int j = 0; j < 4; ++j) {
+                        bsum += bf2f((bf16_t)(ws[j] & 0xffffu));
+                        bsum += bf2f((bf16_t)(ws[j] >> 16));
+                    }
+                }
+            }
+        // products 4 s + wave: tap t, output rows mt, input rows nt
+        for (int kh = 0; kh < kt / 32; ++kh) {
 #pragma unroll
-                for (int kh = 0; kh < kTileV / 32; ++kh) {
-                    const bf16x8 a = __builtin_bit_cast(bf16x8, *(const uint4 *)&sg[mt * 16 + r][32 * kh + 8 * q]);
-                    const bf16x8 b = __builtin_bit_cast(bf16x8, *(const uint4 *)&sx[nt * 16 + r][32 * kh + 8 * q]);
+            for (int s = 0; s < NA; ++s) {
+                const int u = wv + 4 * s;
+                if (u < TX * tiles) {
+                    const int t = u / tiles, mn = u - t * tiles, mt = mn / nnt, nt = mn - mt * nnt;
+                    const bf16x8 a = __builtin_bit_cast(
+                        bf16x8, *(const uint4 *)(sg + (mt * 16 + r) * row + 64 * kh + 16 * q));
+                    const bf16x8 b = __builtin_bit_cast(
+                        bf16x8, *(const uint4 *)(sx + (t * cxp + nt * 16 + r) * row + 64 * kh + 16 * q));
                     acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[s], 0, 0, 0);
                 }
             }
         }
         __syncthreads();
     }
-    float *out = part + ((size_t)split * taps + tap) * cg * cxp;
 #pragma unroll
-    for (int s = 0; s < 6; ++s) {
-        const int t = wv + 4 * s;
-        if (t < tiles) {
-            const int mt = t / nnt, nt = t - mt * nnt;
+    for (int s = 0; s < NA; ++s) {
+        const int u = wv + 4 * s;
+        if (u < TX * tiles) {
+            const int t = u / tiles, mn = u - t * tiles, mt = mn / nnt, nt = mn - mt * nnt;
+            float *out = part + ((size_t)split * taps + (TX == 3 ? 3 * yz + t : 0)) * cg * cxp;
 #pragma unroll
             for (int j = 0; j < 4; ++j) out[(size_t)(mt * 16 + 4 * q + j) * cxp + nt * 16 + r] = acc[s][j];
         }
     }
-    if (tap == 0) {  // uniform per workgroup
+    if (yz == 0) {  // uniform per workgroup
         __shared__ float bred[4 * kMaxCg];
         if (bias) bred[tid] = bsum;
         __syncthreads();
@@ -222,46 +389,63 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
 }
 
 // grad[(o taps + tap) ci + i] = sum over splits (in order) of part[split][tap][o][i]; the bias
-// gradient follows the weights: grad[co taps ci + o] = sum over splits of bpart[split][o]
-__global__ void k_wgrad_reduce(const float *__restrict__ part, const float *__restrict__ bpart, int nsplit, int taps,
-                               int cg, int cxp, int co, int ci, float *__restrict__ grad) {
+// gradient follows the weights: grad[co taps ci + o] = sum over splits of bpart[split][o].  The adds
+// are a serial chain per parameter (the order is fixed); its loads are not, so 16 are in flight at
+// once (the head's 1,024 splits for 221 parameters: 423 us with one load per add).
+__device__ __forceinline__ float sum_splits(const float *__restrict__ p, size_t stride, int n) {
+    float s = 0.f;
+    int i = 0;
+    for (; i + 16 <= n; i += 16) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = p[(size_t)(i + j) * stride];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s += v[j];
+    }
+    for (; i < n; ++i) s += p[(size_t)i * stride];
+    return s;
+}
+__global__ void __launch_bounds__(64) k_wgrad_reduce(const float *__restrict__ part, const float *__restrict__ bpart,
+                                                     int nsplit, int taps, int cg, int cxp, int co, int ci,
+                                                     float *__restrict__ grad) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     const int nw = co * taps * ci;
     if (n >= nw + co) return;
-    float s = 0.f;
     if (n < nw) {
         const int i = n % ci, t = (n / ci) % taps, o = n / (ci * taps);
-        for (int p = 0; p < nsplit; ++p) s += part[(((size_t)p * taps + t) * cg + o) * cxp + i];
+        grad[n] = sum_splits(part + ((size_t)t * cg + o) * cxp + i, (size_t)taps * cg * cxp, nsplit);
     } else {
-        for (int p = 0; p < nsplit; ++p) s += bpart[(size_t)p * cg + (n - nw)];
+        grad[n] = sum_splits(bpart + (n - nw), (size_t)cg, nsplit);
     }
-    grad[n] = s;
 }
 
 // ---- weight packing -----------------------------------------------------------------------------
-// forward: wp[o][tap cis + i] = W[o][tap][i] (W is [co][taps][ci] FP32), zero elsewhere
-__global__ void k_pack_fwd(const float *__restrict__ W, int co, int taps, int ci, int cis, int kpad, int rows,
-                           bf16_t *__restrict__ wp) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= rows * kpad) return;
-    const int o = n / kpad, k = n - o * kpad, t = k / cis, i = k - t * cis;
-    float v = 0.f;
-    if (o < co && t < taps && i < ci) v = W[((size_t)o * taps + t) * ci + i];
-    wp[n] = f2bf(v);
-}
-// input gradient: wt[i][tap cos + o] = W[o][taps - 1 - tap][i] (mirrored taps, transposed channels)
-__global__ void k_pack_bwd(const float *__restrict__ W, int co, int taps, int ci, int cos, int kpad, int rows,
-                           bf16_t *__restrict__ wt) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= rows * kpad) return;
-    const int i = n / kpad, k = n - i * kpad, t = k / cos, o = k - t * cos;
-    float v = 0.f;
-    if (i < ci && t < taps && o < co) v = W[((size_t)o * taps + (taps - 1 - t)) * ci + i];
-    wt[n] = f2bf(v);
-}
-__global__ void k_pack_bias(const float *__restrict__ b, int co, int rows, float *__restrict__ bp) {
-    const int o = threadIdx.x;
-    if (o < rows) bp[o] = o < co ? b[o] : 0.f;
+// All convolutions' bfloat16 copies in one launch (blockIdx.y = convolution):
+//   forward: wp[o][tap cis + i] = W[o][tap][i] (W is [co][taps][ci] FP32), zero elsewhere;
+//   input gradient: wt[i][tap cos + o] = W[o][taps - 1 - tap][i] (mirrored taps, transposed channels);
+//   bias: bp[o] = b[o], zero for padded channels.
+struct Pack {
+    const float *W, *b;
+    bf16_t *wp, *wt;
+    float *bp;
+    int co, taps, ci, cis, cos, kpad, kpadT, rows, rowsT;
+};
+__global__ void __launch_bounds__(256) k_pack(const Pack *__restrict__ packs) {
+    const Pack k = packs[blockIdx.y];
+    int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n < k.rows * k.kpad) {
+        const int o = n / k.kpad, kk = n - o * k.kpad, t = kk / k.cis, i = kk - t * k.cis;
+        k.wp[n] = f2bf(o < k.co && t < k.taps && i < k.ci ? k.W[((size_t)o * k.taps + t) * k.ci + i] : 0.f);
+        return;
+    }
+    n -= k.rows * k.kpad;
+    if (n < k.rowsT * k.kpadT) {
+        const int i = n / k.kpadT, kk = n - i * k.kpadT, t = kk / k.cos, o = kk - t * k.cos;
+        k.wt[n] = f2bf(i < k.ci && t < k.taps && o < k.co ? k.W[((size_t)o * k.taps + (k.taps - 1 - t)) * k.ci + i] : 0.f);
+        return;
+    }
+    n -= k.rowsT * k.kpadT;
+    if (n < k.rows) k.bp[n] = n < k.co ? k.b[n] : 0.f;
 }
 
 // ---- elementwise pieces ---------------------------------------------------------------------------
@@ -299,32 +483,61 @@ __global__ void k_scatter(const float *__restrict__ y, int cs, int nf, int V, Fi
     F.f[c][v] = fmin(fmax(f, F.lo[c]), F.hi[c]);
 }
 
+// The elementwise kernels below take 8 channels (16 bytes of bfloat16) per thread: bandwidth-bound
+// copies and sums, which 2-byte accesses left at a few hundred GB/s (the level-1 concatenation at
+// 96x96x48, 85 MB: 122 us).
+__device__ __forceinline__ void unpack8(const bf16_t *p, float (&v)[8]) {
+    const uint4 d = *(const uint4 *)p;
+    const uint32_t w[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[2 * j] = bf2f((bf16_t)(w[j] & 0xffffu));
+        v[2 * j + 1] = bf2f((bf16_t)(w[j] >> 16));
+    }
+}
+__device__ __forceinline__ void pack8(bf16_t *p, const float (&v)[8]) {
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = (uint32_t)f2bf(v[2 * j]) | (uint32_t)f2bf(v[2 * j + 1]) << 16;
+    *(uint4 *)p = uint4{w[0], w[1], w[2], w[3]};
+}
 // 2x2x2 average pooling, fine grid (nx, ny, nz)
-__global__ void k_pool(const bf16_t *__restrict__ x, int C, int nx, int ny, int nz, bf16_t *__restrict__ out) {
-    const int mx = nx / 2, my = ny / 2, mz = nz / 2;
+__global__ void __launch_bounds__(256) k_pool(const bf16_t *__restrict__ x, int C, int nx, int ny, int nz,
+                                              bf16_t *__restrict__ out) {
+    const int mx = nx / 2, my = ny / 2, mz = nz / 2, U = C / 8;
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= mx * my * mz * C) return;
-    const int c = n % C, vc = n / C;
+    if (n >= mx * my * mz * U) return;
+    const int c = (n % U) * 8, vc = n / U;
     const int i = vc % mx, j = (vc / mx) % my, k = vc / (mx * my);
-    float s = 0.f;
-    for (int e = 0; e < 2; ++e)
-        for (int b = 0; b < 2; ++b)
-            for (int a = 0; a < 2; ++a) s += bf2f(x[((size_t)(2 * i + a) + nx * ((2 * j + b) + ny * (2 * k + e))) * C + c]);
-    out[n] = f2bf(s * 0.125f);
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ch = 0; ch < 8; ++ch) {  // x fastest
+        const int a = ch & 1, b = ch >> 1 & 1, e = ch >> 2;
+        float v[8];
+        unpack8(x + ((size_t)(2 * i + a) + nx * ((2 * j + b) + ny * (2 * k + e))) * C + c, v);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) s[t] += v[t];
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) s[t] *= 0.125f;
+    pack8(out + (size_t)vc * C + c, s);
 }
 // out[v] = [coarse[parent(v)] (cu channels), skip[v] (cs channels)]
-__global__ void k_upcat(const bf16_t *__restrict__ coarse, int cu, const bf16_t *__restrict__ skip, int cs, int nx,
-                        int ny, int nz, bf16_t *__restrict__ out) {
-    const int C = cu + cs;
+__global__ void __launch_bounds__(256) k_upcat(const bf16_t *__restrict__ coarse, int cu,
+                                               const bf16_t *__restrict__ skip, int cs, int nx, int ny, int nz,
+                                               bf16_t *__restrict__ out) {
+    const int U = (cu + cs) / 8;
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= nx * ny * nz * C) return;
-    const int c = n % C, v = n / C;
+    if (n >= nx * ny * nz * U) return;
+    const int c = (n % U) * 8, v = n / U;
+    uint4 d;
     if (c < cu) {
         const int i = v % nx, j = (v / nx) % ny, k = v / (nx * ny);
-        out[n] = coarse[((size_t)(i / 2) + (nx / 2) * ((j / 2) + (ny / 2) * (k / 2))) * cu + c];
+        d = *(const uint4 *)(coarse + ((size_t)(i / 2) + (nx / 2) * ((j / 2) + (ny / 2) * (k / 2))) * cu + c);
     } else {
-        out[n] = skip[(size_t)v * cs + (c - cu)];
+        d = *(const uint4 *)(skip + (size_t)v * cs + (c - cu));
     }
+    *(uint4 *)(out + (size_t)n * 8) = d;
 }
 // g[v][c] = bf16(2 (y - t) / (V nf)) for c < nf, zero to cs; lpart[block] = sum of (y - t)^2
 __global__ void __launch_bounds__(256) k_loss(const float *__restrict__ y, const float *__restrict__ t, int cs, int nf,
@@ -361,38 +574,53 @@ __global__ void __launch_bounds__(256) k_loss_final(const float *__restrict__ lp
     }
     if (threadIdx.x == 0) out[0] = red[0] * inv;
 }
-// out[v][c] = act[v][c] > 0 ? bf16(d[v][c]) : 0   (d has stride cd)
-__global__ void k_relu_bwd(const float *__restrict__ d, int cd, const bf16_t *__restrict__ act, int C, int V,
-                           bf16_t *__restrict__ out) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= V * C) return;
-    const int v = n / C, c = n - v * C;
-    out[n] = bf2f(act[n]) > 0.f ? f2bf(d[(size_t)v * cd + c]) : (bf16_t)0;
+__device__ __forceinline__ void unpack8(const float *p, float (&v)[8]) {
+    const f4 a = *(const f4 *)p, b = *(const f4 *)(p + 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[j] = a[j];
+        v[4 + j] = b[j];
+    }
 }
 // coarse grid: out[vc][c] = act > 0 ? bf16(sum over the 8 children of d[v][c]) : 0  (fine dims given)
-__global__ void k_up_bwd(const float *__restrict__ d, int cd, const bf16_t *__restrict__ act, int C, int nx, int ny,
-                         int nz, bf16_t *__restrict__ out) {
-    const int mx = nx / 2, my = ny / 2, mz = nz / 2;
+__global__ void __launch_bounds__(256) k_up_bwd(const float *__restrict__ d, int cd, const bf16_t *__restrict__ act,
+                                                int C, int nx, int ny, int nz, bf16_t *__restrict__ out) {
+    const int mx = nx / 2, my = ny / 2, mz = nz / 2, U = C / 8;
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= mx * my * mz * C) return;
-    const int c = n % C, vc = n / C;
+    if (n >= mx * my * mz * U) return;
+    const int c = (n % U) * 8, vc = n / U;
     const int i = vc % mx, j = (vc / mx) % my, k = vc / (mx * my);
-    float s = 0.f;
-    for (int e = 0; e < 2; ++e)
-        for (int b = 0; b < 2; ++b)
-            for (int a = 0; a < 2; ++a) s += d[((size_t)(2 * i + a) + nx * ((2 * j + b) + ny * (2 * k + e))) * cd + c];
-    out[n] = bf2f(act[n]) > 0.f ? f2bf(s) : (bf16_t)0;
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, on[8];
+#pragma unroll
+    for (int ch = 0; ch < 8; ++ch) {
+        const int a = ch & 1, b = ch >> 1 & 1, e = ch >> 2;
+        float v[8];
+        unpack8(d + ((size_t)(2 * i + a) + nx * ((2 * j + b) + ny * (2 * k + e))) * cd + c, v);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) s[t] += v[t];
+    }
+    unpack8(act + (size_t)n * 8, on);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) s[t] = on[t] > 0.f ? s[t] : 0.f;
+    pack8(out + (size_t)n * 8, s);
 }
 // fine grid: out[v][c] = act > 0 ? bf16(skip[v][off + c] + dc[parent(v)][c] / 8) : 0
-__global__ void k_pool_bwd(const float *__restrict__ dc, const float *__restrict__ skip, int cskip, int off,
-                           const bf16_t *__restrict__ act, int C, int nx, int ny, int nz, bf16_t *__restrict__ out) {
+__global__ void __launch_bounds__(256) k_pool_bwd(const float *__restrict__ dc, const float *__restrict__ skip,
+                                                  int cskip, int off, const bf16_t *__restrict__ act, int C, int nx,
+                                                  int ny, int nz, bf16_t *__restrict__ out) {
+    const int U = C / 8;
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= nx * ny * nz * C) return;
-    const int c = n % C, v = n / C;
+    if (n >= nx * ny * nz * U) return;
+    const int c = (n % U) * 8, v = n / U;
     const int i = v % nx, j = (v / nx) % ny, k = v / (nx * ny);
     const size_t p = (size_t)(i / 2) + (nx / 2) * ((j / 2) + (ny / 2) * (k / 2));
-    const float s = skip[(size_t)v * cskip + off + c] + dc[p * C + c] * 0.125f;
-    out[n] = bf2f(act[n]) > 0.f ? f2bf(s) : (bf16_t)0;
+    float s[8], h[8], on[8];
+    unpack8(skip + (size_t)v * cskip + off + c, s);
+    unpack8(dc + p * C + c, h);
+    unpack8(act + (size_t)n * 8, on);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) s[t] = on[t] > 0.f ? s[t] + h[t] * 0.125f : 0.f;
+    pack8(out + (size_t)n * 8, s);
 }
 // Adam (Kingma & Ba 2015, Algorithm 1); bc1 = 1 - beta1^t, bc2 = 1 - beta2^t
 __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
@@ -454,6 +682,8 @@ struct lbm_unet {
     float *dx1, *dx2, *dxt, *wpart, *bpart, *lpart;
     double *dloss, *hloss;
     size_t wpart_n = 0, bpart_n = 0;
+    Pack *packs = nullptr;  // the convolutions' packing tables, on the device
+    size_t pack_n = 0;      // the most values one of them packs
     bool have_target = false;
 };
 
@@ -477,21 +707,48 @@ int alloc(lbm_unet *N, T **p, size_t n) {
     return LBM_OK;
 }
 
-int launch_conv(lbm_unet *N, const bf16_t *x, int cin, int taps, const bf16_t *w, int kpad, const float *bias,
-                bf16_t *y, float *y32, int cstore, int creal, int relu, const int *d) {
-    const int V = d[0] * d[1] * d[2];
-    const int tiles = cstore > 0 ? r16(cstore) / 16 : 0;
-    int MT = tiles % 4 == 0 ? 4 : (tiles % 3 == 0 ? 3 : (tiles % 2 == 0 ? 2 : 1));
-    if (cin % 8 || kpad % 32 || tiles <= 0) return lbm::set_error(LBM_ERR_ARG, "conv shape: cin %d kpad %d", cin, kpad);
-    dim3 grid(blocks(V, 256), tiles / MT);
-    switch (MT) {
-    case 4: k_conv<4><<<grid, 256, 0, N->s>>>(x, cin, taps, w, kpad, bias, y, y32, cstore, creal, relu, d[0], d[1], d[2]); break;
-    case 3: k_conv<3><<<grid, 256, 0, N->s>>>(x, cin, taps, w, kpad, bias, y, y32, cstore, creal, relu, d[0], d[1], d[2]); break;
-    case 2: k_conv<2><<<grid, 256, 0, N->s>>>(x, cin, taps, w, kpad, bias, y, y32, cstore, creal, relu, d[0], d[1], d[2]); break;
-    default: k_conv<1><<<grid, 256, 0, N->s>>>(x, cin, taps, w, kpad, bias, y, y32, cstore, creal, relu, d[0], d[1], d[2]); break;
-    }
+template <int CIN, int MT, int WM, int WN>
+int launch_conv3(lbm_unet *N, const bf16_t *x, const bf16_t *w, const ConvOut &out, int tiles, const int *d) {
+    const int ntx = (d[0] + 15) / 16, nty = (d[1] + 3) / 4, ntz = (d[2] + WN - 1) / WN;
+    const int lds = 18 * 6 * (WN + 2) * Brick<CIN>::VS;
+    if (lds > 65536)
+        UCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_conv3<CIN, MT, WM, WN>),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    k_conv3<CIN, MT, WM, WN><<<dim3(ntx * nty * ntz, tiles / (MT * WM)), 64 * WM * WN, lds, N->s>>>(
+        x, w, out, d[0], d[1], d[2], ntx, nty);
     UCHK(hipGetLastError());
     return LBM_OK;
+}
+// The network's shapes.  The waves of a workgroup share its brick: across the output channels as far
+// as there are tiles of 16 (every one of them would otherwise stage the same voxels), the rest along z;
+// three tiles to a wave where their number is a multiple of three.  At 96x96x48, 16 -> 16 channels:
+// 58 us before.
+int launch_conv(lbm_unet *N, const bf16_t *x, int cin, int taps, const bf16_t *w, int kpad, const ConvOut &out,
+                const int *d) {
+    const int V = d[0] * d[1] * d[2];
+    const int tiles = out.cstore > 0 ? out.cstore / 16 : 0;
+    if (cin % 8 || kpad % 32 || tiles <= 0 || out.cstore % 16)
+        return lbm::set_error(LBM_ERR_ARG, "conv shape: cin %d kpad %d", cin, kpad);
+    if (taps == 1) {
+        k_conv1<<<dim3(blocks(V, 256), tiles), 256, 0, N->s>>>(x, cin, w, kpad, out, V);
+        UCHK(hipGetLastError());
+        return LBM_OK;
+    }
+    switch (100 * cin + tiles) {
+    case 801: return launch_conv3<8, 1, 1, 4>(N, x, w, out, tiles, d);
+    case 1601: return launch_conv3<16, 1, 1, 4>(N, x, w, out, tiles, d);
+    case 1602: return launch_conv3<16, 1, 2, 2>(N, x, w, out, tiles, d);
+    case 1603: return launch_conv3<16, 3, 1, 4>(N, x, w, out, tiles, d);
+    case 3201: return launch_conv3<32, 1, 1, 4>(N, x, w, out, tiles, d);
+    case 3202: return launch_conv3<32, 1, 2, 2>(N, x, w, out, tiles, d);
+    case 3204: return launch_conv3<32, 1, 4, 1>(N, x, w, out, tiles, d);
+    case 3206: return launch_conv3<32, 3, 2, 2>(N, x, w, out, tiles, d);
+    case 4801: return launch_conv3<48, 1, 1, 4>(N, x, w, out, tiles, d);
+    case 6402: return launch_conv3<64, 1, 2, 2>(N, x, w, out, tiles, d);
+    case 6404: return launch_conv3<64, 1, 4, 1>(N, x, w, out, tiles, d);
+    case 9602: return launch_conv3<96, 1, 2, 1>(N, x, w, out, tiles, d);
+    }
+    return lbm::set_error(LBM_ERR_ARG, "conv shape: cin %d, %d output tiles", cin, tiles);
 }
 
 // splits of a voxel range for the weight gradient: about 1024 workgroups over all taps
@@ -514,11 +771,22 @@ int conv_grads(lbm_unet *N, const lbm_unet::Conv &c, const bf16_t *g, const bf16
     wsplit(V, c.taps, &nsplit, &chunk);
     if ((size_t)nsplit * c.taps * cg * cxp > N->wpart_n) return lbm::set_error(LBM_ERR_ARG, "weight partials overflow");
     if ((size_t)nsplit * cg > N->bpart_n) return lbm::set_error(LBM_ERR_ARG, "bias partials overflow");
-    k_conv_wgrad<<<dim3(nsplit, c.taps), 256, 0, N->s>>>(g, cg, x, c.cis, c.taps, d[0], d[1], d[2], chunk, N->wpart,
-                                                         N->bpart);
+    const int tx = c.taps == 27 ? 3 : 1, tiles = tx * (cg / 16) * (cxp / 16);
+    if (tiles > (tx == 3 ? 48 : 16)) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d tiles", tiles);
+    // voxels per LDS tile: the most for which a thread has one unit and the rows fit 64 kB
+    int kt = 256;
+    auto rows = [&](int k) { return (cg + tx * cxp) * (k + 8) * 2; };
+    while (kt > kTileV && (kt / 8 * (cg + cxp) / 8 > 256 || rows(kt) > 65536 - 4 * kMaxCg * (int)sizeof(float))) kt /= 2;
+    if (kt / 8 * (cg + cxp) / 8 > 256) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d x %d channels", cg, cxp);
+    if (tx == 3)
+        k_conv_wgrad<3><<<dim3(nsplit, 9), 256, rows(kt), N->s>>>(g, cg, x, c.cis, d[0], d[1], d[2], chunk, kt, N->wpart,
+                                                                  N->bpart);
+    else
+        k_conv_wgrad<1><<<dim3(nsplit, 1), 256, rows(kt), N->s>>>(g, cg, x, c.cis, d[0], d[1], d[2], chunk, kt, N->wpart,
+                                                                  N->bpart);
     UCHK(hipGetLastError());
     const int nw = c.co * c.taps * c.ci;  // the bias follows the weights in the parameter vector
-    k_wgrad_reduce<<<blocks(nw + c.co), 256, 0, N->s>>>(N->wpart, N->bpart, nsplit, c.taps, cg, cxp, c.co, c.ci,
+    k_wgrad_reduce<<<blocks(nw + c.co, 64), 64, 0, N->s>>>(N->wpart, N->bpart, nsplit, c.taps, cg, cxp, c.co, c.ci,
                                                          N->g + c.wo);
     UCHK(hipGetLastError());
     return LBM_OK;
@@ -526,23 +794,18 @@ int conv_grads(lbm_unet *N, const lbm_unet::Conv &c, const bf16_t *g, const bf16
 
 int conv_fwd(lbm_unet *N, int i, const bf16_t *x, bf16_t *y, float *y32, int relu) {
     const auto &c = N->conv[i];
-    return launch_conv(N, x, c.cis, c.taps, c.wp, c.kpad, c.bp, y, y32, r16(c.co), c.co, relu, N->dims[c.level]);
+    return launch_conv(N, x, c.cis, c.taps, c.wp, c.kpad, ConvOut{c.bp, y, y32, nullptr, r16(c.co), c.co, relu},
+                       N->dims[c.level]);
 }
-// input gradient of conv i into dx (FP32, cis channels)
-int conv_dx(lbm_unet *N, int i, const bf16_t *g, float *dx) {
+// input gradient of conv i (cis channels): into dx as FP32, or through the ReLU that gave act, into gb
+int conv_dx(lbm_unet *N, int i, const bf16_t *g, float *dx, bf16_t *gb = nullptr, const bf16_t *act = nullptr) {
     const auto &c = N->conv[i];
-    return launch_conv(N, g, r16(c.co), c.taps, c.wt, c.kpadT, nullptr, nullptr, dx, c.cis, c.cis, 0, N->dims[c.level]);
+    return launch_conv(N, g, r16(c.co), c.taps, c.wt, c.kpadT, ConvOut{nullptr, gb, dx, act, c.cis, c.cis, 0},
+                       N->dims[c.level]);
 }
 
 int repack(lbm_unet *N) {
-    for (auto &c : N->conv) {
-        const int rows = r16(c.co);
-        k_pack_fwd<<<blocks((size_t)rows * c.kpad), 256, 0, N->s>>>(N->p + c.wo, c.co, c.taps, c.ci, c.cis, c.kpad,
-                                                                   rows, c.wp);
-        k_pack_bwd<<<blocks((size_t)c.rowsT * c.kpadT), 256, 0, N->s>>>(N->p + c.wo, c.co, c.taps, c.ci, r16(c.co),
-                                                                        c.kpadT, c.rowsT, c.wt);
-        k_pack_bias<<<1, 64, 0, N->s>>>(N->p + c.bo, c.co, rows, c.bp);
-    }
+    k_pack<<<dim3(blocks(N->pack_n), (unsigned)N->conv.size()), 256, 0, N->s>>>(N->packs);
     UCHK(hipGetLastError());
     return LBM_OK;
 }
@@ -557,16 +820,16 @@ int forward(lbm_unet *N) {
     F(conv_fwd(N, E1A, N->x0, N->e1a, nullptr, 1));
     F(conv_fwd(N, E1B, N->e1a, N->e1b, nullptr, 1));
     const int *d1 = N->dims[0], *d2 = N->dims[1];
-    k_pool<<<blocks((size_t)N->V[1] * c1), 256, 0, N->s>>>(N->e1b, c1, d1[0], d1[1], d1[2], N->p1);
+    k_pool<<<blocks((size_t)N->V[1] * c1 / 8), 256, 0, N->s>>>(N->e1b, c1, d1[0], d1[1], d1[2], N->p1);
     F(conv_fwd(N, E2A, N->p1, N->e2a, nullptr, 1));
     F(conv_fwd(N, E2B, N->e2a, N->e2b, nullptr, 1));
-    k_pool<<<blocks((size_t)N->V[2] * c2), 256, 0, N->s>>>(N->e2b, c2, d2[0], d2[1], d2[2], N->p2);
+    k_pool<<<blocks((size_t)N->V[2] * c2 / 8), 256, 0, N->s>>>(N->e2b, c2, d2[0], d2[1], d2[2], N->p2);
     F(conv_fwd(N, E3A, N->p2, N->e3a, nullptr, 1));
     F(conv_fwd(N, E3B, N->e3a, N->e3b, nullptr, 1));
-    k_upcat<<<blocks((size_t)N->V[1] * (c3 + c2)), 256, 0, N->s>>>(N->e3b, c3, N->e2b, c2, d2[0], d2[1], d2[2], N->cat2);
+    k_upcat<<<blocks((size_t)N->V[1] * (c3 + c2) / 8), 256, 0, N->s>>>(N->e3b, c3, N->e2b, c2, d2[0], d2[1], d2[2], N->cat2);
     F(conv_fwd(N, D2A, N->cat2, N->d2a, nullptr, 1));
     F(conv_fwd(N, D2B, N->d2a, N->d2b, nullptr, 1));
-    k_upcat<<<blocks((size_t)N->V[0] * (c2 + c1)), 256, 0, N->s>>>(N->d2b, c2, N->e1b, c1, d1[0], d1[1], d1[2], N->cat1);
+    k_upcat<<<blocks((size_t)N->V[0] * (c2 + c1) / 8), 256, 0, N->s>>>(N->d2b, c2, N->e1b, c1, d1[0], d1[1], d1[2], N->cat1);
     F(conv_fwd(N, D1A, N->cat1, N->d1a, nullptr, 1));
     F(conv_fwd(N, D1B, N->d1a, N->d1b, nullptr, 1));
     F(conv_fwd(N, HEAD, N->d1b, nullptr, N->y32, 0));
@@ -584,41 +847,35 @@ int backward(lbm_unet *N) {
     k_loss_final<<<1, 256, 0, N->s>>>(N->lpart, nl, 1.0 / ((double)V1 * N->cout), N->dloss);
     // head and level-1 decoder
     F(conv_grads(N, N->conv[HEAD], N->gb0, N->d1b));
-    F(conv_dx(N, HEAD, N->gb0, N->dxt));
-    k_relu_bwd<<<blocks((size_t)V1 * c1), 256, 0, N->s>>>(N->dxt, c1, N->d1b, c1, V1, N->gb1);
+    F(conv_dx(N, HEAD, N->gb0, nullptr, N->gb1, N->d1b));
     F(conv_grads(N, N->conv[D1B], N->gb1, N->d1a));
-    F(conv_dx(N, D1B, N->gb1, N->dxt));
-    k_relu_bwd<<<blocks((size_t)V1 * c1), 256, 0, N->s>>>(N->dxt, c1, N->d1a, c1, V1, N->gb0);
+    F(conv_dx(N, D1B, N->gb1, nullptr, N->gb0, N->d1a));
     F(conv_grads(N, N->conv[D1A], N->gb0, N->cat1));
     F(conv_dx(N, D1A, N->gb0, N->dx1));  // [V1][c2 + c1]: upsampled part, then the skip of e1b
-    k_up_bwd<<<blocks((size_t)V2 * c2), 256, 0, N->s>>>(N->dx1, c2 + c1, N->d2b, c2, d1[0], d1[1], d1[2], N->gb1);
+    k_up_bwd<<<blocks((size_t)V2 * c2 / 8), 256, 0, N->s>>>(N->dx1, c2 + c1, N->d2b, c2, d1[0], d1[1], d1[2], N->gb1);
     // level-2 decoder
     F(conv_grads(N, N->conv[D2B], N->gb1, N->d2a));
-    F(conv_dx(N, D2B, N->gb1, N->dxt));
-    k_relu_bwd<<<blocks((size_t)V2 * c2), 256, 0, N->s>>>(N->dxt, c2, N->d2a, c2, V2, N->gb0);
+    F(conv_dx(N, D2B, N->gb1, nullptr, N->gb0, N->d2a));
     F(conv_grads(N, N->conv[D2A], N->gb0, N->cat2));
     F(conv_dx(N, D2A, N->gb0, N->dx2));  // [V2][c3 + c2]
-    k_up_bwd<<<blocks((size_t)V3 * c3), 256, 0, N->s>>>(N->dx2, c3 + c2, N->e3b, c3, d2[0], d2[1], d2[2], N->gb1);
+    k_up_bwd<<<blocks((size_t)V3 * c3 / 8), 256, 0, N->s>>>(N->dx2, c3 + c2, N->e3b, c3, d2[0], d2[1], d2[2], N->gb1);
     // bottleneck
     F(conv_grads(N, N->conv[E3B], N->gb1, N->e3a));
-    F(conv_dx(N, E3B, N->gb1, N->dxt));
-    k_relu_bwd<<<blocks((size_t)V3 * c3), 256, 0, N->s>>>(N->dxt, c3, N->e3a, c3, V3, N->gb0);
+    F(conv_dx(N, E3B, N->gb1, nullptr, N->gb0, N->e3a));
     F(conv_grads(N, N->conv[E3A], N->gb0, N->p2));
     F(conv_dx(N, E3A, N->gb0, N->dxt));  // [V3][c2]
-    k_pool_bwd<<<blocks((size_t)V2 * c2), 256, 0, N->s>>>(N->dxt, N->dx2, c3 + c2, c3, N->e2b, c2, d2[0], d2[1], d2[2],
+    k_pool_bwd<<<blocks((size_t)V2 * c2 / 8), 256, 0, N->s>>>(N->dxt, N->dx2, c3 + c2, c3, N->e2b, c2, d2[0], d2[1], d2[2],
                                                          N->gb1);
     // level-2 encoder
     F(conv_grads(N, N->conv[E2B], N->gb1, N->e2a));
-    F(conv_dx(N, E2B, N->gb1, N->dxt));
-    k_relu_bwd<<<blocks((size_t)V2 * c2), 256, 0, N->s>>>(N->dxt, c2, N->e2a, c2, V2, N->gb0);
+    F(conv_dx(N, E2B, N->gb1, nullptr, N->gb0, N->e2a));
     F(conv_grads(N, N->conv[E2A], N->gb0, N->p1));
     F(conv_dx(N, E2A, N->gb0, N->dxt));  // [V2][c1]
-    k_pool_bwd<<<blocks((size_t)V1 * c1), 256, 0, N->s>>>(N->dxt, N->dx1, c2 + c1, c2, N->e1b, c1, d1[0], d1[1], d1[2],
+    k_pool_bwd<<<blocks((size_t)V1 * c1 / 8), 256, 0, N->s>>>(N->dxt, N->dx1, c2 + c1, c2, N->e1b, c1, d1[0], d1[1], d1[2],
                                                          N->gb1);
     // level-1 encoder
     F(conv_grads(N, N->conv[E1B], N->gb1, N->e1a));
-    F(conv_dx(N, E1B, N->gb1, N->dxt));
-    k_relu_bwd<<<blocks((size_t)V1 * c1), 256, 0, N->s>>>(N->dxt, c1, N->e1a, c1, V1, N->gb0);
+    F(conv_dx(N, E1B, N->gb1, nullptr, N->gb0, N->e1a));
     F(conv_grads(N, N->conv[E1A], N->gb0, N->x0));
 #undef F
     UCHK(hipGetLastError());
@@ -799,6 +1056,7 @@ int lbm_unet_create(lbm_context *ctx, int nx, int ny, int nz, int cin, int cout,
     A(N->bpart, N->bpart_n);
     A(N->lpart, blocks(V1 * r16(cout)));
     A(N->dloss, 1);
+    A(N->packs, N->conv.size());
 #undef A
     if (rc == LBM_OK && hipHostMalloc(&N->hloss, sizeof(double), hipHostMallocDefault) != hipSuccess)
         rc = lbm::set_error(LBM_ERR_HIP, "hipHostMalloc failed");
@@ -821,6 +1079,14 @@ int lbm_unet_create(lbm_context *ctx, int nx, int ny, int nz, int cin, int cout,
     if (e == hipSuccess) e = hipMemsetAsync(N->g, 0, N->np * sizeof(float), N->s);
     if (e == hipSuccess) e = hipMemsetAsync(N->x0, 0, V1 * 8 * sizeof(bf16_t), N->s);
     if (e == hipSuccess) e = hipMemsetAsync(N->tgt, 0, V1 * r16(cout) * sizeof(float), N->s);
+    std::vector<Pack> packs;
+    for (const auto &c : N->conv) {
+        packs.push_back(Pack{N->p + c.wo, N->p + c.bo, c.wp, c.wt, c.bp, c.co, c.taps, c.ci, c.cis, r16(c.co), c.kpad,
+                             c.kpadT, r16(c.co), c.rowsT});
+        N->pack_n = std::max(N->pack_n, (size_t)r16(c.co) * (c.kpad + 1) + (size_t)c.rowsT * c.kpadT);
+    }
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(N->packs, packs.data(), packs.size() * sizeof(Pack), hipMemcpyHostToDevice, N->s);
     if (e == hipSuccess) e = hipStreamSynchronize(N->s);
     if (e != hipSuccess) {
         destroy(N);
