@@ -159,15 +159,25 @@ __global__ void __launch_bounds__(64 * WM * WN) k_conv3(const bf16_t *__restrict
     const int wm = wv % WM, wn = wv / WM;
     const int bx = blockIdx.x % ntx, by = (blockIdx.x / ntx) % nty, bz = blockIdx.x / (ntx * nty);
     const int x0 = bx * 16, y0 = by * 4, z0 = bz * WN;
-    constexpr int CU = CIN / 8;
-    for (int u = tid; u < NV * CU; u += THREADS) {
-        const int vox = u / CU, c = u - vox * CU;
-        const int px = vox % 18, py = (vox / 18) % 6, pz = vox / 108;
-        const int xx = x0 + px - 1, yy = y0 + py - 1, zz = z0 + pz - 1;
-        uint4 d = {0u, 0u, 0u, 0u};
-        if ((unsigned)xx < (unsigned)nx && (unsigned)yy < (unsigned)ny && (unsigned)zz < (unsigned)nz)
-            d = *(const uint4 *)(x + (size_t)(xx + nx * (yy + ny * zz)) * CIN + 8 * c);
-        *(uint4 *)(lds + vox * VS + 16 * c) = d;
+    // loads from clamped addresses, zeroed afterwards, so that a batch of them is in flight at once
+    constexpr int CU = CIN / 8, UNITS = NV * CU, IT = (UNITS + THREADS - 1) / THREADS, BATCH = IT < 8 ? IT : 8;
+#pragma unroll
+    for (int it = 0; it < IT; it += BATCH) {
+        uint4 d[BATCH];
+        bool in[BATCH];
+#pragma unroll
+        for (int h = 0; h < BATCH; ++h) {
+            const int u = min(tid + (it + h) * THREADS, UNITS - 1), vox = u / CU, c = u - vox * CU;
+            const int xx = x0 + vox % 18 - 1, yy = y0 + (vox / 18) % 6 - 1, zz = z0 + vox / 108 - 1;
+            in[h] = (unsigned)xx < (unsigned)nx && (unsigned)yy < (unsigned)ny && (unsigned)zz < (unsigned)nz;
+            const int v = in[h] ? xx + nx * (yy + ny * zz) : 0;
+            d[h] = *(const uint4 *)(x + (size_t)v * CIN + 8 * c);
+        }
+#pragma unroll
+        for (int h = 0; h < BATCH; ++h) {
+            const int u = tid + (it + h) * THREADS, vox = u / CU, c = u - vox * CU;
+            if (u < UNITS) *(uint4 *)(lds + vox * VS + 16 * c) = in[h] ? d[h] : uint4{0u, 0u, 0u, 0u};
+        }
     }
     f4 acc[MT][NT];
 #pragma unroll
@@ -238,61 +248,74 @@ __device__ __forceinline__ void transpose8(const uint4 (&d)[8], uint4 (&o)[8]) {
 template <int TX>
 __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g, int cg,
                                                     const bf16_t *__restrict__ x, int cx, int nx, int ny, int nz,
-                                                    int chunk, int kt, float *__restrict__ part,
+                                                    int chunk, int kt, int cxg, float *__restrict__ part,
                                                     float *__restrict__ bpart) {
     constexpr int NA = TX == 3 ? 12 : 4;  // products a wave owns at most: TX (cg / 16) (cxp / 16) / 4
     constexpr int NL = TX == 3 ? 10 : 8;  // voxels a thread of x loads: its 8 and their x neighbours
     extern __shared__ __align__(16) unsigned char lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 15, q = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int split = blockIdx.x, yz = blockIdx.y, taps = TX * gridDim.y;
     const int V = nx * ny * nz;
     const int dy = TX == 3 ? yz % 3 - 1 : 0, dz = TX == 3 ? yz / 3 - 1 : 0;
     const int vbeg = split * chunk, vend = min(V, vbeg + chunk);
     const int cxp = (cx + 15) & ~15;
-    const int nmt = cg / 16, nnt = cxp / 16, tiles = nmt * nnt;
+    const int xo = blockIdx.z * cxg;  // this workgroup's input channels: [xo, xo + cxg)
+    const int nmt = cg / 16, nnt = cxg / 16, tiles = nmt * nnt;
     const int row = (kt + 8) * 2;  // bytes of an LDS row
     unsigned char *sg = lds, *sx = lds + cg * row;
+    // products 4 s + wave: tap t, output rows mt, input rows nt
     f4 acc[NA];
+    int arow[NA], brow[NA];
 #pragma unroll
-    for (int s = 0; s < NA; ++s) acc[s] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < NA; ++s) {
+        acc[s] = f4{0.f, 0.f, 0.f, 0.f};
+        const int u = min(wv + 4 * s, TX * tiles - 1);
+        const int t = u / tiles, mn = u - t * tiles, mt = mn / nnt, nt = mn - mt * nnt;
+        arow[s] = mt * 16 * row;
+        brow[s] = (t * cxg + nt * 16) * row;
+    }
     // the thread's unit: 8 voxels x 8 channels of g, or of x
-    const int groups = kt / 8, gunits = groups * (cg / 8), units = gunits + groups * (cxp / 8);
+    const int groups = kt / 8, gunits = groups * (cg / 8), units = gunits + groups * (cxg / 8);
     const bool is_g = tid < gunits, is_x = !is_g && tid < units;
     const int un = is_g ? tid : tid - gunits, vg = un % groups, c8 = (un / groups) * 8;
-    const bool bias = yz == 0 && tid < 4 * cg;
+    const bool bias = yz == 0 && xo == 0 && tid < 4 * cg;
     const int bo = tid >> 2, bq = tid & 3;
     float bsum = 0.f;
     uint4 d[NL];
-    uint32_t edge = 0;  // bit i: the thread's voxel i is at x = 0; bit 8 + i: at x = nx - 1
+    // bit i: the thread's voxel i is at x = 0; 8 + i: at x = nx - 1; 16 + i: it counts (in the split, its
+    // row at (dy, dz) in the grid).  Loads go to clamped addresses and are masked when they are used:
+    // a load under a condition is waited for before the next one is issued.
+    uint32_t edge = 0;
     auto load = [&](int vb) {
         const int v0 = vb + 8 * vg;
         edge = 0;
-#pragma unroll
-        for (int i = 0; i < NL; ++i) d[i] = uint4{0u, 0u, 0u, 0u};
         if (is_g) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (v0 + i < vend) d[i] = *(const uint4 *)(g + (size_t)(v0 + i) * cg + c8);
-        } else if (is_x && c8 < cx) {
+            for (int i = 0; i < 8; ++i) {
+                d[i] = *(const uint4 *)(g + (size_t)min(v0 + i, V - 1) * cg + c8);
+                edge |= (uint32_t)(v0 + i < vend) << (16 + i);
+            }
+        } else if (is_x) {
+            const bool real = xo + c8 < cx;
+            const int cl = real ? xo + c8 : 0;
             if constexpr (TX == 1) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (v0 + i < vend) d[i] = *(const uint4 *)(x + (size_t)(v0 + i) * cx + c8);
+                for (int i = 0; i < 8; ++i) {
+                    d[i] = *(const uint4 *)(x + (size_t)min(v0 + i, V - 1) * cx + cl);
+                    edge |= (uint32_t)(v0 + i < vend && real) << (16 + i);
+                }
             } else {
-                // voxel v0 + i of the row at (dy, dz), and the x neighbours of the first and last
+                const int l0 = v0 - 1 + (dy + ny * dz) * nx;
+#pragma unroll
+                for (int i = 0; i < 10; ++i)
+                    d[i] = *(const uint4 *)(x + (size_t)min(max(l0 + i, 0), V - 1) * cx + cl);
                 int xx = v0 % nx, yy = (v0 / nx) % ny, zz = v0 / (nx * ny);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    const int v = v0 + i;
-                    const bool in = v < vend && (unsigned)(yy + dy) < (unsigned)ny && (unsigned)(zz + dz) < (unsigned)nz;
-                    const bf16_t *p = x + ((size_t)v + (size_t)((dy + ny * dz) * nx)) * cx + c8;
-                    if (in) d[i + 1] = *(const uint4 *)p;
-                    if (i == 0 && in && xx > 0) d[0] = *(const uint4 *)(p - cx);
-                    if (i == 7 && in && xx < nx - 1) d[9] = *(const uint4 *)(p + cx);
-                    // a neighbour is also wanted where its own voxel lies past the split
-                    if (i < 7 && in && xx < nx - 1 && v + 1 >= vend) d[i + 2] = *(const uint4 *)(p + cx);
-                    edge |= (uint32_t)(xx == 0) << i | (uint32_t)(xx == nx - 1) << (8 + i);
-                    edge |= (uint32_t)in << (16 + i);
+                    const bool in = v0 + i < vend && real && (unsigned)(yy + dy) < (unsigned)ny &&
+                                    (unsigned)(zz + dz) < (unsigned)nz;
+                    edge |= (uint32_t)(xx == 0) << i | (uint32_t)(xx == nx - 1) << (8 + i) | (uint32_t)in << (16 + i);
                     if (++xx == nx) {
                         xx = 0;
                         if (++yy == ny) {
@@ -315,13 +338,13 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
         if (is_g) {
             uint4 v[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = d[i];
+            for (int i = 0; i < 8; ++i) v[i] = edge >> (16 + i) & 1u ? d[i] : uint4{0u, 0u, 0u, 0u};
             put(sg, v);
         } else if (is_x) {
             if constexpr (TX == 1) {
                 uint4 v[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = d[i];
+                for (int i = 0; i < 8; ++i) v[i] = edge >> (16 + i) & 1u ? d[i] : uint4{0u, 0u, 0u, 0u};
                 put(sx, v);
             } else {
 #pragma unroll
@@ -333,7 +356,7 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
                                          (t == 2 && (edge >> (8 + i) & 1u));
                         v[i] = off ? uint4{0u, 0u, 0u, 0u} : d[i + t];
                     }
-                    put(sx + t * cxp * row, v);
+                    put(sx + t * cxg * row, v);
                 }
             }
         }
@@ -353,17 +376,14 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
                     }
                 }
             }
-        // products 4 s + wave: tap t, output rows mt, input rows nt
+        const unsigned char *ga = sg + r * row + 16 * q, *xa = sx + r * row + 16 * q;
+#pragma unroll 4
         for (int kh = 0; kh < kt / 32; ++kh) {
 #pragma unroll
             for (int s = 0; s < NA; ++s) {
-                const int u = wv + 4 * s;
-                if (u < TX * tiles) {
-                    const int t = u / tiles, mn = u - t * tiles, mt = mn / nnt, nt = mn - mt * nnt;
-                    const bf16x8 a = __builtin_bit_cast(
-                        bf16x8, *(const uint4 *)(sg + (mt * 16 + r) * row + 64 * kh + 16 * q));
-                    const bf16x8 b = __builtin_bit_cast(
-                        bf16x8, *(const uint4 *)(sx + (t * cxp + nt * 16 + r) * row + 64 * kh + 16 * q));
+                if (wv + 4 * s < TX * tiles) {
+                    const bf16x8 a = __builtin_bit_cast(bf16x8, *(const uint4 *)(ga + arow[s] + 64 * kh));
+                    const bf16x8 b = __builtin_bit_cast(bf16x8, *(const uint4 *)(xa + brow[s] + 64 * kh));
                     acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[s], 0, 0, 0);
                 }
             }
@@ -377,10 +397,10 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
             const int t = u / tiles, mn = u - t * tiles, mt = mn / nnt, nt = mn - mt * nnt;
             float *out = part + ((size_t)split * taps + (TX == 3 ? 3 * yz + t : 0)) * cg * cxp;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) out[(size_t)(mt * 16 + 4 * q + j) * cxp + nt * 16 + r] = acc[s][j];
+            for (int j = 0; j < 4; ++j) out[(size_t)(mt * 16 + 4 * q + j) * cxp + xo + nt * 16 + r] = acc[s][j];
         }
     }
-    if (yz == 0) {  // uniform per workgroup
+    if (yz == 0 && xo == 0) {  // uniform per workgroup
         __shared__ float bred[4 * kMaxCg];
         if (bias) bred[tid] = bsum;
         __syncthreads();
@@ -771,19 +791,21 @@ int conv_grads(lbm_unet *N, const lbm_unet::Conv &c, const bf16_t *g, const bf16
     wsplit(V, c.taps, &nsplit, &chunk);
     if ((size_t)nsplit * c.taps * cg * cxp > N->wpart_n) return lbm::set_error(LBM_ERR_ARG, "weight partials overflow");
     if ((size_t)nsplit * cg > N->bpart_n) return lbm::set_error(LBM_ERR_ARG, "bias partials overflow");
-    const int tx = c.taps == 27 ? 3 : 1, tiles = tx * (cg / 16) * (cxp / 16);
+    // A workgroup's time is its chain of tiles, each a memory round trip, a transposition and its
+    // products, so: as many voxels per tile as give every thread a unit and fit 72 kB of rows (two
+    // workgroups per CU), and 48 input channels as three workgroups of 16, each with the longer tile.
+    const int tx = c.taps == 27 ? 3 : 1, cxg = cxp == 48 ? 16 : cxp, tiles = tx * (cg / 16) * (cxg / 16);
     if (tiles > (tx == 3 ? 48 : 16)) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d tiles", tiles);
-    // voxels per LDS tile: the most for which a thread has one unit and the rows fit 64 kB
-    int kt = 256;
-    auto rows = [&](int k) { return (cg + tx * cxp) * (k + 8) * 2; };
-    while (kt > kTileV && (kt / 8 * (cg + cxp) / 8 > 256 || rows(kt) > 65536 - 4 * kMaxCg * (int)sizeof(float))) kt /= 2;
-    if (kt / 8 * (cg + cxp) / 8 > 256) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d x %d channels", cg, cxp);
-    if (tx == 3)
-        k_conv_wgrad<3><<<dim3(nsplit, 9), 256, rows(kt), N->s>>>(g, cg, x, c.cis, d[0], d[1], d[2], chunk, kt, N->wpart,
-                                                                  N->bpart);
-    else
-        k_conv_wgrad<1><<<dim3(nsplit, 1), 256, rows(kt), N->s>>>(g, cg, x, c.cis, d[0], d[1], d[2], chunk, kt, N->wpart,
-                                                                  N->bpart);
+    int kt = 512;
+    auto rows = [&](int k) { return (cg + tx * cxg) * (k + 8) * 2; };
+    while (kt > kTileV && (kt / 8 * ((cg + cxg) / 8) > 256 || rows(kt) > 72 * 1024)) kt /= 2;
+    if (kt / 8 * ((cg + cxg) / 8) > 256) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d x %d channels", cg, cxp);
+    auto *kernel = tx == 3 ? &k_conv_wgrad<3> : &k_conv_wgrad<1>;
+    if (rows(kt) > 60 * 1024)
+        UCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 rows(kt)));
+    kernel<<<dim3(nsplit, c.taps / tx, cxp / cxg), 256, rows(kt), N->s>>>(g, cg, x, c.cis, d[0], d[1], d[2], chunk, kt,
+                                                                         cxg, N->wpart, N->bpart);
     UCHK(hipGetLastError());
     const int nw = c.co * c.taps * c.ci;  // the bias follows the weights in the parameter vector
     k_wgrad_reduce<<<blocks(nw + c.co, 64), 64, 0, N->s>>>(N->wpart, N->bpart, nsplit, c.taps, cg, cxp, c.co, c.ci,
