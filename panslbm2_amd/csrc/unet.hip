@@ -130,6 +130,11 @@ __global__ void __launch_bounds__(256) k_conv1(const bf16_t *__restrict__ x, int
     }
 }
 
+// d where bit is set, zero where not, without a branch
+__device__ __forceinline__ uint4 keep(const uint4 &d, uint32_t bit) {
+    const uint32_t m = 0u - (bit & 1u);
+    return uint4{d.x & m, d.y & m, d.z & m, d.w & m};
+}
 // 3x3x3 convolution.  A workgroup of WM x WN waves stages a brick of 18 x 6 x (WN + 2) voxels (its 16
 // x 4 x WN outputs and their halo, zero outside the grid) with all CIN channels in LDS once; wave
 // (m, n) computes 16 MT output channels of z layer n, 4 rows of 16 voxels.  Read from global memory
@@ -176,7 +181,7 @@ __global__ void __launch_bounds__(64 * WM * WN) k_conv3(const bf16_t *__restrict
 #pragma unroll
         for (int h = 0; h < BATCH; ++h) {
             const int u = tid + (it + h) * THREADS, vox = u / CU, c = u - vox * CU;
-            if (u < UNITS) *(uint4 *)(lds + vox * VS + 16 * c) = in[h] ? d[h] : uint4{0u, 0u, 0u, 0u};
+            if (u < UNITS) *(uint4 *)(lds + vox * VS + 16 * c) = keep(d[h], in[h]);
         }
     }
     f4 acc[MT][NT];
@@ -338,13 +343,13 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
         if (is_g) {
             uint4 v[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = edge >> (16 + i) & 1u ? d[i] : uint4{0u, 0u, 0u, 0u};
+            for (int i = 0; i < 8; ++i) v[i] = keep(d[i], edge >> (16 + i));
             put(sg, v);
         } else if (is_x) {
             if constexpr (TX == 1) {
                 uint4 v[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = edge >> (16 + i) & 1u ? d[i] : uint4{0u, 0u, 0u, 0u};
+                for (int i = 0; i < 8; ++i) v[i] = keep(d[i], edge >> (16 + i));
                 put(sx, v);
             } else {
 #pragma unroll
@@ -352,9 +357,10 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
                     uint4 v[8];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
-                        const bool off = !(edge >> (16 + i) & 1u) || (t == 0 && (edge >> i & 1u)) ||
-                                         (t == 2 && (edge >> (8 + i) & 1u));
-                        v[i] = off ? uint4{0u, 0u, 0u, 0u} : d[i + t];
+                        uint32_t on = edge >> (16 + i);
+                        if (t == 0) on &= ~(edge >> i);
+                        if (t == 2) on &= ~(edge >> (8 + i));
+                        v[i] = keep(d[i + t], on);
                     }
                     put(sx + t * cxg * row, v);
                 }
