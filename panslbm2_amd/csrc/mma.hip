@@ -125,11 +125,21 @@ __global__ void k_start(int n, Vec v) {
     }
 }
 
+// One design variable's part of the squared KKT residual (mma.h:551-602): (5.9a)^2 + (5.9e)^2 + (5.9f)^2
+__device__ __forceinline__ void kkt_terms(double &acc, double x, double gsi, double ita, double L, double U, double al,
+                                          double be, double pl, double ql, double eps) {
+    acc += sq(pl / sq(U - x) - ql / sq(x - L) - gsi + ita);
+    acc += sq(gsi * (x - al) - eps);
+    acc += sq(ita * (be - x) - eps);
+}
+
 // mma.h:325-396 (the n-long part): G, Dx, deltilx, and partials of
-// sum_j p/(U-x) + q/(x-L) (M), sum_j G_a G_b / Dx (M x M), sum_j G_a deltilx / Dx (M)
+// sum_j p/(U-x) + q/(x-L) (M), sum_j G_a G_b / Dx (M x M), sum_j G_a deltilx / Dx (M), and of the
+// squared KKT residual at the current point, which the line search starts from and which reads the
+// same vectors (a pass and a wait of its own before)
 template <int M>
 __global__ void __launch_bounds__(kBlock) k_newton1(int n, Vec v, Scal s, double eps, double *part) {
-    constexpr int K = M + M * M + M;
+    constexpr int K = M + M * M + M + 1;
     double acc[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = 0.0;
@@ -160,6 +170,7 @@ __global__ void __launch_bounds__(kBlock) k_newton1(int n, Vec v, Scal s, double
             for (int b = 0; b < M; ++b) acc[M + a * M + b] += G[a] * G[b] / Dx;
             acc[M + M * M + a] += G[a] * dtx / Dx;
         }
+        kkt_terms(acc[K - 1], x, v.gsi[j], v.ita[j], L, U, al, be, pl, ql, eps);
     }
     block_reduce<K, 0>(acc, part);
 }
@@ -186,25 +197,18 @@ __global__ void __launch_bounds__(kBlock) k_newton2(int n, Vec v, Scal s, double
     block_reduce<1, 1>(tmax, part);
 }
 
-// mma.h:551-602 (the n-long part) at the point x + tau dx (tau = 0: the current point; trial != 0
-// also stores the point): partials of sum_j [(5.9a)^2 + (5.9e)^2 + (5.9f)^2] and of
-// g_i = sum_j p/(U-x) + q/(x-L)
+// mma.h:551-602 (the n-long part) at the trial point x + tau dx, which it stores: partials of
+// sum_j [(5.9a)^2 + (5.9e)^2 + (5.9f)^2] and of g_i = sum_j p/(U-x) + q/(x-L)
 template <int M>
-__global__ void __launch_bounds__(kBlock) k_kkt(int n, Vec v, Scal s, double eps, double tau, int trial,
-                                                double *part) {
+__global__ void __launch_bounds__(kBlock) k_kkt(int n, Vec v, Scal s, double eps, double tau, double *part) {
     double acc[1 + M];
 #pragma unroll
     for (int k = 0; k <= M; ++k) acc[k] = 0.0;
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
-        double x = v.x[j], gsi = v.gsi[j], ita = v.ita[j];
-        if (trial) {
-            x = x + tau * v.dx[j];
-            gsi = gsi + tau * v.dgsi[j];
-            ita = ita + tau * v.dita[j];
-            v.xt[j] = x;
-            v.gsit[j] = gsi;
-            v.itat[j] = ita;
-        }
+        const double x = v.x[j] + tau * v.dx[j], gsi = v.gsi[j] + tau * v.dgsi[j], ita = v.ita[j] + tau * v.dita[j];
+        v.xt[j] = x;
+        v.gsit[j] = gsi;
+        v.itat[j] = ita;
         const double L = v.L[j], U = v.U[j];
         double pl = v.p0[j], ql = v.q0[j];
 #pragma unroll
@@ -214,9 +218,7 @@ __global__ void __launch_bounds__(kBlock) k_kkt(int n, Vec v, Scal s, double eps
             ql += s.lambda[i] * qij;
             acc[1 + i] += pij / (U - x) + qij / (x - L);
         }
-        acc[0] += sq(pl / sq(U - x) - ql / sq(x - L) - gsi + ita);
-        acc[0] += sq(gsi * (x - v.alpha[j]) - eps);
-        acc[0] += sq(ita * (v.beta[j] - x) - eps);
+        kkt_terms(acc[0], x, gsi, ita, L, U, v.alpha[j], v.beta[j], pl, ql, eps);
     }
     block_reduce<1 + M, 0>(acc, part);
 }
@@ -262,7 +264,10 @@ struct lbm_mma {
     double previous = 0.0;
     Vec v{};
     std::vector<void *> allocs;
-    double *part = nullptr, *hpart = nullptr;  // device and pinned host partials
+    // The kernels' partial sums, in pinned host memory that the kernels write to: a few kB per kernel,
+    // read after a wait for the stream (a copy of its own between the two cost about 8 us of the
+    // 70 waits of an update).
+    double *part = nullptr;
     int last_iters = 0;
 };
 
@@ -280,42 +285,36 @@ void destroy(lbm_mma *O) {
     (void)hipSetDevice(lbm::context_device(O->ctx));
     (void)hipStreamSynchronize(O->s);
     for (void *q : O->allocs) (void)hipFree(q);
-    if (O->hpart) (void)hipHostFree(O->hpart);
+    if (O->part) (void)hipHostFree(O->part);
     delete O;
 }
 
 // sums (or maxima) of K partials per block, added in block order on the host
 int fetch(lbm_mma *O, int K, int op, double *out) {
-    MCHK(hipMemcpyAsync(O->hpart, O->part, sizeof(double) * K * O->nb, hipMemcpyDeviceToHost, O->s));
     MCHK(hipStreamSynchronize(O->s));
     for (int k = 0; k < K; ++k) {
-        double r = O->hpart[k];
-        for (int b = 1; b < O->nb; ++b) r = op == 0 ? r + O->hpart[(size_t)b * K + k] : std::max(r, O->hpart[(size_t)b * K + k]);
+        double r = O->part[k];
+        for (int b = 1; b < O->nb; ++b) r = op == 0 ? r + O->part[(size_t)b * K + k] : std::max(r, O->part[(size_t)b * K + k]);
         out[k] = r;
     }
     return LBM_OK;
 }
 
+// The KKT norm (mma.h:551-602) from its n-long sums: nn (the squares) and g_i
 template <int M>
-int kkt(lbm_mma *O, const Scal &sc, double eps, double tau, int trial, const double *y, double z, const double *mu,
-        double zeta, const double *sv, const double *b, double *norm) {
-    k_kkt<M><<<O->nb, kBlock, 0, O->s>>>(O->n, O->v, sc, eps, tau, trial, O->part);
-    MCHK(hipGetLastError());
-    double r[1 + M];
-    int rc = fetch(O, 1 + M, 0, r);
-    if (rc != LBM_OK) return rc;
-    double nn = r[0], la = 0.0;
+double kkt_norm(const lbm_mma *O, const Scal &sc, double eps, double nn, const double *g, const double *y, double z,
+                const double *mu, double zeta, const double *sv, const double *b) {
+    double la = 0.0;
     for (int i = 0; i < M; ++i) {
         nn += sq(O->c[i] + O->d[i] * y[i] - sc.lambda[i] - mu[i]);
-        nn += sq(r[1 + i] - O->a[i] * z - y[i] + sv[i] - b[i]);
+        nn += sq(g[i] - O->a[i] * z - y[i] + sv[i] - b[i]);
         nn += sq(mu[i] * y[i] - eps);
         nn += sq(sc.lambda[i] * sv[i] - eps);
         la += sc.lambda[i] * O->a[i];
     }
     nn += sq(O->a0 - zeta - la);
     nn += sq(zeta * z - eps);
-    *norm = std::sqrt(nn);
-    return LBM_OK;
+    return std::sqrt(nn);
 }
 
 template <int M>
@@ -345,7 +344,7 @@ int update(lbm_mma *O, double *xk, double f, const double *dfdx, const double *g
     for (; eps > 1.0e-7 && it < kMaxIter; ++it) {
         k_newton1<M><<<O->nb, kBlock, 0, st>>>(n, v, sc, eps, O->part);
         MCHK(hipGetLastError());
-        constexpr int K = M + M * M + M;
+        constexpr int K = M + M * M + M + 1;
         double r[K];
         if ((rc = fetch(O, K, 0, r)) != LBM_OK) return rc;
         double Dy[M], Dly[M], dly[M], dtily[M], la = 0.0;
@@ -386,8 +385,7 @@ int update(lbm_mma *O, double *xk, double f, const double *dfdx, const double *g
         }
         const double dzeta = -zeta * dz / z - zeta + eps / z;
         double tau = 1.0 / std::max(std::max(std::max(1.0, txmax), tymax), std::max(-1.01 * dz / z, -1.01 * dzeta / zeta));
-        double w0;
-        if ((rc = kkt<M>(O, sc, eps, 0.0, 0, y, z, mu, zeta, sv, b, &w0)) != LBM_OK) return rc;
+        const double w0 = kkt_norm<M>(O, sc, eps, r[K - 1], r, y, z, mu, zeta, sv, b);
         double yt[M], mut[M], svt[M], w1 = 0.0, zt = z, zetat = zeta;
         Scal st_{};
         for (int ll = 0; ll < 50; ++ll) {
@@ -399,7 +397,11 @@ int update(lbm_mma *O, double *xk, double f, const double *dfdx, const double *g
             }
             zt = z + tau * dz;
             zetat = zeta + tau * dzeta;
-            if ((rc = kkt<M>(O, st_, eps, tau, 1, yt, zt, mut, zetat, svt, b, &w1)) != LBM_OK) return rc;
+            k_kkt<M><<<O->nb, kBlock, 0, st>>>(n, v, st_, eps, tau, O->part);
+            MCHK(hipGetLastError());
+            double rt[1 + M];
+            if ((rc = fetch(O, 1 + M, 0, rt)) != LBM_OK) return rc;
+            w1 = kkt_norm<M>(O, st_, eps, rt[0], rt + 1, yt, zt, mut, zetat, svt, b);
             if (w1 < w0) break;
             tau *= 0.5;
         }
@@ -468,14 +470,12 @@ int lbm_mma_create(lbm_context *ctx, int n, int m, double a0, const double *a, c
         }
         O->allocs.push_back(*p);
     }
-    const size_t pn = (size_t)O->nb * (kMaxM + kMaxM * kMaxM + kMaxM);
-    if (hipMalloc((void **)&O->part, sizeof(double) * pn) != hipSuccess ||
-        hipHostMalloc((void **)&O->hpart, sizeof(double) * pn, hipHostMallocDefault) != hipSuccess) {
-        if (O->part) O->allocs.push_back(O->part);
+    const size_t pn = (size_t)O->nb * (kMaxM + kMaxM * kMaxM + kMaxM + 1);
+    if (hipHostMalloc((void **)&O->part, sizeof(double) * pn, hipHostMallocDefault) != hipSuccess) {
+        O->part = nullptr;
         destroy(O);
         return lbm::set_error(LBM_ERR_HIP, "partials allocation failed");
     }
-    O->allocs.push_back(O->part);
     hipError_t e = hipMemcpyAsync(O->v.xmin, xmin, sizeof(double) * n, hipMemcpyDefault, O->s);
     if (e == hipSuccess) e = hipMemcpyAsync(O->v.xmax, xmax, sizeof(double) * n, hipMemcpyDefault, O->s);
     if (e == hipSuccess) e = hipMemsetAsync(O->v.xkm1, 0, sizeof(double) * n, O->s);
