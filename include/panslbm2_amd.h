@@ -90,8 +90,8 @@ int lbm_context_create(int device, lbm_context **out);
 int lbm_context_destroy(lbm_context *ctx);
 int lbm_context_synchronize(lbm_context *ctx);
 /* No reference counterpart.  3D programs with SmoothCorner: finish the smoothed edges and corners
- * on a second stream concurrently with the fused pass, each lane rebuilding its face neighbours'
- * post-boundary states (on = 1, the default), or after the pass from the states it saves (0).
+ * inside the fused pass, whose first workgroups rebuild their face neighbours' post-boundary states
+ * (on = 1, the default), or after the pass from the states it saves (0).
  * Both give the same values; the concurrent form is used only when no field a boundary operator
  * reads is one the collide writes. */
 int lbm_context_set_concurrent_smoothing(lbm_context *ctx, int on);
@@ -312,6 +312,13 @@ int lbm_heaviside_filter_region(lbm_context *ctx, int lx, int ly, int lz, double
 int lbm_heaviside_sensitivity_region(lbm_context *ctx, int lx, int ly, int lz, double R, double beta, int mx, int my,
                                      int mz, const double *v, const double *dfdrho, double *dfds);
 int lbm_density_filter(lbm_context *ctx, int lx, int ly, int lz, double R, const double *v, double *out);
+/* The coefficient fields of a 3D duct from its filtered design (heatsink.cpp:104-117 interpolation).
+ * gamma (in: filtered design; out: with 1 outside the box [0,mx) x [0,my) x [0,mz) and 0 below plate),
+ * dgamma = gamma - prev (0 without have_prev), prev = gamma, alpha, dads, diff and dkds per node. */
+int lbm_duct_coefficients(lbm_context *ctx, int lx, int ly, int lz, int mx, int my, int mz, int plate,
+                          double alpha_max, double qf, double qg, double dfl, double dso, double *gamma,
+                          double *prev, int have_prev, double *dgamma, double *alpha, double *dads, double *diff,
+                          double *dkds);
 
 /* ---- recording and fused steps ---- */
 int lbm_record_begin(lbm_context *ctx);

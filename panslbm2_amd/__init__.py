@@ -152,6 +152,7 @@ def load():
         "lbm_normalize": [VP, VP, I],
         "lbm_gather_sum": [VP, VP, VP, I, ctypes.POINTER(D)],
         "lbm_density_filter": [VP, I, I, I, D, VP, VP],
+        "lbm_duct_coefficients": [VP] + [I] * 7 + [D] * 5 + [VP, VP, I] + [VP] * 5,
         "lbm_record_begin": [VP],
         "lbm_record_end": [VP, ctypes.POINTER(VP)],
         "lbm_record_end_deferred": [VP, ctypes.POINTER(VP)],

@@ -1624,9 +1624,10 @@ int lbm_sensitivity_temperature_at_heat_source_c(lbm_lattice *q, double *dfds, c
         if (cs != hipStreamCaptureStatusNone)
             return fail(LBM_ERR_STATE, "heat-source faces changed during graph capture: call once outside the capture");
     }
-    int rc = lbm_sensitivity_brinkman_diffusivity(q, dfds, ux, uy, uz, imx, imy, imz, dads, tem, item, iqx, iqy, iqz, g,
-                                                  ig, diff, dkds);
-    if (rc) return rc;
+    if (!fields_ok({dfds, ux, uy, imx, imy, dads, tem, item, iqx, iqy, g, ig, diff, dkds}) ||
+        (q->nd == 3 && (!imz || !iqz)))
+        return fail(LBM_ERR_ARG, "bad arguments");
+    int rc;
     if (!same) {
         lbm_program *P = new lbm_program;
         P->ctx = q->ctx;
@@ -1641,9 +1642,11 @@ int lbm_sensitivity_temperature_at_heat_source_c(lbm_lattice *q, double *dfds, c
         q->hs_mask.assign(mask, mask + nf);
         q->hs_qn.assign(qn, qn + nf);
     }
-    if (q->hs_prog->ops.empty()) return LBM_OK;
-    ProgView v = prog_view(q->hs_prog);
-    HIPCHK(lbm::launch_sens_hs_boundary(q->kind, dfds, q->N, v, ux, uy, uz, ig, diff, dkds, compat, q->ctx->stream));
+    if (q->hs_prog->ops.empty())
+        return lbm_sensitivity_brinkman_diffusivity(q, dfds, ux, uy, uz, imx, imy, imz, dads, tem, item, iqx, iqy, iqz,
+                                                    g, ig, diff, dkds);
+    const double *a[16] = {ux, uy, uz, imx, imy, imz, dads, tem, item, iqx, iqy, iqz, g, ig, diff, dkds};
+    HIPCHK(lbm::launch_sens_bd_hs(q->kind, dfds, q->grid(), a, prog_view(q->hs_prog), compat, q->ctx->stream));
     return LBM_OK;
 }
 int lbm_sensitivity_temperature_at_heat_source(lbm_lattice *q, double *dfds, const double *ux, const double *uy,
@@ -1753,6 +1756,20 @@ int lbm_density_filter(lbm_context *C, int lx, int ly, int lz, double R, const d
     HIPCHK(lbm::launch_density_filter(v, out, lx, ly, lz, nR, nd, (const double *)C->scratch.p, C->stream));
     HIPCHK(hipStreamSynchronize(C->stream));
     return LBM_OK;
+}
+
+int lbm_duct_coefficients(lbm_context *C, int lx, int ly, int lz, int mx, int my, int mz, int plate, double alpha_max,
+                          double qf, double qg, double dfl, double dso, double *gamma, double *prev, int have_prev,
+                          double *dgamma, double *alpha, double *dads, double *diff, double *dkds) {
+    if (!C || !fields_ok({gamma, prev, dgamma, alpha, dads, diff, dkds}) || lx < 1 || ly < 2 || lz < 1)
+        return fail(LBM_ERR_ARG, "bad arguments");
+    const long N = (long)lx * ly * lz;
+    if (N > (1L << 31) - 1) return fail(LBM_ERR_UNSUPPORTED, "grid too large for 32-bit indexing");
+    const lbm::DuctCoefficients c{alpha_max / (ly - 1.0) * qf, -alpha_max / (ly - 1.0) * qf * (1.0 + qf), dso, dfl - dso,
+                                  (dfl - dso) * qg * (1.0 + qg), qf, qg};
+    return hip_result(lbm::launch_duct_coefficients(lbm::make_grid(lx, ly, lz, (int)N), make_int3(mx, my, mz), plate, c,
+                                                    gamma, prev, have_prev, dgamma, alpha, dads, diff, dkds, C->stream),
+                      "duct coefficients");
 }
 
 // ---- recording ------------------------------------------------------------------------------

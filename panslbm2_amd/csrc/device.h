@@ -112,9 +112,16 @@ hipError_t launch_sens_brinkman(int nd, double *dfds, int N, const double *const
 hipError_t launch_sens_he(int nd, double *dfds, int N, const double *const *p, hipStream_t s);
 hipError_t launch_sens_hsrc(int nd, double *dfds, int N, const double *const *p, hipStream_t s);
 hipError_t launch_sens_bd(int kind, double *dfds, int N, const double *const *p, hipStream_t s);
-hipError_t launch_sens_hs_boundary(int kind, double *dfds, int N, const ProgView &pv, const double *ux,
-                                   const double *uy, const double *uz, const double *ig, const double *diff,
-                                   const double *dkds, int compat, hipStream_t s);
+hipError_t launch_sens_bd_hs(int kind, double *dfds, const Grid &g, const double *const *p, const ProgView &pv,
+                             int compat, hipStream_t s);
+// scalars of lbm_duct_coefficients: alpha = alpha (1 - s) / (s + qf), dads = dads / (s + qf)^2,
+// diff = dso + ddiff s (1 + qg) / (s + qg), dkds = dkds / (s + qg)^2
+struct DuctCoefficients {
+    double alpha, dads, dso, ddiff, dkds, qf, qg;
+};
+hipError_t launch_duct_coefficients(const Grid &g, int3 box, int plate, const DuctCoefficients &c, double *gamma,
+                                    double *prev, int have_prev, double *dgamma, double *alpha, double *dads,
+                                    double *diff, double *dkds, hipStream_t s);
 hipError_t launch_residual(int ncomp, const double *const *a, const double *const *b, int n, double *part,
                            double *out, hipStream_t s);
 // Residual sums of many arrays sets in one launch pair (lbm_residual_batch)

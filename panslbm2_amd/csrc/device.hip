@@ -139,15 +139,14 @@ __global__ void __launch_bounds__(kBlock) k_sens_hsrc(double *dfds, int N, const
     dfds[n] += -dhds[n] * (item[n] + 3.0 * omegag * uq);
 }
 
+// dfds at node n with the Brinkman and diffusivity terms (adjointadvection.h:1461-1493)
 template <class L>
-__global__ void __launch_bounds__(kBlock) k_sens_bd(double *dfds, int N, const double *ux, const double *uy,
-                                                    const double *uz, const double *imx, const double *imy,
-                                                    const double *imz, const double *dads, const double *tem,
-                                                    const double *item, const double *iqx, const double *iqy,
-                                                    const double *iqz, const double *g, const double *ig,
-                                                    const double *diff, const double *dkds) {
-    int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
+__device__ __forceinline__ double sens_bd_node(const double *dfds, int N, int n, const double *ux, const double *uy,
+                                               const double *uz, const double *imx, const double *imy,
+                                               const double *imz, const double *dads, const double *tem,
+                                               const double *item, const double *iqx, const double *iqy,
+                                               const double *iqz, const double *g, const double *ig,
+                                               const double *diff, const double *dkds) {
     double d = dfds[n];
     if constexpr (L::nd == 2) d += 3.0 * dads[n] * (ux[n] * imx[n] + uy[n] * imy[n]);
     else d += 3.0 * dads[n] * (ux[n] * imx[n] + uy[n] * imy[n] + uz[n] * imz[n]);
@@ -161,7 +160,19 @@ __global__ void __launch_bounds__(kBlock) k_sens_bd(double *dfds, int N, const d
     else uq = ux[n] * iqx[n] + uy[n] * iqy[n] + uz[n] * iqz[n];
     double s = 3.0 * diff[n] + 0.5;
     d += -3.0 / (s * s) * dkds[n] * (sumg - tem[n] * (item[n] + 3.0 * uq));
-    dfds[n] = d;
+    return d;
+}
+
+template <class L>
+__global__ void __launch_bounds__(kBlock) k_sens_bd(double *dfds, int N, const double *ux, const double *uy,
+                                                    const double *uz, const double *imx, const double *imy,
+                                                    const double *imz, const double *dads, const double *tem,
+                                                    const double *item, const double *iqx, const double *iqy,
+                                                    const double *iqz, const double *g, const double *ig,
+                                                    const double *diff, const double *dkds) {
+    int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= N) return;
+    dfds[n] = sens_bd_node<L>(dfds, N, n, ux, uy, uz, imx, imy, imz, dads, tem, item, iqx, iqy, iqz, g, ig, diff, dkds);
 }
 
 // Heat-source boundary term of AAD::SensitivityTemperatureAtHeatSource, one thread per boundary
@@ -208,17 +219,15 @@ __device__ __forceinline__ double hs_face_term(int face, const double *igl, doub
     return qn * dk * num / (S * (dd < 0 ? 1.0 - 3.0 * u[a] : 1.0 + 3.0 * u[a]) * D2);
 }
 
+// d plus the terms of entry e of pv (node n)
 template <class L>
-__global__ void __launch_bounds__(kBlock) k_sens_hs_boundary(double *dfds, int N, ProgView pv, const double *ux,
-                                                             const double *uy, const double *uz, const double *ig,
-                                                             const double *diff, const double *dkds, int compat) {
-    int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= pv.nentry) return;
-    int n = pv.entry_node[e];
+__device__ __forceinline__ double sens_hs_terms(double d, int N, int n, int e, const ProgView &pv, const double *ux,
+                                                const double *uy, const double *uz, const double *ig,
+                                                const double *diff, const double *dkds, int compat) {
     int2 r = pv.entry_ops[e];
     double igl[L::nc];
     sfor<0, L::nc>([&](auto c) { igl[decltype(c)::value] = ig[(size_t)decltype(c)::value * N + n]; });
-    double vx = ux[n], vy = uy[n], D2 = diff[n] * diff[n], dk = dkds[n], acc_ = dfds[n];
+    double vx = ux[n], vy = uy[n], D2 = diff[n] * diff[n], dk = dkds[n], acc_ = d;
     double u[3] = {vx, vy, L::nd == 3 ? uz[n] : 0.0};
     for (int t = r.x; t < r.x + r.y; ++t) {
         Op op = pv.ops[t];
@@ -235,7 +244,29 @@ __global__ void __launch_bounds__(kBlock) k_sens_hs_boundary(double *dfds, int N
         }
         acc_ += term;
     }
-    dfds[n] = acc_;
+    return acc_;
+}
+
+// Both in one pass: a boundary node finds its entry by its slot.  A transient adjoint calls this every
+// step on a grid of some 20,000 nodes, where a launch of its own for a few edge nodes cost 3 to 4 us
+// of a 20 us step.
+template <class L>
+__global__ void __launch_bounds__(kBlock) k_sens_bd_hs(double *dfds, Grid gr, const double *ux, const double *uy,
+                                                       const double *uz, const double *imx, const double *imy,
+                                                       const double *imz, const double *dads, const double *tem,
+                                                       const double *item, const double *iqx, const double *iqy,
+                                                       const double *iqz, const double *g, const double *ig,
+                                                       const double *diff, const double *dkds, ProgView pv, int compat) {
+    int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= gr.N) return;
+    int i, j, k;
+    coords(n, gr, i, j, k);
+    const int slot = boundary_slot(i, j, k, gr.nx, gr.ny, gr.nz, L::nd);
+    const int e = slot >= 0 && slot < pv.nslot ? pv.slot_entry[slot] : -1;
+    double d =
+        sens_bd_node<L>(dfds, gr.N, n, ux, uy, uz, imx, imy, imz, dads, tem, item, iqx, iqy, iqz, g, ig, diff, dkds);
+    if (e >= 0) d = sens_hs_terms<L>(d, gr.N, n, e, pv, ux, uy, uz, ig, diff, dkds, compat);
+    dfds[n] = d;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -370,13 +401,44 @@ __global__ void __launch_bounds__(kBlock) k_divide(double *v, int n, const doubl
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) v[t] /= by[0];
 }
-// sequential sum over an index list, in list order (the reference's serial loop)
-__global__ void k_gather_sum(const double *v, const int *idx, int count, double *out) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        double s = 0.0;
-        for (int t = 0; t < count; ++t) s += v[idx[t]];
-        out[0] = s;
+// Sum over an index list, in list order (the reference's serial loop): the adds are one serial chain,
+// so one lane makes them, from LDS, while the workgroup fetches the next kGather values.  Bound by
+// the chain of FP64 additions (16,384 values: 1,570 us when that lane also fetched its own values).
+constexpr int kGather = 1024;
+__global__ void __launch_bounds__(kBlock) k_gather_sum(const double *__restrict__ v, const int *__restrict__ idx,
+                                                       int count, double *out) {
+    __shared__ __align__(16) double buf[kGather];
+    constexpr int PER = kGather / kBlock;
+    double next[PER];
+    auto fetch = [&](int base) {
+        int at[PER];
+#pragma unroll
+        for (int h = 0; h < PER; ++h) at[h] = idx[min(base + h * kBlock + (int)threadIdx.x, count - 1)];
+#pragma unroll
+        for (int h = 0; h < PER; ++h) next[h] = v[at[h]];
+    };
+    double s = 0.0;
+    if (count > 0) fetch(0);
+    for (int base = 0; base < count; base += kGather) {
+#pragma unroll
+        for (int h = 0; h < PER; ++h) buf[h * kBlock + threadIdx.x] = next[h];
+        __syncthreads();
+        if (base + kGather < count) fetch(base + kGather);
+        if (threadIdx.x == 0) {
+            const int m = min(kGather, count - base);
+            int t = 0;
+            for (; t + 16 <= m; t += 16) {
+                double x[16];
+#pragma unroll
+                for (int h = 0; h < 16; ++h) x[h] = buf[t + h];
+#pragma unroll
+                for (int h = 0; h < 16; ++h) s += x[h];
+            }
+            for (; t < m; ++t) s += buf[t];
+        }
+        __syncthreads();
     }
+    if (threadIdx.x == 0) out[0] = s;
 }
 __global__ void __launch_bounds__(kBlock) k_fill(double *p, size_t n, double v) {
     size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -455,6 +517,28 @@ __global__ void __launch_bounds__(kBlock) k_heaviside_sens2(const double *tmp, d
     if (n >= lx * ly * lz) return;
     double ws, s = hat_mean(tmp, lx, ly, lz, nR, w, box, n, &ws);
     out[n] = s / ws;
+}
+
+// Design gamma and the coefficient fields of a 3D duct from the filtered design (lbm_duct_coefficients)
+__global__ void __launch_bounds__(kBlock) k_duct_coefficients(Grid g, int3 box, int plate, DuctCoefficients c,
+                                                              double *gamma, double *prev, int have_prev,
+                                                              double *dgamma, double *alpha, double *dads,
+                                                              double *diff, double *dkds) {
+    int n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= g.N) return;
+    int i, j, k;
+    coords(n, g, i, j, k);
+    double s = gamma[n];
+    if (!(i < box.x && j < box.y && k < box.z)) s = 1.0;
+    if (k < plate) s = 0.0;
+    gamma[n] = s;
+    dgamma[n] = have_prev ? s - prev[n] : 0.0;
+    prev[n] = s;
+    const double sf = s + c.qf, sg = s + c.qg;
+    alpha[n] = c.alpha * (1.0 - s) / sf;
+    dads[n] = c.dads / (sf * sf);
+    diff[n] = c.dso + c.ddiff * s * (1.0 + c.qg) / sg;
+    dkds[n] = c.dkds / (sg * sg);
 }
 
 // ==========================================================================================
@@ -604,13 +688,12 @@ hipError_t launch_sens_bd(int kind, double *dfds, int N, const double *const *p,
     }
     return hipErrorInvalidValue;
 }
-hipError_t launch_sens_hs_boundary(int kind, double *dfds, int N, const ProgView &pv, const double *ux,
-                                   const double *uy, const double *uz, const double *ig, const double *diff,
-                                   const double *dkds, int compat, hipStream_t s) {
-    if (pv.nentry <= 0) return hipSuccess;
+hipError_t launch_sens_bd_hs(int kind, double *dfds, const Grid &g, const double *const *p, const ProgView &pv,
+                             int compat, hipStream_t s) {
     auto go = [&](auto l) {
         using L = decltype(l);
-        LBM_LAUNCH((k_sens_hs_boundary<L>), nblocks(pv.nentry), s, dfds, N, pv, ux, uy, uz, ig, diff, dkds, compat);
+        LBM_LAUNCH((k_sens_bd_hs<L>), nblocks(g.N), s, dfds, g, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8],
+                   p[9], p[10], p[11], p[12], p[13], p[14], p[15], pv, compat);
         return hipGetLastError();
     };
     switch (kind) {
@@ -640,7 +723,7 @@ hipError_t launch_normalize(double *v, int n, double *part, double *out, hipStre
     return hipGetLastError();
 }
 hipError_t launch_gather_sum(const double *v, const int *idx, int count, double *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_gather_sum, dim3(1), dim3(64), 0, s, v, idx, count, out);
+    LBM_LAUNCH(k_gather_sum, 1, s, v, idx, count, out);
     return hipGetLastError();
 }
 hipError_t launch_fill(double *p, size_t n, double v, hipStream_t s) {
@@ -661,6 +744,13 @@ hipError_t launch_heaviside_sens(const double *v, const double *dfdrho, double *
                                  int lz, int nR, const double *w, int3 box, double beta, double tb, hipStream_t s) {
     LBM_LAUNCH(k_heaviside_sens1, nblocks((long)lx * ly * lz), s, v, dfdrho, tmp, lx, ly, lz, nR, w, box, beta, tb);
     LBM_LAUNCH(k_heaviside_sens2, nblocks((long)lx * ly * lz), s, tmp, out, lx, ly, lz, nR, w, box);
+    return hipGetLastError();
+}
+hipError_t launch_duct_coefficients(const Grid &g, int3 box, int plate, const DuctCoefficients &c, double *gamma,
+                                    double *prev, int have_prev, double *dgamma, double *alpha, double *dads,
+                                    double *diff, double *dkds, hipStream_t s) {
+    LBM_LAUNCH(k_duct_coefficients, nblocks(g.N), s, g, box, plate, c, gamma, prev, have_prev, dgamma, alpha, dads, diff,
+               dkds);
     return hipGetLastError();
 }
 int reduction_blocks() { return kRedBlocks; }

@@ -15,9 +15,7 @@ set of a duct heat sink:
 By default no SmoothCorner: the corner and edge nodes lie on bounce-back walls, and each time step
 is one fused kernel pass.  With smooth_corners=True both lattices are smoothed after the boundary
 calls of every forward and adjoint step, as the reference's 3D driver does (heatsink3D.cpp:175-176,
-215-216); the fused pass then skips the edge and corner nodes, which a kernel on the context's
-second stream smooths, collides and stores concurrently with the pass (107.8 vs 91.7 us per step at
-128x128x64).
+215-216), by the fused pass's first workgroups (79 us per smoothed step at 128x128x64, 78 without).
 The Navier-Stokes lattice is D3Q15 (the reference's) or D3Q27 (ns_kind=D3Q27, no reference
 counterpart; its velocity and pressure boundaries are non-equilibrium bounce-back).
 """
@@ -79,7 +77,7 @@ class Heatsink3D(Heatsink2D):
         self.dso = 10.0 * self.dfl
         rng = np.random.default_rng(seed)
         self.d = {name: c.array((N,), fill=0.0)
-                  for name in ("alpha", "dads", "diff", "dkds", "raw", "design", "dgamma")}
+                  for name in ("alpha", "dads", "diff", "dkds", "raw", "design", "prev", "dgamma")}
         self.d["heat"] = c.array((N,), data=np.where(k < plate, heat, 0.0))
         self.set_design(rng.uniform(0.0, 1.0, N))
         for name in ("rho", "tem", "ip", "imx", "imy", "imz", "item", "dfds"):
@@ -131,18 +129,13 @@ class Heatsink3D(Heatsink2D):
         else:
             check(self.L.lbm_density_filter(c.h, lx, ly, lz, D(self.filter_radius), d["raw"].ptr,
                                             d["design"].ptr))
-        s = d["design"].download()
-        s[~self.in_box] = 1.0  # fluid outside the design box
-        s[self.k < self.plate] = 0.0  # the base plate is solid
-        d["design"].upload(s)
-        prev = getattr(self, "gamma", None)
-        d["dgamma"].upload(s - prev if prev is not None else np.zeros_like(s))
-        self.gamma = s
-        am, qf, qg, dfl, dso = self.alpha_max, self.qf, self.qg, self.dfl, self.dso
-        d["alpha"].upload(am / (ly - 1.0) * qf * (1.0 - s) / (s + qf))
-        d["dads"].upload(-am / (ly - 1.0) * qf * (1.0 + qf) / (s + qf) ** 2)
-        d["diff"].upload(dso + (dfl - dso) * s * (1.0 + qg) / (s + qg))
-        d["dkds"].upload((dfl - dso) * qg * (1.0 + qg) / (s + qg) ** 2)
+        # fluid outside the design box, solid base plate, and the coefficients, in one pass on the device
+        # (in numpy, with the uploads of its five arrays: 4 ms of an 8.6 ms design update at 96x96x48)
+        check(self.L.lbm_duct_coefficients(
+            c.h, lx, ly, lz, *self.design_box, self.plate, D(self.alpha_max), D(self.qf), D(self.qg), D(self.dfl),
+            D(self.dso), d["design"].ptr, d["prev"].ptr, int(hasattr(self, "gamma")), d["dgamma"].ptr, d["alpha"].ptr,
+            d["dads"].ptr, d["diff"].ptr, d["dkds"].ptr))
+        self.gamma = d["design"].download()
 
     def design_update(self, vf=0.4, move=0.05, optimizer="mma"):
         """One design step over the design variables (the design box's nodes above the plate).
