@@ -568,6 +568,15 @@ struct AADBody<LA, LB, float> {
     }
 };
 
+// Where a body's coefficient fields are loaded after the boundary operators instead of before the
+// pull.  The FP32 2D adjoint's seven fields held across the operators cost 132-148 VGPRs, three
+// wavefronts per SIMD; loaded late they leave 116-128 and four, without scratch.  The other
+// bodies fit without it, or not with it (FP32 3D: 64-308 bytes of scratch under the four-wavefront bound).
+template <class Body>
+constexpr bool kLateCoef = false;
+template <class LA, class LB>
+constexpr bool kLateCoef<AADBody<LA, LB, float>> = LA::nd == 2;
+
 // ------------------------------------------------------------------------------------------
 // Collide kernels.  In place: the reference's own collide (no pending stream / boundaries).
 // Fused: pull + boundary program + collide, reading `s*` and writing `d*`.  Smoothed nodes: by the
@@ -662,7 +671,8 @@ __device__ __forceinline__ void fused_block(const S *__restrict__ sa, const S *_
     }
     R fa[LA::nc], fb[NB];
     const Sh4 oa = own_shift<S>(body.ea), ob = own_shift<S>(body.eb);
-    const auto coef = body.load(n);
+    typename Body::Coef coef;
+    if constexpr (!kLateCoef<Body>) coef = body.load(n);
     node_state<LA, LB>(sa, sb, g, pv, n, fa, fb, body.ea, body.eb, oa, ob, ops);
     if (sm) {
         if ((pv.smooth_bits >> (0 ^ pv.latswap)) & 1) smooth_lanes_mean<LA>(fa, body.ea, corner3);
@@ -675,6 +685,10 @@ __device__ __forceinline__ void fused_block(const S *__restrict__ sa, const S *_
         put_state<LA>(sp, fa, body.ea, oa);
         if constexpr (LB::nc > 0) put_state<LB>(sp + LA::nc, fb, body.eb, ob);
     }
+    if constexpr (kLateCoef<Body>) {
+        asm volatile("" : "+v"(n));  // or the compiler hoists the loads over the operators
+        coef = body.load(n);
+    }
     body(fa, fb, coef, n, nb > 0, oa, ob);
     if (LA::nd == 3 && g.nt) {
         store_raw<LA, true>(da, g.N, n, fa);
@@ -685,7 +699,7 @@ __device__ __forceinline__ void fused_block(const S *__restrict__ sa, const S *_
     }
 }
 template <class LA, class LB, class Body, class S>
-__global__ void __launch_bounds__(kBlock) k_collide_fused(const S *__restrict__ sa, const S *__restrict__ sb,
+__global__ void __launch_bounds__(kBlock, kLateCoef<Body> ? 4 : 1) k_collide_fused(const S *__restrict__ sa, const S *__restrict__ sb,
                                                           S *__restrict__ da, S *__restrict__ db, Grid g, ProgView pv,
                                                           int any_smooth, Body body) {
     fused_block<LA, LB, Body, S>(sa, sb, da, db, g, pv, any_smooth, body, blockIdx.x, gridDim.x, pv.xcd);
@@ -706,7 +720,7 @@ struct BatchItem {
     int any_smooth;
 };
 template <class LA, class LB, class Body, class S>
-__global__ void __launch_bounds__(kBlock) k_collide_batch(const BatchItem<Body, S> *__restrict__ items,
+__global__ void __launch_bounds__(kBlock, kLateCoef<Body> ? 4 : 1) k_collide_batch(const BatchItem<Body, S> *__restrict__ items,
                                                           const int2 *__restrict__ tiles,
                                                           const int *__restrict__ active, int nitem, int xcd,
                                                           int rows) {

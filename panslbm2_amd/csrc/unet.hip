@@ -268,7 +268,8 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
     const int xo = blockIdx.z * cxg;  // this workgroup's input channels: [xo, xo + cxg)
     const int nmt = cg / 16, nnt = cxg / 16, tiles = nmt * nnt;
     const int row = (kt + 8) * 2;  // bytes of an LDS row
-    unsigned char *sg = lds, *sx = lds + cg * row;
+    auto at = [&](int c) { return c * row + c / 8 * 16; };  // where row c begins
+    unsigned char *sg = lds, *sx = lds + at(cg);
     // products 4 s + wave: tap t, output rows mt, input rows nt
     f4 acc[NA];
     int arow[NA], brow[NA];
@@ -277,13 +278,13 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
         acc[s] = f4{0.f, 0.f, 0.f, 0.f};
         const int u = min(wv + 4 * s, TX * tiles - 1);
         const int t = u / tiles, mn = u - t * tiles, mt = mn / nnt, nt = mn - mt * nnt;
-        arow[s] = mt * 16 * row;
-        brow[s] = (t * cxg + nt * 16) * row;
+        arow[s] = at(mt * 16);
+        brow[s] = at(t * cxg + nt * 16);
     }
     // the thread's unit: 8 voxels x 8 channels of g, or of x
     const int groups = kt / 8, gunits = groups * (cg / 8), units = gunits + groups * (cxg / 8);
     const bool is_g = tid < gunits, is_x = !is_g && tid < units;
-    const int un = is_g ? tid : tid - gunits, vg = un % groups, c8 = (un / groups) * 8;
+    const int un = is_g ? tid : tid - gunits, n8 = (is_g ? cg : cxg) / 8, vg = un / n8, c8 = un % n8 * 8;
     const bool bias = yz == 0 && xo == 0 && tid < 4 * cg;
     const int bo = tid >> 2, bq = tid & 3;
     float bsum = 0.f;
@@ -336,7 +337,7 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
         uint4 o[8];
         transpose8(v, o);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) *(uint4 *)(rows + (c8 + j) * row + vg * 16) = o[j];
+        for (int j = 0; j < 8; ++j) *(uint4 *)(rows + at(c8) + j * row + vg * 16) = o[j];
     };
     load(vbeg);
     for (int vb = vbeg; vb < vend; vb += kt) {
@@ -362,7 +363,7 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
                         if (t == 2) on &= ~(edge >> (8 + i));
                         v[i] = keep(d[i + t], on);
                     }
-                    put(sx + t * cxg * row, v);
+                    put(sx + at(t * cxg), v);
                 }
             }
         }
@@ -370,7 +371,7 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
         if (vb + kt < vend) load(vb + kt);
         if (bias)
             for (int v64 = 0; v64 < kt; v64 += 64) {
-                const uint4 *e = (const uint4 *)(sg + bo * row + (v64 + bq * 16) * 2);
+                const uint4 *e = (const uint4 *)(sg + at(bo) + (v64 + bq * 16) * 2);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const uint4 w = e[h];
@@ -382,7 +383,7 @@ __global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g
                     }
                 }
             }
-        const unsigned char *ga = sg + r * row + 16 * q, *xa = sx + r * row + 16 * q;
+        const unsigned char *ga = sg + at(r) + 16 * q, *xa = sx + at(r) + 16 * q;
 #pragma unroll 4
         for (int kh = 0; kh < kt / 32; ++kh) {
 #pragma unroll
@@ -803,7 +804,7 @@ int conv_grads(lbm_unet *N, const lbm_unet::Conv &c, const bf16_t *g, const bf16
     const int tx = c.taps == 27 ? 3 : 1, cxg = cxp == 48 ? 16 : cxp, tiles = tx * (cg / 16) * (cxg / 16);
     if (tiles > (tx == 3 ? 48 : 16)) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d tiles", tiles);
     int kt = 512;
-    auto rows = [&](int k) { return (cg + tx * cxg) * (k + 8) * 2; };
+    auto rows = [&](int k) { return (cg + tx * cxg) * (k + 9) * 2; };
     while (kt > kTileV && (kt / 8 * ((cg + cxg) / 8) > 256 || rows(kt) > 72 * 1024)) kt /= 2;
     if (kt / 8 * ((cg + cxg) / 8) > 256) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d x %d channels", cg, cxp);
     auto *kernel = tx == 3 ? &k_conv_wgrad<3> : &k_conv_wgrad<1>;
