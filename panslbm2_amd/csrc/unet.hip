@@ -35,6 +35,7 @@
 
 #include "../../include/panslbm2_amd.h"
 #include "context.h"
+#include "lattice.h"
 
 namespace {
 
@@ -43,8 +44,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f4;
 
 constexpr int kMaxFields = 16;
-constexpr int kMaxCg = 64;   // widest output gradient a weight-gradient launch stages
-constexpr int kMaxCx = 96;   // widest input it stages
 constexpr int kTileV = 64;   // voxel ranges of the weight gradient are multiples of this
 
 __host__ __device__ inline bf16_t f2bf(float f) {
@@ -140,7 +139,7 @@ __device__ __forceinline__ uint4 keep(const uint4 &d, uint32_t bit) {
 // (m, n) computes 16 MT output channels of z layer n, 4 rows of 16 voxels.  Read from global memory
 // per tap, as it was, every input came through L1 27 times and each of those reads cost an address
 // and three bounds checks: at 96x96x48 and 16 -> 16 channels 58 us (109 TFLOP/s), bound by vector
-// instructions and L1.  Here a K step of 32 costs one LDS read of 16 bytes per lane and row at an
+// instructions and L1; 25 us (249 TFLOP/s) now.  Here a K step of 32 costs one LDS read of 16 bytes per lane and row at an
 // address the compiler knows up to a per-lane base, and its weights; all K steps are unrolled.
 // A voxel's row in LDS is 16 bytes longer than its channels (CIN = 8: not), so that the 16 lanes of a
 // row fall into different banks.  The products are summed in the order k = 0, 32, ... as before.
@@ -229,207 +228,193 @@ __global__ void __launch_bounds__(64 * WM * WN) k_conv3(const bf16_t *__restrict
 // ---- weight gradient ----------------------------------------------------------------------------
 // part[split][tap][o][i] = sum over the split's voxels v of g[v][o] x[v + off(tap)][i].
 // Matrix core: A[m = o][k = v], B[k = v][n = i], K steps of 32 voxels in ascending order.
-// The first tap's workgroups also sum the staged g: bpart[split][o] = sum over the split of g[v][o],
-// as four sums over every fourth 16-voxel run.
+// bpart[split][o] = sum over the split of g[v][o], as four sums over every fourth 16-voxel run.
 //
-// A workgroup takes the TX taps along x of one (dy, dz) (3, or 1 for the 1x1x1 head) over one split.
-// Per tile of kt voxels a thread loads 8 channels of the 8 (or, shifted, 10) voxels it owns, transposes
-// them in registers (v_perm) and writes 8-voxel rows of 16 bytes to LDS, once per tap: the operands
-// then are 16-byte LDS reads.  The next tile's loads are issued before the products of this one.
-// One tap per workgroup, element-wise LDS writes and no prefetch, as it was, read g and x 27 times:
-// 178 us on average over the layers at 96x96x48.  LDS rows are kt + 8 voxels, so that the 16 rows of an
-// operand fall into different banks.
-__device__ __forceinline__ void transpose8(const uint4 (&d)[8], uint4 (&o)[8]) {
-    const uint32_t *s = reinterpret_cast<const uint32_t *>(d);  // s[4 voxel + p]: channels 2p, 2p + 1
-    uint32_t *t = reinterpret_cast<uint32_t *>(o);              // t[4 channel + m]: voxels 2m, 2m + 1
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            t[4 * (2 * p) + m] = __builtin_amdgcn_perm(s[4 * (2 * m + 1) + p], s[4 * (2 * m) + p], 0x05040100u);
-            t[4 * (2 * p + 1) + m] = __builtin_amdgcn_perm(s[4 * (2 * m + 1) + p], s[4 * (2 * m) + p], 0x07060302u);
-        }
+// 3x3x3: a workgroup takes the three taps along x of one (dy, dz) over one split, a wavefront per tap
+// with all of its CG x CX products (the fourth only stages).  Tiles of KT voxels go to LDS as they lie in
+// memory, voxel by voxel, so that every load is a run of 16-byte pieces; the matrix core's operands want
+// eight voxels of one channel, which the transposing LDS read gives (16 lanes read four voxels of 16
+// channels, each lane gets four voxels of one).  The three taps read the same x, one voxel apart; a lane
+// whose voxel has no x neighbour reads a row of zeros.  The next tile's loads are issued before the
+// products of this one.  What bounds it is the chain of tiles: 38 splits x 9 workgroups on 256 CUs, each
+// of a tile's loads, stores and products in turn.  KT: 16384 voxel-channels, 32 kB of loads in flight.
+// At 96x96x48, 16 x 16 channels 60 us and 16 x 48 99 us, 3.8e2 us over the ten layers; one tap per
+// workgroup with element-wise LDS writes took 178 us a layer, rows transposed in registers with a copy of
+// x per tap in LDS 138, 377 and 1.0e3 us.  More splits would fill the chip better (56: a fifth less time
+// for the former kernel) but change the order of the sums.
+template <int CG, int CX>
+struct WgradTile {
+    static constexpr int CXP = (CX + 15) & ~15;
+    static constexpr int KT = CG + CXP <= 32 ? 512 : (CG + CXP <= 64 ? 256 : 128);
+};
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+// four voxels (rows) of 16 channels: lane l of 16 points at channels 4 (l % 4).. of row l / 4 and gets
+// the four rows of channel l; two of them are an operand's eight voxels
+__device__ __forceinline__ s16x4 tr4(const unsigned char *p) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p);
 }
-template <int TX>
-__global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g, int cg,
-                                                    const bf16_t *__restrict__ x, int cx, int nx, int ny, int nz,
-                                                    int chunk, int kt, int cxg, float *__restrict__ part,
+__device__ __forceinline__ bf16x8 tr8(const unsigned char *p, const unsigned char *p4) {
+    const s16x4 a = tr4(p), b = tr4(p4);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+// TAPS 1 (the head): one tap, one wavefront of products, and a thousand splits of one tile.
+template <int CG, int CX, int TAPS>
+__global__ void __launch_bounds__(256) k_conv_wgrad(const bf16_t *__restrict__ g, const bf16_t *__restrict__ x,
+                                                    int nx, int ny, int nz, lbm::FastDiv by_nx, lbm::FastDiv by_ny,
+                                                    int nsplit, int chunk, float *__restrict__ part,
                                                     float *__restrict__ bpart) {
-    constexpr int NA = TX == 3 ? 12 : 4;  // products a wave owns at most: TX (cg / 16) (cxp / 16) / 4
-    constexpr int NL = TX == 3 ? 10 : 8;  // voxels a thread of x loads: its 8 and their x neighbours
-    extern __shared__ __align__(16) unsigned char lds[];
+    constexpr int CXP = WgradTile<CG, CX>::CXP, KT = WgradTile<CG, CX>::KT, NM = CG / 16, NN = CXP / 16;
+    constexpr int TX = TAPS == 27 ? 3 : 1, NYZ = TAPS / TX;
+    constexpr int G8 = CG / 8, X8 = CX / 8;                         // 16-byte pieces of a voxel
+    constexpr int GU = KT * G8 / 256, XU = KT * X8 / 256;           // pieces a thread stages per tile
+    // K steps at once, so that their LDS reads are under way together (the rows past the split are zeros)
+    constexpr int U = NM * NN <= 2 ? 8 : (NM * NN <= 4 ? 4 : 2);
+    constexpr int SG = CG * 2, SX = CXP * 2, ZERO = (KT + 2) * SX;  // bytes of an LDS row; the row of zeros
+    static_assert(KT * G8 % 256 == 0 && KT * X8 % 256 == 0 && KT / 32 % U == 0, "whole pieces per thread, whole groups of steps");
+    __shared__ __align__(16) unsigned char sg[KT * SG];
+    __shared__ __align__(16) unsigned char sx[(KT + 3) * SX];  // voxels vb - 1 .. vb + KT, zeros
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int split = blockIdx.x, yz = blockIdx.y, taps = TX * gridDim.y;
-    const int V = nx * ny * nz;
-    const int dy = TX == 3 ? yz % 3 - 1 : 0, dz = TX == 3 ? yz / 3 - 1 : 0;
+    // the workgroups of a split are on one XCD (workgroup id mod 8), one after another
+    const int slot = blockIdx.x >> 3, split = slot / NYZ * 8 + (blockIdx.x & 7), yz = slot % NYZ;
+    if (split >= nsplit) return;
+    const int V = nx * ny * nz, dy = TAPS == 27 ? yz % 3 - 1 : 0, dz = TAPS == 27 ? yz / 3 - 1 : 0;
+    const int off = (dy + ny * dz) * nx;
     const int vbeg = split * chunk, vend = min(V, vbeg + chunk);
-    const int cxp = (cx + 15) & ~15;
-    const int xo = blockIdx.z * cxg;  // this workgroup's input channels: [xo, xo + cxg)
-    const int nmt = cg / 16, nnt = cxg / 16, tiles = nmt * nnt;
-    const int row = (kt + 8) * 2;  // bytes of an LDS row
-    auto at = [&](int c) { return c * row + c / 8 * 16; };  // where row c begins
-    unsigned char *sg = lds, *sx = lds + at(cg);
-    // products 4 s + wave: tap t, output rows mt, input rows nt
-    f4 acc[NA];
-    int arow[NA], brow[NA];
-#pragma unroll
-    for (int s = 0; s < NA; ++s) {
-        acc[s] = f4{0.f, 0.f, 0.f, 0.f};
-        const int u = min(wv + 4 * s, TX * tiles - 1);
-        const int t = u / tiles, mn = u - t * tiles, mt = mn / nnt, nt = mn - mt * nnt;
-        arow[s] = at(mt * 16);
-        brow[s] = at(t * cxg + nt * 16);
-    }
-    // the thread's unit: 8 voxels x 8 channels of g, or of x
-    const int groups = kt / 8, gunits = groups * (cg / 8), units = gunits + groups * (cxg / 8);
-    const bool is_g = tid < gunits, is_x = !is_g && tid < units;
-    const int un = is_g ? tid : tid - gunits, n8 = (is_g ? cg : cxg) / 8, vg = un / n8, c8 = un % n8 * 8;
-    const bool bias = yz == 0 && xo == 0 && tid < 4 * cg;
-    const int bo = tid >> 2, bq = tid & 3;
-    float bsum = 0.f;
-    uint4 d[NL];
-    // bit i: the thread's voxel i is at x = 0; 8 + i: at x = nx - 1; 16 + i: it counts (in the split, its
-    // row at (dy, dz) in the grid).  Loads go to clamped addresses and are masked when they are used:
-    // a load under a condition is waited for before the next one is issued.
-    uint32_t edge = 0;
+    const uint4 none{0u, 0u, 0u, 0u};
+    if (tid < SX / 16) *(uint4 *)(sx + ZERO + 16 * tid) = none;
+    if constexpr (CX < CXP)  // the channels that pad x
+        for (int i = tid; i < (KT + 2) * (CXP - CX) / 8; i += 256)
+            *(uint4 *)(sx + i / ((CXP - CX) / 8) * SX + CX * 2 + i % ((CXP - CX) / 8) * 16) = none;
+    uint4 dg[GU], dx[XU], dh = none;
+    uint32_t in = 0;  // bit i: piece i of g counts; 16 + i: of x; 31: the halo piece
+    // x of voxel u + off counts if u is a voxel whose row at (dy, dz) is in the grid
+    auto load_x = [&](int u, int c, uint32_t &ok) {
+        const int row = (int)lbm::div_by((uint32_t)max(u, 0), by_nx), zz = (int)lbm::div_by((uint32_t)row, by_ny);
+        ok = u >= 0 && u < V && (unsigned)(row - zz * ny + dy) < (unsigned)ny && (unsigned)(zz + dz) < (unsigned)nz;
+        return *(const uint4 *)(x + (size_t)min(max(u + off, 0), V - 1) * CX + c * 8);
+    };
+    const int hs = tid / X8;  // threads of the halo: 0 the voxel before the tile, 1 the one after it
     auto load = [&](int vb) {
-        const int v0 = vb + 8 * vg;
-        edge = 0;
-        if (is_g) {
+        in = 0;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                d[i] = *(const uint4 *)(g + (size_t)min(v0 + i, V - 1) * cg + c8);
-                edge |= (uint32_t)(v0 + i < vend) << (16 + i);
-            }
-        } else if (is_x) {
-            const bool real = xo + c8 < cx;
-            const int cl = real ? xo + c8 : 0;
-            if constexpr (TX == 1) {
+        for (int i = 0; i < GU; ++i) {
+            const int p = tid + 256 * i, v = vb + p / G8;
+            dg[i] = *(const uint4 *)(g + (size_t)min(v, V - 1) * CG + p % G8 * 8);
+            in |= (uint32_t)(v < vend) << i;
+        }
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    d[i] = *(const uint4 *)(x + (size_t)min(v0 + i, V - 1) * cx + cl);
-                    edge |= (uint32_t)(v0 + i < vend && real) << (16 + i);
-                }
-            } else {
-                const int l0 = v0 - 1 + (dy + ny * dz) * nx;
-#pragma unroll
-                for (int i = 0; i < 10; ++i)
-                    d[i] = *(const uint4 *)(x + (size_t)min(max(l0 + i, 0), V - 1) * cx + cl);
-                int xx = v0 % nx, yy = (v0 / nx) % ny, zz = v0 / (nx * ny);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const bool in = v0 + i < vend && real && (unsigned)(yy + dy) < (unsigned)ny &&
-                                    (unsigned)(zz + dz) < (unsigned)nz;
-                    edge |= (uint32_t)(xx == 0) << i | (uint32_t)(xx == nx - 1) << (8 + i) | (uint32_t)in << (16 + i);
-                    if (++xx == nx) {
-                        xx = 0;
-                        if (++yy == ny) {
-                            yy = 0;
-                            ++zz;
-                        }
-                    }
-                }
-            }
+        for (int i = 0; i < XU; ++i) {
+            const int p = tid + 256 * i;
+            uint32_t ok;
+            dx[i] = load_x(vb + p / X8, p % X8, ok);
+            in |= ok << (16 + i);
+        }
+        if (hs < 2) {
+            uint32_t ok;
+            dh = load_x(hs ? vb + KT : vb - 1, tid % X8, ok);
+            in |= ok << 31;
         }
     };
-    auto put = [&](unsigned char *rows, const uint4 (&v)[8]) {
-        uint4 o[8];
-        transpose8(v, o);
+    f4 acc[NM][NN];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) *(uint4 *)(rows + at(c8) + j * row + vg * 16) = o[j];
-    };
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int n = 0; n < NN; ++n) acc[m][n] = f4{0.f, 0.f, 0.f, 0.f};
+    const int rot = 32 % nx, none_at = TX == 1 || wv == 1 ? -1 : (wv == 0 ? 0 : nx - 1);  // x without a neighbour at this tap
+    const int shift = TX == 1 ? 1 : wv;  // of the tap's x rows against g's
+    const int l4 = 8 * q + (r >> 2), lc = (r & 3) * 8;
+    const int bt = tid - (256 - 4 * CG);  // the bias's threads, from the fourth wavefront down
+    const bool bias = yz == 0 && bt >= 0;
+    const int bo = bt & (CG - 1), bq = bt / CG;
+    float bsum = 0.f;
     load(vbeg);
-    for (int vb = vbeg; vb < vend; vb += kt) {
-        if (is_g) {
-            uint4 v[8];
+    for (int vb = vbeg; vb < vend; vb += KT) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = keep(d[i], edge >> (16 + i));
-            put(sg, v);
-        } else if (is_x) {
-            if constexpr (TX == 1) {
-                uint4 v[8];
+        for (int i = 0; i < GU; ++i) *(uint4 *)(sg + (tid + 256 * i) * 16) = keep(dg[i], in >> i);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = keep(d[i], edge >> (16 + i));
-                put(sx, v);
-            } else {
-#pragma unroll
-                for (int t = 0; t < 3; ++t) {
-                    uint4 v[8];
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        uint32_t on = edge >> (16 + i);
-                        if (t == 0) on &= ~(edge >> i);
-                        if (t == 2) on &= ~(edge >> (8 + i));
-                        v[i] = keep(d[i + t], on);
-                    }
-                    put(sx + at(t * cxg), v);
-                }
-            }
+        for (int i = 0; i < XU; ++i) {
+            const int p = tid + 256 * i;
+            *(uint4 *)(sx + (1 + p / X8) * SX + p % X8 * 16) = keep(dx[i], in >> (16 + i));
         }
+        if (hs < 2) *(uint4 *)(sx + (hs ? KT + 1 : 0) * SX + tid % X8 * 16) = keep(dh, in >> 31);
         __syncthreads();
-        if (vb + kt < vend) load(vb + kt);
+        if (vb + KT < vend) load(vb + KT);
+        const int steps = (min(KT, vend - vb) + 31) / 32;
         if (bias)
-            for (int v64 = 0; v64 < kt; v64 += 64) {
-                const uint4 *e = (const uint4 *)(sg + at(bo) + (v64 + bq * 16) * 2);
+            for (int v64 = 0; v64 < 32 * steps; v64 += 64) {
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const uint4 w = e[h];
-                    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+                for (int j = 0; j < 16; ++j) bsum += bf2f(*(const bf16_t *)(sg + (v64 + bq * 16 + j) * SG + bo * 2));
+            }
+        if (wv < TX) {
+            int x0 = vb + l4, x4 = x0 + 4;  // the x of the lane's voxels
+            x0 -= (int)lbm::div_by((uint32_t)x0, by_nx) * nx;
+            x4 -= (int)lbm::div_by((uint32_t)x4, by_nx) * nx;
+            for (int k0 = 0; k0 < steps; k0 += U) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        bsum += bf2f((bf16_t)(ws[j] & 0xffffu));
-                        bsum += bf2f((bf16_t)(ws[j] >> 16));
+                for (int k = k0; k < k0 + U; ++k) {
+                    const unsigned char *ga = sg + (32 * k + l4) * SG + lc, *xa = sx + (32 * k + l4 + shift) * SX + lc;
+                    const unsigned char *b0 = x0 == none_at ? sx + ZERO + lc : xa;
+                    const unsigned char *b4 = x4 == none_at ? sx + ZERO + lc : xa + 4 * SX;
+                    bf16x8 a[NM];
+#pragma unroll
+                    for (int m = 0; m < NM; ++m) a[m] = tr8(ga + 32 * m, ga + 4 * SG + 32 * m);
+#pragma unroll
+                    for (int n = 0; n < NN; ++n) {
+                        const bf16x8 b = tr8(b0 + 32 * n, b4 + 32 * n);
+#pragma unroll
+                        for (int m = 0; m < NM; ++m)
+                            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b, acc[m][n], 0, 0, 0);
                     }
-                }
-            }
-        const unsigned char *ga = sg + at(r) + 16 * q, *xa = sx + at(r) + 16 * q;
-#pragma unroll 4
-        for (int kh = 0; kh < kt / 32; ++kh) {
-#pragma unroll
-            for (int s = 0; s < NA; ++s) {
-                if (wv + 4 * s < TX * tiles) {
-                    const bf16x8 a = __builtin_bit_cast(bf16x8, *(const uint4 *)(ga + arow[s] + 64 * kh));
-                    const bf16x8 b = __builtin_bit_cast(bf16x8, *(const uint4 *)(xa + brow[s] + 64 * kh));
-                    acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[s], 0, 0, 0);
+                    x0 += rot;
+                    x0 -= x0 >= nx ? nx : 0;
+                    x4 += rot;
+                    x4 -= x4 >= nx ? nx : 0;
                 }
             }
         }
         __syncthreads();
     }
+    if (wv < TX) {
+        float *out = part + ((size_t)split * TAPS + 3 * yz + wv) * CG * CXP;
 #pragma unroll
-    for (int s = 0; s < NA; ++s) {
-        const int u = wv + 4 * s;
-        if (u < TX * tiles) {
-            const int t = u / tiles, mn = u - t * tiles, mt = mn / nnt, nt = mn - mt * nnt;
-            float *out = part + ((size_t)split * taps + (TX == 3 ? 3 * yz + t : 0)) * cg * cxp;
+        for (int m = 0; m < NM; ++m)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) out[(size_t)(mt * 16 + 4 * q + j) * cxp + xo + nt * 16 + r] = acc[s][j];
-        }
+            for (int n = 0; n < NN; ++n)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) out[(size_t)(m * 16 + 4 * q + j) * CXP + n * 16 + r] = acc[m][n][j];
     }
-    if (yz == 0 && xo == 0) {  // uniform per workgroup
-        __shared__ float bred[4 * kMaxCg];
-        if (bias) bred[tid] = bsum;
+    if (yz == 0) {  // uniform per workgroup
+        float *bred = reinterpret_cast<float *>(sg);
+        if (bias) bred[4 * bo + bq] = bsum;
         __syncthreads();
-        if (tid < cg) bpart[(size_t)split * cg + tid] = (bred[4 * tid] + bred[4 * tid + 1]) + (bred[4 * tid + 2] + bred[4 * tid + 3]);
+        if (tid < CG) bpart[(size_t)split * CG + tid] = (bred[4 * tid] + bred[4 * tid + 1]) + (bred[4 * tid + 2] + bred[4 * tid + 3]);
     }
 }
 
 // grad[(o taps + tap) ci + i] = sum over splits (in order) of part[split][tap][o][i]; the bias
 // gradient follows the weights: grad[co taps ci + o] = sum over splits of bpart[split][o].  The adds
-// are a serial chain per parameter (the order is fixed); its loads are not, so 16 are in flight at
-// once (the head's 1,024 splits for 221 parameters: 423 us with one load per add).
-__device__ __forceinline__ float sum_splits(const float *__restrict__ p, size_t stride, int n) {
+// are a serial chain per parameter (the order is fixed); its loads are not, so 64 are in flight at
+// once, then 16 (the head's 988 splits for 221 parameters: 423 us with one load per add, 46 with 16 in
+// flight, now 27; 64 for the other layers' 38, with a clamped rest: 12 us instead of 4.7).
+template <int B>
+__device__ __forceinline__ void sum_batches(float &s, int &i, const float *__restrict__ &base, uint32_t at,
+                                            size_t stride, int n) {
+    for (; i + B <= n; i += B) {  // base is the same for all lanes: one scalar add per load
+        float v[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j, base += stride) v[j] = base[at];
+#pragma unroll
+        for (int j = 0; j < B; ++j) s += v[j];
+    }
+}
+__device__ __forceinline__ float sum_splits(const float *__restrict__ base, uint32_t at, size_t stride, int n) {
     float s = 0.f;
     int i = 0;
-    for (; i + 16 <= n; i += 16) {
-        float v[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) v[j] = p[(size_t)(i + j) * stride];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) s += v[j];
-    }
-    for (; i < n; ++i) s += p[(size_t)i * stride];
+    sum_batches<64>(s, i, base, at, stride, n);
+    sum_batches<16>(s, i, base, at, stride, n);
+    sum_batches<1>(s, i, base, at, stride, n);
     return s;
 }
 __global__ void __launch_bounds__(64) k_wgrad_reduce(const float *__restrict__ part, const float *__restrict__ bpart,
@@ -440,9 +425,9 @@ __global__ void __launch_bounds__(64) k_wgrad_reduce(const float *__restrict__ p
     if (n >= nw + co) return;
     if (n < nw) {
         const int i = n % ci, t = (n / ci) % taps, o = n / (ci * taps);
-        grad[n] = sum_splits(part + ((size_t)t * cg + o) * cxp + i, (size_t)taps * cg * cxp, nsplit);
+        grad[n] = sum_splits(part, (t * cg + o) * cxp + i, (size_t)taps * cg * cxp, nsplit);
     } else {
-        grad[n] = sum_splits(bpart + (n - nw), (size_t)cg, nsplit);
+        grad[n] = sum_splits(bpart, n - nw, (size_t)cg, nsplit);
     }
 }
 
@@ -789,30 +774,33 @@ void wsplit(int V, int taps, int *nsplit, int *chunk) {
     *nsplit = (V + ch - 1) / ch;
 }
 
+template <int CG, int CX, int TAPS>
+void launch_wgrad(lbm_unet *N, const bf16_t *g, const bf16_t *x, const int *d, int nsplit, int chunk) {
+    k_conv_wgrad<CG, CX, TAPS><<<(nsplit + 7) / 8 * 8 * (TAPS == 27 ? 9 : 1), 256, 0, N->s>>>(
+        g, x, d[0], d[1], d[2], lbm::fast_div(d[0]), lbm::fast_div(d[1]), nsplit, chunk, N->wpart, N->bpart);
+}
+
 // gradient of conv c: g is the output gradient (bf16, r16(co) channels), x its input (cis channels)
 int conv_grads(lbm_unet *N, const lbm_unet::Conv &c, const bf16_t *g, const bf16_t *x) {
     const int *d = N->dims[c.level];
     const int V = N->V[c.level], cg = r16(c.co), cxp = r16(c.cis);
-    if (cg > kMaxCg || c.cis > kMaxCx) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d x %d channels", cg, c.cis);
     int nsplit, chunk;
     wsplit(V, c.taps, &nsplit, &chunk);
     if ((size_t)nsplit * c.taps * cg * cxp > N->wpart_n) return lbm::set_error(LBM_ERR_ARG, "weight partials overflow");
     if ((size_t)nsplit * cg > N->bpart_n) return lbm::set_error(LBM_ERR_ARG, "bias partials overflow");
-    // A workgroup's time is its chain of tiles, each a memory round trip, a transposition and its
-    // products, so: as many voxels per tile as give every thread a unit and fit 72 kB of rows (two
-    // workgroups per CU), and 48 input channels as three workgroups of 16, each with the longer tile.
-    const int tx = c.taps == 27 ? 3 : 1, cxg = cxp == 48 ? 16 : cxp, tiles = tx * (cg / 16) * (cxg / 16);
-    if (tiles > (tx == 3 ? 48 : 16)) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d tiles", tiles);
-    int kt = 512;
-    auto rows = [&](int k) { return (cg + tx * cxg) * (k + 9) * 2; };
-    while (kt > kTileV && (kt / 8 * ((cg + cxg) / 8) > 256 || rows(kt) > 72 * 1024)) kt /= 2;
-    if (kt / 8 * ((cg + cxg) / 8) > 256) return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d x %d channels", cg, cxp);
-    auto *kernel = tx == 3 ? &k_conv_wgrad<3> : &k_conv_wgrad<1>;
-    if (rows(kt) > 60 * 1024)
-        UCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 rows(kt)));
-    kernel<<<dim3(nsplit, c.taps / tx, cxp / cxg), 256, rows(kt), N->s>>>(g, cg, x, c.cis, d[0], d[1], d[2], chunk, kt,
-                                                                         cxg, N->wpart, N->bpart);
+    const int shape = (c.taps == 27 ? 0 : 10000) + cg * 100 + c.cis;
+    switch (shape) {
+    case 1608: launch_wgrad<16, 8, 27>(N, g, x, d, nsplit, chunk); break;
+    case 1616: launch_wgrad<16, 16, 27>(N, g, x, d, nsplit, chunk); break;
+    case 1648: launch_wgrad<16, 48, 27>(N, g, x, d, nsplit, chunk); break;
+    case 3216: launch_wgrad<32, 16, 27>(N, g, x, d, nsplit, chunk); break;
+    case 3232: launch_wgrad<32, 32, 27>(N, g, x, d, nsplit, chunk); break;
+    case 3296: launch_wgrad<32, 96, 27>(N, g, x, d, nsplit, chunk); break;
+    case 6432: launch_wgrad<64, 32, 27>(N, g, x, d, nsplit, chunk); break;
+    case 6464: launch_wgrad<64, 64, 27>(N, g, x, d, nsplit, chunk); break;
+    case 11616: launch_wgrad<16, 16, 1>(N, g, x, d, nsplit, chunk); break;
+    default: return lbm::set_error(LBM_ERR_ARG, "weight gradient: %d x %d channels, %d taps", cg, c.cis, c.taps);
+    }
     UCHK(hipGetLastError());
     const int nw = c.co * c.taps * c.ci;  // the bias follows the weights in the parameter vector
     k_wgrad_reduce<<<blocks(nw + c.co, 64), 64, 0, N->s>>>(N->wpart, N->bpart, nsplit, c.taps, cg, cxp, c.co, c.ci,
