@@ -23,7 +23,7 @@ Also reported:
                    sensitivity's error against the FP64 evaluation.
   c3_smoothed   -- the same evaluation with SmoothCorner on both lattices every step (the
                    reference's 3D driver sequence, heatsink3D.cpp:175-176, 215-216), FP64: the
-                   fused pass plus the edges and corners on a second stream concurrently with it.
+                   fused pass with the edges and corners finished by its first lanes.
   heatsink2d    -- the 2D heat sink (200 x 400, D2Q9 + D2Q5, FP64): MLUPS, its fused step's roofline,
                    the same kernel on 4096^2 (HBM bound), FP32 / FP16 variants, the reference pairing
                    D2Q9 + D2Q9 and the reference CPU path on it.

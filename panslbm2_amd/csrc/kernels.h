@@ -214,7 +214,9 @@ __device__ __forceinline__ void settle(double *f) {
 // itself which operator and which face to run, the wavefront walked every branch of a decision
 // tree per operator, in four inlined copies, after three dependent memory round trips.  Here the
 // wavefront takes the forms its lanes have one after the other (nearly always one or two); a form's
-// words are uniform, so the choice of operator and face is scalar branches over one copy.
+// words are uniform, so the choice of operator and face is scalar branches over one copy.  FP64 forward
+// steps: 200x400 heat sink 9.1 -> 7.6 us (5.9 without boundaries), 96x96x48 duct 36.7 -> 34 us, 128x128x64
+// 84 -> 78 us.
 template <class LA, class LB, class Smooth>
 __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, int n, double *a, double *b,
                                         Smooth &&smooth) {

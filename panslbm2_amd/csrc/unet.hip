@@ -139,8 +139,9 @@ __device__ __forceinline__ uint4 keep(const uint4 &d, uint32_t bit) {
 // (m, n) computes 16 MT output channels of z layer n, 4 rows of 16 voxels.  Read from global memory
 // per tap, as it was, every input came through L1 27 times and each of those reads cost an address
 // and three bounds checks: at 96x96x48 and 16 -> 16 channels 58 us (109 TFLOP/s), bound by vector
-// instructions and L1; 25 us (249 TFLOP/s) now.  Here a K step of 32 costs one LDS read of 16 bytes per lane and row at an
-// address the compiler knows up to a per-lane base, and its weights; all K steps are unrolled.
+// instructions and L1; 25 us (249 TFLOP/s) now.  Here a K step of 32 costs one LDS read of 16 bytes
+// per lane and row at an address the compiler knows up to a per-lane base, and its weights; all K
+// steps are unrolled.
 // A voxel's row in LDS is 16 bytes longer than its channels (CIN = 8: not), so that the 16 lanes of a
 // row fall into different banks.  The products are summed in the order k = 0, 32, ... as before.
 template <int CIN>
@@ -163,6 +164,15 @@ __global__ void __launch_bounds__(64 * WM * WN) k_conv3(const bf16_t *__restrict
     const int wm = wv % WM, wn = wv / WM;
     const int bx = blockIdx.x % ntx, by = (blockIdx.x / ntx) % nty, bz = blockIdx.x / (ntx * nty);
     const int x0 = bx * 16, y0 = by * 4, z0 = bz * WN;
+    // the weights of the first AHEAD steps; in the loop a step loads those of the step AHEAD later
+    constexpr int AHEAD = MT == 1 ? 8 : 4;
+    const int co0 = (blockIdx.y * WM + wm) * 16 * MT;
+    const bf16_t *wr = w + (size_t)(co0 + r) * KPAD + 8 * q;
+    bf16x8 a[AHEAD][MT];
+#pragma unroll
+    for (int s = 0; s < AHEAD && s < KS; ++s)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) a[s][mt] = ld8(wr + (size_t)mt * 16 * KPAD + 32 * s);
     // loads from clamped addresses, zeroed afterwards, so that a batch of them is in flight at once
     constexpr int CU = CIN / 8, UNITS = NV * CU, IT = (UNITS + THREADS - 1) / THREADS, BATCH = IT < 8 ? IT : 8;
 #pragma unroll
@@ -189,14 +199,9 @@ __global__ void __launch_bounds__(64 * WM * WN) k_conv3(const bf16_t *__restrict
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
     __syncthreads();
-    const int co0 = (blockIdx.y * WM + wm) * 16 * MT;
-    const bf16_t *wr = w + (size_t)(co0 + r) * KPAD + 8 * q;
     const unsigned char *base = lds + (wn * 108 + r) * VS;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-        bf16x8 a[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) a[mt] = ld8(wr + (size_t)mt * 16 * KPAD + 32 * s);
         // the four lane groups' units: one tap with the next channels, or taps of their own
         const int o0 = B::off(4 * s), o1 = B::off(4 * s + 1), o2 = B::off(4 * s + 2), o3 = B::off(4 * s + 3);
         const int at = (o1 == o0 + 16 && o2 == o0 + 32 && o3 == o0 + 48)
@@ -210,7 +215,12 @@ __global__ void __launch_bounds__(64 * WM * WN) k_conv3(const bf16_t *__restrict
             const bf16x8 b = __builtin_bit_cast(bf16x8, d);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], b, acc[mt][nt], 0, 0, 0);
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s % AHEAD][mt], b, acc[mt][nt], 0, 0, 0);
+        }
+        if (s + AHEAD < KS) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) a[s % AHEAD][mt] = ld8(wr + (size_t)mt * 16 * KPAD + 32 * (s + AHEAD));
+            __builtin_amdgcn_sched_barrier(0x38f);  // or the compiler moves the loads down to their use
         }
     }
     const int vx = x0 + r, vz = z0 + wn;
@@ -497,7 +507,7 @@ __global__ void k_scatter(const float *__restrict__ y, int cs, int nf, int V, Fi
 
 // The elementwise kernels below take 8 channels (16 bytes of bfloat16) per thread: bandwidth-bound
 // copies and sums, which 2-byte accesses left at a few hundred GB/s (the level-1 concatenation at
-// 96x96x48, 85 MB: 122 us).
+// 96x96x48, 85 MB: 122 us, 13 us now).
 __device__ __forceinline__ void unpack8(const bf16_t *p, float (&v)[8]) {
     const uint4 d = *(const uint4 *)p;
     const uint32_t w[4] = {d.x, d.y, d.z, d.w};
@@ -733,8 +743,8 @@ int launch_conv3(lbm_unet *N, const bf16_t *x, const bf16_t *w, const ConvOut &o
 }
 // The network's shapes.  The waves of a workgroup share its brick: across the output channels as far
 // as there are tiles of 16 (every one of them would otherwise stage the same voxels), the rest along z;
-// three tiles to a wave where their number is a multiple of three.  At 96x96x48, 16 -> 16 channels:
-// 58 us before.
+// three tiles to a wave where their number is a multiple of three.  At 96x96x48: 16 -> 16 channels 25 us,
+// 16 -> 48 58 us, 48 -> 16 76 us, 32 -> 32 (48x48x24) 17 us.
 int launch_conv(lbm_unet *N, const bf16_t *x, int cin, int taps, const bf16_t *w, int kpad, const ConvOut &out,
                 const int *d) {
     const int V = d[0] * d[1] * d[2];
