@@ -156,26 +156,22 @@ struct lbm_program {
     // device tables
     bool uploaded = false;
     bool dev_used = false;  // device copies exist (a launch may still read them)
-    DevBuf d_slot_entry, d_entry_node, d_entry_ops, d_ops, d_form_ops, d_list_ops, d_slot_list, d_place_list;
+    // all tables in one allocation and one copy
+    DevBuf d_tables;
+    struct Table {
+        void *p = nullptr;
+    };
+    Table d_slot_entry, d_entry_node, d_entry_ops, d_ops, d_form_ops, d_sym, d_list_ops, d_slot_list, d_place_list;
     unsigned shared_places = 0, slot_places = 0;  // ProgView::shared, by_slot
-    DevBuf d_side_of_slot, d_smoothed, d_side;  // smoothing after the pass, from side states
-    DevBuf d_smooth_lanes;                      // 3D smoothing inside the pass (ProgView::smooth_lanes)
-    int nentry = 0, nslot = 0, maxops = 0, n_smoothed = 0, smooth_stride = 1, n_smooth_lanes = 0;
+    DevBuf d_side;                      // smoothing after the pass, from side states
+    Table d_side_of_slot, d_smoothed;
+    Table d_smooth_lanes;               // 3D smoothing inside the pass (ProgView::smooth_lanes)
+    int nentry = 0, nslot = 0, maxops = 0, nsym = 0, n_smoothed = 0, smooth_stride = 1, n_smooth_lanes = 0;
     bool smooth_in_pass_ok = false;  // the smoothed nodes may be done by the fused pass's first workgroups
     bool owned_by_ctx = false;  // eager scratch program
     ~lbm_program() {
-        d_slot_entry.release();
-        d_entry_node.release();
-        d_entry_ops.release();
-        d_ops.release();
-        d_form_ops.release();
-        d_list_ops.release();
-        d_slot_list.release();
-        d_place_list.release();
-        d_side_of_slot.release();
-        d_smoothed.release();
+        d_tables.release();
         d_side.release();
-        d_smooth_lanes.release();
     }
 };
 
@@ -395,6 +391,49 @@ lbm::ListVals pack_list(const Op *o, int count, uint32_t *words) {
     return v;
 }
 
+// The distinct operators of the forms (form -> maxops words, OP_NONE after its own), at most 64, in an
+// order that keeps every form's, and per form which of them it has.  False: more of them, or no order.
+bool merge_forms(const std::vector<uint32_t> &form_ops, int maxops, std::vector<uint32_t> &sym,
+                 std::vector<uint64_t> &has) {
+    const size_t nform = maxops ? form_ops.size() / maxops : 0;
+    std::map<std::pair<uint32_t, int>, int> id;  // (word, how often before it in the form)
+    std::vector<uint32_t> word;
+    std::vector<uint64_t> before;  // bit b of before[c]: some form has b right ahead of c
+    std::vector<std::vector<int>> ids(nform);
+    for (size_t f = 0; f < nform; ++f) {
+        const uint32_t *w = &form_ops[f * maxops];
+        for (int t = 0; t < maxops; ++t) {
+            if (!w[t]) {  // past the form's end, or an operator that does nothing
+                if (std::any_of(w + t, w + maxops, [](uint32_t x) { return x != 0; })) return false;
+                break;
+            }
+            const auto at = id.emplace(std::make_pair(w[t], (int)std::count(w, w + t, w[t])), (int)word.size());
+            if (at.second) {
+                if (word.size() == 64) return false;
+                word.push_back(w[t]);
+                before.push_back(0);
+            }
+            if (t) before[at.first->second] |= uint64_t(1) << ids[f].back();
+            ids[f].push_back(at.first->second);
+        }
+    }
+    std::vector<int> place(word.size(), -1);
+    uint64_t done = 0;
+    sym.clear();
+    while (sym.size() < word.size()) {
+        size_t c = 0;
+        while (c < word.size() && ((done >> c & 1u) || (before[c] & ~done))) ++c;
+        if (c == word.size()) return false;  // two forms have two operators in opposite orders
+        done |= uint64_t(1) << c;
+        place[c] = (int)sym.size();
+        sym.push_back(word[c]);
+    }
+    has.assign(nform, 0);
+    for (size_t f = 0; f < nform; ++f)
+        for (int c : ids[f]) has[f] |= uint64_t(1) << place[c];
+    return true;
+}
+
 int prog_upload(lbm_program *P) {
     if (P->uploaded) return LBM_OK;
     lbm_lattice *L = P->lat[0];
@@ -467,6 +506,12 @@ int prog_upload(lbm_program *P) {
         for (int t = 0; t < std::min(count, lbm::kWordOps); ++t) so.w[t / 4] |= (uint64_t)words[t] << (16 * (t % 4));
         slot_list[s] = so;
     }
+    std::vector<uint32_t> sym;
+    std::vector<uint64_t> has;
+    P->nsym = L->nd == 3 && merge_forms(form_ops, P->maxops, sym, has) ? (int)sym.size() : 0;  // see run_ops
+    if (P->nsym > 0)
+        for (lbm::NodeList &so : slot_list)
+            if (so.form >= 0) so.w[0] = has[so.form];
     // places whose nodes share one list (or have none), and places that have several
     std::vector<lbm::NodeList> place_list(lbm::kPlaces, lbm::NodeList{-1, -1, 0, 0, {0, 0}, {}});
     unsigned seen = 0;
@@ -580,23 +625,36 @@ int prog_upload(lbm_program *P) {
             return fail(LBM_ERR_HIP, "device allocation of the side states failed");
     }
     P->n_smoothed = (int)sm_ents.size() / P->smooth_stride;
-    auto up = [&](DevBuf &b, const void *src, size_t bytes) -> int {
-        if (b.ensure(bytes ? bytes : 8)) return fail(LBM_ERR_HIP, "device allocation of %zu bytes failed", bytes);
-        if (bytes) HIPCHK(hipMemcpy(b.p, src, bytes, hipMemcpyHostToDevice));
-        return LBM_OK;
+    struct Part {
+        lbm_program::Table *to;
+        const void *from;
+        size_t bytes, at;
     };
-    int rc;
-    if ((rc = up(P->d_slot_entry, slot_entry.data(), slot_entry.size() * sizeof(int)))) return rc;
-    if ((rc = up(P->d_entry_node, entry_node.data(), entry_node.size() * sizeof(int)))) return rc;
-    if ((rc = up(P->d_entry_ops, entry_ops.data(), entry_ops.size() * sizeof(int2)))) return rc;
-    if ((rc = up(P->d_ops, ops.data(), ops.size() * sizeof(Op)))) return rc;
-    if ((rc = up(P->d_form_ops, form_ops.data(), form_ops.size() * sizeof(uint32_t)))) return rc;
-    if ((rc = up(P->d_place_list, place_list.data(), place_list.size() * sizeof(lbm::NodeList)))) return rc;
-    if ((rc = up(P->d_list_ops, list_ops.data(), list_ops.size() * sizeof(Op)))) return rc;
-    if ((rc = up(P->d_slot_list, slot_list.data(), slot_list.size() * sizeof(lbm::NodeList)))) return rc;
-    if ((rc = up(P->d_side_of_slot, side_of_slot.data(), side_of_slot.size() * sizeof(int)))) return rc;
-    if ((rc = up(P->d_smoothed, sm_ents.data(), sm_ents.size() * sizeof(int4)))) return rc;
-    if ((rc = up(P->d_smooth_lanes, lanes.data(), lanes.size() * sizeof(int2)))) return rc;
+    Part parts[] = {
+        {&P->d_slot_entry, slot_entry.data(), slot_entry.size() * sizeof(int), 0},
+        {&P->d_entry_node, entry_node.data(), entry_node.size() * sizeof(int), 0},
+        {&P->d_entry_ops, entry_ops.data(), entry_ops.size() * sizeof(int2), 0},
+        {&P->d_ops, ops.data(), ops.size() * sizeof(Op), 0},
+        {&P->d_form_ops, form_ops.data(), form_ops.size() * sizeof(uint32_t), 0},
+        {&P->d_sym, sym.data(), P->nsym * sizeof(uint32_t), 0},
+        {&P->d_place_list, place_list.data(), place_list.size() * sizeof(lbm::NodeList), 0},
+        {&P->d_list_ops, list_ops.data(), list_ops.size() * sizeof(Op), 0},
+        {&P->d_slot_list, slot_list.data(), slot_list.size() * sizeof(lbm::NodeList), 0},
+        {&P->d_side_of_slot, side_of_slot.data(), side_of_slot.size() * sizeof(int), 0},
+        {&P->d_smoothed, sm_ents.data(), sm_ents.size() * sizeof(int4), 0},
+        {&P->d_smooth_lanes, lanes.data(), lanes.size() * sizeof(int2), 0},
+    };
+    size_t bytes = 0;
+    for (Part &t : parts) {
+        t.at = bytes;
+        bytes += (t.bytes + 255) / 256 * 256 + (t.bytes ? 0 : 256);
+    }
+    std::vector<unsigned char> packed(bytes);
+    for (const Part &t : parts)
+        if (t.bytes) memcpy(packed.data() + t.at, t.from, t.bytes);
+    if (P->d_tables.ensure(bytes)) return fail(LBM_ERR_HIP, "device allocation of %zu bytes failed", bytes);
+    HIPCHK(hipMemcpy(P->d_tables.p, packed.data(), bytes, hipMemcpyHostToDevice));
+    for (const Part &t : parts) t.to->p = static_cast<unsigned char *>(P->d_tables.p) + t.at;
     P->n_smooth_lanes = (int)lanes.size();
     P->uploaded = true;
     P->dev_used = true;
@@ -615,6 +673,8 @@ ProgView prog_view(const lbm_program *P) {
     v.slot_list = (const lbm::NodeList *)P->d_slot_list.p;
     v.list_ops = (const Op *)P->d_list_ops.p;
     v.form_ops = (const uint32_t *)P->d_form_ops.p;
+    v.sym = (const uint32_t *)P->d_sym.p;
+    v.nsym = P->nsym;
     v.maxops = P->maxops;
     v.side_of_slot = P->n_smoothed > 0 ? (const int *)P->d_side_of_slot.p : nullptr;
     v.side = P->n_smoothed > 0 ? (double *)P->d_side.p : nullptr;

@@ -213,45 +213,85 @@ __device__ __forceinline__ void settle(double *f) {
 // nodes holds one or two x-face nodes, which it all waits for, and with each lane deciding for
 // itself which operator and which face to run, the wavefront walked every branch of a decision
 // tree per operator, in four inlined copies, after three dependent memory round trips.  Here the
-// wavefront takes the forms its lanes have one after the other (nearly always one or two); a form's
-// words are uniform, so the choice of operator and face is scalar branches over one copy.  FP64 forward
-// steps: 200x400 heat sink 9.1 -> 7.6 us (5.9 without boundaries), 96x96x48 duct 36.7 -> 34 us, 128x128x64
-// 84 -> 78 us.
+// choice of operator and face is scalar branches over one copy.
+// 2D: the wavefront takes the forms its lanes have one after the other (nearly always one or two); the
+// words come with the node's list.  200x400 heat sink, FP64 forward step: 9.1 -> 7.6 us (5.9 without
+// boundaries); in the 3D manner, whose first word is a round trip of its own, 8.1 us.
+// 3D, where the program's operators fit 64 bits (ProgView::nsym; the forms are the general path): it
+// takes those its lanes have in an order that keeps every list's, each once for all lanes that have it.
+// A wavefront along an edge of the grid has up to six forms, and on grids of few workgroups the step
+// waits for it: 44x40x30 duct, forward / adjoint, 16.7 / 21.4 us by forms, 12.2 / 13.2 by operators (12.2 /
+// 13.8 with each lane deciding for itself); 113x36x43 19.7 / 22.6, 17.8 / 21.8 (18.7 / 21.0 so).
+// 96x96x48 forward 36.7 -> 34 us, 128x128x64 84 -> 78 us before the operators were merged, and
+// an evaluation of 300 + 300 steps there 52.4 -> 49.8 ms with it.
 template <class LA, class LB, class Smooth>
 __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, int n, double *a, double *b,
                                         Smooth &&smooth) {
     const NodeList &o = no.o;
-    unsigned long long todo = __ballot(o.form >= 0);
-    if (todo == 0) return;
-    do {
-        const int lead = __builtin_ctzll(todo);
-        const int form = __builtin_amdgcn_readlane(o.form, lead);
-        const int count = __builtin_amdgcn_readlane(o.count, lead);
-        uint64_t w0 = readlane64(o.w[0], lead), w1 = readlane64(o.w[1], lead);
-        const bool mine = o.form == form;
-        todo &= ~__ballot(mine);
-        for (int t = 0; t < count; ++t) {
-            uint32_t w = (uint32_t)w0 & 0xffffu;
+    const bool merged = LA::nd == 3 && pv.nsym > 0;
+    unsigned long long all = 0;   // merged: the operators left; else the lanes left
+    if (merged) {
+        for (unsigned long long left = __ballot(o.w[0] != 0); left;) {
+            all |= readlane64(o.w[0], __builtin_ctzll(left));
+            left = __ballot((o.w[0] & ~all) != 0);
+        }
+    } else {
+        all = __ballot(o.form >= 0);
+    }
+    if (all == 0) return;
+    auto symbol = [&](int bit) {
+        return ((const __attribute__((address_space(4))) uint32_t *)pv.sym)[bit];
+    };
+    uint32_t next = merged ? symbol(__builtin_ctzll(all)) : 0u;
+    int form = -1, count = 0, t = 0;
+    uint64_t w0 = 0, w1 = 0;
+    for (;;) {
+        uint32_t w;
+        unsigned long long before = 0;  // merged: the operators ahead of this one
+        bool mine;
+        if (merged) {
+            if (all == 0) break;
+            const int bit = __builtin_ctzll(all);
+            all &= all - 1;
+            w = next;
+            if (all) next = symbol(__builtin_ctzll(all));
+            before = (1ull << bit) - 1;
+            mine = o.w[0] >> bit & 1u;
+        } else {
+            if (t == count) {
+                if (all == 0) break;
+                const int lead = __builtin_ctzll(all);
+                form = __builtin_amdgcn_readlane(o.form, lead);
+                count = __builtin_amdgcn_readlane(o.count, lead);
+                w0 = readlane64(o.w[0], lead);
+                w1 = readlane64(o.w[1], lead);
+                all &= ~__ballot(o.form == form);
+                t = 0;
+            }
+            w = (uint32_t)w0 & 0xffffu;
             w0 = w0 >> 16 | w1 << 48;
             w1 >>= 16;
             if (t >= kWordOps)
                 w = (uint32_t)__builtin_amdgcn_readfirstlane((int)pv.form_ops[(size_t)form * pv.maxops + t]);
-            const OpWord op = op_fields(w);
-            if (mine) {
-                OpIn q{{o.vals.a[0], o.vals.a[1], o.vals.a[2], o.vals.a[3]}, {o.vals.b[0][0], o.vals.b[0][1]}};
-                if (op.src == kFromSecond) {
-                    q.b[0] = o.vals.b[1][0];
-                    q.b[1] = o.vals.b[1][1];
-                } else if (op.src == kFromList) {
-                    q = op_in(pv.list_ops[(size_t)o.list * pv.maxops + t]);
-                }
-                if (op.code == OP_SMOOTH) smooth((int)op.lat ^ pv.latswap);
-                else if (op.code != OP_NONE) apply_op<LA, LB>(op, q, a, b, pv, n, no.f);
-                settle<LA>(a);
-                settle<LB>(b);
-            }
+            ++t;
+            mine = o.form == form;
         }
-    } while (todo);
+        const OpWord op = op_fields(w);
+        if (mine) {
+            OpIn q{{o.vals.a[0], o.vals.a[1], o.vals.a[2], o.vals.a[3]}, {o.vals.b[0][0], o.vals.b[0][1]}};
+            if (op.src == kFromSecond) {
+                q.b[0] = o.vals.b[1][0];
+                q.b[1] = o.vals.b[1][1];
+            } else if (op.src == kFromList) {
+                const int at = merged ? __popcll(o.w[0] & before) : t - 1;
+                q = op_in(pv.list_ops[(size_t)o.list * pv.maxops + at]);
+            }
+            if (op.code == OP_SMOOTH) smooth((int)op.lat ^ pv.latswap);
+            else if (op.code != OP_NONE) apply_op<LA, LB>(op, q, a, b, pv, n, no.f);
+            settle<LA>(a);
+            settle<LB>(b);
+        }
+    }
 }
 
 // E_c of a shift, in FP64
