@@ -139,7 +139,7 @@ __device__ __forceinline__ uint4 keep(const uint4 &d, uint32_t bit) {
 // (m, n) computes 16 MT output channels of z layer n, 4 rows of 16 voxels.  Read from global memory
 // per tap, as it was, every input came through L1 27 times and each of those reads cost an address
 // and three bounds checks: at 96x96x48 and 16 -> 16 channels 58 us (109 TFLOP/s), bound by vector
-// instructions and L1; 25 us (249 TFLOP/s) now.  Here a K step of 32 costs one LDS read of 16 bytes
+// instructions and L1; 22 us (272 TFLOP/s) now.  Here a K step of 32 costs one LDS read of 16 bytes
 // per lane and row at an address the compiler knows up to a per-lane base, and its weights; all K
 // steps are unrolled.
 // A voxel's row in LDS is 16 bytes longer than its channels (CIN = 8: not), so that the 16 lanes of a
@@ -743,8 +743,8 @@ int launch_conv3(lbm_unet *N, const bf16_t *x, const bf16_t *w, const ConvOut &o
 }
 // The network's shapes.  The waves of a workgroup share its brick: across the output channels as far
 // as there are tiles of 16 (every one of them would otherwise stage the same voxels), the rest along z;
-// three tiles to a wave where their number is a multiple of three.  At 96x96x48: 16 -> 16 channels 25 us,
-// 16 -> 48 58 us, 48 -> 16 76 us, 32 -> 32 (48x48x24) 17 us.
+// three tiles to a wave where their number is a multiple of three.  At 96x96x48: 16 -> 16 channels 22 us,
+// 16 -> 48 56 us, 48 -> 16 52 us, 32 -> 32 (48x48x24) 11.5 us (25, 58, 76 and 17 with the weights loaded at their use).
 int launch_conv(lbm_unet *N, const bf16_t *x, int cin, int taps, const bf16_t *w, int kpad, const ConvOut &out,
                 const int *d) {
     const int V = d[0] * d[1] * d[2];
