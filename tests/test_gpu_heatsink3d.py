@@ -4,6 +4,8 @@ against the same boundary calls run one by one (each value-identical to the refe
 import numpy as np
 import pytest
 
+from _oracle import ref
+
 pytestmark = pytest.mark.gpu
 
 DIMS = dict(lx=14, ly=10, lz=9, plate=3)
@@ -152,6 +154,7 @@ def test_continuation_stages(ctx):
     hs.close()
 
 
+@pytest.mark.skipif(ref() is None, reason="reference harness not built")
 def test_design_loop_matches_oracle_loop(ctx):
     """The 3D MMA design loop (Heaviside projection with the design sub-box, base plate, the
     reference driver's (qf, beta) continuation advanced every iteration) against its CPU replica
