@@ -337,6 +337,10 @@ int lbm_program_bind_fields(lbm_program *prog, int set, const double *rho, const
 int lbm_program_num_field_sets(const lbm_program *prog);
 /* whether a program runs fused with a collide (1) or falls back to apply + collide (0) */
 int lbm_program_fusable(const lbm_program *prog);
+/* No reference counterpart.  How the program's last fused collide took its boundary operators: *symbols
+ * of them in the one order of the calls (0: more than 64, taken position by position), *longest the most
+ * at one node, *smoothing 0 none, 1 inside the pass, 2 after it.  LBM_ERR_STATE before a fused collide. */
+int lbm_program_fused_route(const lbm_program *prog, int *symbols, int *longest, int *smoothing);
 /* 1 when two programs record the same calls with the same values and field pointers */
 int lbm_program_equal(const lbm_program *a, const lbm_program *b);
 

@@ -161,6 +161,7 @@ def load():
         "lbm_program_bind_fields": [VP, I] + [VP] * 6,
         "lbm_program_num_field_sets": [VP],
         "lbm_program_fusable": [VP],
+        "lbm_program_fused_route": [VP] + [ctypes.POINTER(I)] * 3,
         "lbm_program_equal": [VP, VP],
         "lbm_graph_begin": [VP],
         "lbm_graph_end": [VP, ctypes.POINTER(VP)],

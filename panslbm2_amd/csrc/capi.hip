@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <limits>
 #include <cstdarg>
@@ -138,6 +139,7 @@ struct lbm_lattice {
 
 struct HostOp {
     int node;
+    int call;  // the recorded call it belongs to
     Op op;
 };
 
@@ -152,6 +154,7 @@ struct lbm_program {
     std::vector<HostOp> ops;
     std::vector<FieldSet> fsets;
     int seg = 0;
+    int calls = 0;           // boundary and SmoothCorner calls recorded
     bool ordered_ok = true;  // no operator on a lattice after its SmoothCorner
     // device tables
     bool uploaded = false;
@@ -161,13 +164,15 @@ struct lbm_program {
     struct Table {
         void *p = nullptr;
     };
-    Table d_slot_entry, d_entry_node, d_entry_ops, d_ops, d_form_ops, d_sym, d_list_ops, d_slot_list, d_place_list;
+    Table d_slot_entry, d_entry_node, d_entry_ops, d_ops, d_form_ops, d_list_ops, d_slot_list, d_place_list;
     unsigned shared_places = 0, slot_places = 0;  // ProgView::shared, by_slot
     DevBuf d_side;                      // smoothing after the pass, from side states
     Table d_side_of_slot, d_smoothed;
     Table d_smooth_lanes;               // 3D smoothing inside the pass (ProgView::smooth_lanes)
-    int nentry = 0, nslot = 0, maxops = 0, nsym = 0, n_smoothed = 0, smooth_stride = 1, n_smooth_lanes = 0;
+    std::vector<uint32_t> sym;          // ProgView::sym, one word to an element
+    int nentry = 0, nslot = 0, maxops = 0, n_smoothed = 0, smooth_stride = 1, n_smooth_lanes = 0;
     bool smooth_in_pass_ok = false;  // the smoothed nodes may be done by the fused pass's first workgroups
+    int route_smooth = -1;           // lbm_program_fused_route; -1: no fused collide yet
     bool owned_by_ctx = false;  // eager scratch program
     ~lbm_program() {
         d_tables.release();
@@ -290,6 +295,7 @@ int prog_record(lbm_program *P, lbm_lattice *L, uint8_t code, const int *sel, co
         if (fset < 0) return fset;
     }
     if (P->smoothed[slot] && code != lbm::OP_SMOOTH) P->ordered_ok = false;
+    const int call = P->calls++;
     int off = 0;
     for (int face = 0; face < 2 * L->nd; ++face) {
         int n = face_len(L, face);
@@ -298,6 +304,7 @@ int prog_record(lbm_program *P, lbm_lattice *L, uint8_t code, const int *sel, co
             if (!s) continue;
             HostOp h{};
             h.node = face_node(L, face, t);
+            h.call = call;
             h.op.code = code;
             h.op.face = (uint8_t)face;
             h.op.lat = (uint8_t)slot;
@@ -321,6 +328,7 @@ int prog_record_smooth(lbm_program *P, lbm_lattice *L) {
     for (const int4 &e : L->sm_edge) {
         HostOp h{};
         h.node = e.x;
+        h.call = P->calls;
         h.op.code = lbm::OP_SMOOTH;
         h.op.lat = (uint8_t)slot;
         h.op.seg = (uint8_t)P->seg;
@@ -329,11 +337,13 @@ int prog_record_smooth(lbm_program *P, lbm_lattice *L) {
     for (const int4 &e : L->sm_corner) {
         HostOp h{};
         h.node = e.x;
+        h.call = P->calls;
         h.op.code = lbm::OP_SMOOTH;
         h.op.lat = (uint8_t)slot;
         h.op.seg = (uint8_t)P->seg;
         P->ops.push_back(h);
     }
+    P->calls++;
     P->smoothed[slot] = 1;
     P->smooth_seg[slot] = P->seg;
     P->seg_closer.push_back(slot);
@@ -391,46 +401,27 @@ lbm::ListVals pack_list(const Op *o, int count, uint32_t *words) {
     return v;
 }
 
-// The distinct operators of the forms (form -> maxops words, OP_NONE after its own), at most 64, in an
-// order that keeps every form's, and per form which of them it has.  False: more of them, or no order.
-bool merge_forms(const std::vector<uint32_t> &form_ops, int maxops, std::vector<uint32_t> &sym,
-                 std::vector<uint64_t> &has) {
-    const size_t nform = maxops ? form_ops.size() / maxops : 0;
-    std::map<std::pair<uint32_t, int>, int> id;  // (word, how often before it in the form)
-    std::vector<uint32_t> word;
-    std::vector<uint64_t> before;  // bit b of before[c]: some form has b right ahead of c
-    std::vector<std::vector<int>> ids(nform);
-    for (size_t f = 0; f < nform; ++f) {
-        const uint32_t *w = &form_ops[f * maxops];
-        for (int t = 0; t < maxops; ++t) {
-            if (!w[t]) {  // past the form's end, or an operator that does nothing
-                if (std::any_of(w + t, w + maxops, [](uint32_t x) { return x != 0; })) return false;
-                break;
-            }
-            const auto at = id.emplace(std::make_pair(w[t], (int)std::count(w, w + t, w[t])), (int)word.size());
-            if (at.second) {
-                if (word.size() == 64) return false;
-                word.push_back(w[t]);
-                before.push_back(0);
-            }
-            if (t) before[at.first->second] |= uint64_t(1) << ids[f].back();
-            ids[f].push_back(at.first->second);
-        }
-    }
-    std::vector<int> place(word.size(), -1);
-    uint64_t done = 0;
+// The program's symbols (ProgView::sym) and per form which of them it has.  Every list is in the order of
+// the calls and, within a call, of the faces, so this order needs no search and never fails; two calls
+// that record the same word on different nodes have two symbols of it.  False: more than kSymbols.
+bool make_symbols(const std::vector<uint32_t> &form_ops, const std::vector<int> &form_calls, int maxops,
+                  std::vector<uint32_t> &sym, std::vector<uint64_t> &has) {
+    std::map<std::array<uint32_t, 3>, int> place;  // (call, face, word)
+    auto key = [&](size_t at) {
+        const uint32_t w = form_ops[at];
+        return std::array<uint32_t, 3>{(uint32_t)form_calls[at], lbm::op_fields(w).face, w};
+    };
+    for (size_t at = 0; at < form_ops.size(); ++at)
+        if (form_ops[at]) place.emplace(key(at), 0);
+    if (place.size() > (size_t)lbm::kSymbols) return false;
     sym.clear();
-    while (sym.size() < word.size()) {
-        size_t c = 0;
-        while (c < word.size() && ((done >> c & 1u) || (before[c] & ~done))) ++c;
-        if (c == word.size()) return false;  // two forms have two operators in opposite orders
-        done |= uint64_t(1) << c;
-        place[c] = (int)sym.size();
-        sym.push_back(word[c]);
+    for (auto &p : place) {
+        p.second = (int)sym.size();
+        sym.push_back(p.first[2]);
     }
-    has.assign(nform, 0);
-    for (size_t f = 0; f < nform; ++f)
-        for (int c : ids[f]) has[f] |= uint64_t(1) << place[c];
+    has.assign(maxops ? form_ops.size() / maxops : 0, 0);
+    for (size_t at = 0; at < form_ops.size(); ++at)
+        if (form_ops[at]) has[at / maxops] |= uint64_t(1) << place[key(at)];
     return true;
 }
 
@@ -449,13 +440,16 @@ int prog_upload(lbm_program *P) {
     std::vector<int> entry_node;
     std::vector<int2> entry_ops;
     std::vector<Op> ops;
+    std::vector<int> op_call;
     ops.reserve(order.size());
+    op_call.reserve(order.size());
     for (int t : order) {
         if (entry_node.empty() || entry_node.back() != P->ops[t].node) {
             entry_node.push_back(P->ops[t].node);
             entry_ops.push_back(make_int2((int)ops.size(), 0));
         }
         ops.push_back(P->ops[t].op);
+        op_call.push_back(P->ops[t].call);
         entry_ops.back().y++;
     }
     P->nentry = (int)entry_node.size();
@@ -469,16 +463,18 @@ int prog_upload(lbm_program *P) {
         slot_entry[s] = e;
     }
     // operator lists for the fused kernels: lists are stored once per distinct one (a face's nodes
-    // mostly share theirs), forms once per distinct sequence of operator words
+    // mostly share theirs), forms once per distinct sequence of operator words and calls
     int most = 0;
     for (const int2 &r : entry_ops) most = std::max(most, r.y);
     P->maxops = most;
     std::vector<Op> list_ops;
     std::vector<uint32_t> form_ops;
+    std::vector<int> form_calls;
     std::vector<lbm::NodeList> slot_list(P->nslot, lbm::NodeList{-1, -1, 0, 0, {0, 0}, {}});
     std::map<std::string, int> form_of, list_of;
     std::vector<Op> one(P->maxops);
     std::vector<uint32_t> words(P->maxops);
+    std::vector<int> calls(P->maxops);
     auto key_of = [](const auto &v) { return std::string(reinterpret_cast<const char *>(v.data()), v.size() * sizeof v[0]); };
     int last = -1;  // the slot before with operators: a face's nodes follow each other and mostly share theirs
     for (int s = 0; s < P->nslot; ++s) {
@@ -488,28 +484,35 @@ int prog_upload(lbm_program *P) {
         last = s;
         if (before >= 0) {
             const int2 x = entry_ops[slot_entry[before]], y = entry_ops[e];
-            if (x.y == y.y && !memcmp(&ops[x.x], &ops[y.x], y.y * sizeof(Op))) {
+            if (x.y == y.y && !memcmp(&ops[x.x], &ops[y.x], y.y * sizeof(Op)) &&
+                !memcmp(&op_call[x.x], &op_call[y.x], y.y * sizeof(int))) {
                 slot_list[s] = slot_list[before];
                 continue;
             }
         }
         std::fill(one.begin(), one.end(), Op{});
         std::fill(words.begin(), words.end(), 0u);
+        std::fill(calls.begin(), calls.end(), -1);
         const int count = entry_ops[e].y;
-        for (int t = 0; t < count; ++t) one[t] = ops[entry_ops[e].x + t];
+        for (int t = 0; t < count; ++t) {
+            one[t] = ops[entry_ops[e].x + t];
+            calls[t] = op_call[entry_ops[e].x + t];
+        }
         const lbm::ListVals vals = pack_list(one.data(), count, words.data());
         auto l = list_of.emplace(key_of(one), (int)list_of.size());
         if (l.second) list_ops.insert(list_ops.end(), one.begin(), one.end());
-        auto f = form_of.emplace(key_of(words), (int)form_of.size());
-        if (f.second) form_ops.insert(form_ops.end(), words.begin(), words.end());
+        auto f = form_of.emplace(key_of(words) + key_of(calls), (int)form_of.size());
+        if (f.second) {
+            form_ops.insert(form_ops.end(), words.begin(), words.end());
+            form_calls.insert(form_calls.end(), calls.begin(), calls.end());
+        }
         lbm::NodeList so{l.first->second, f.first->second, count, 0, {0, 0}, vals};
         for (int t = 0; t < std::min(count, lbm::kWordOps); ++t) so.w[t / 4] |= (uint64_t)words[t] << (16 * (t % 4));
         slot_list[s] = so;
     }
-    std::vector<uint32_t> sym;
     std::vector<uint64_t> has;
-    P->nsym = L->nd == 3 && merge_forms(form_ops, P->maxops, sym, has) ? (int)sym.size() : 0;  // see run_ops
-    if (P->nsym > 0)
+    if (!make_symbols(form_ops, form_calls, P->maxops, P->sym, has)) P->sym.clear();  // see run_ops
+    if (!P->sym.empty())
         for (lbm::NodeList &so : slot_list)
             if (so.form >= 0) so.w[0] = has[so.form];
     // places whose nodes share one list (or have none), and places that have several
@@ -527,7 +530,7 @@ int prog_upload(lbm_program *P) {
                     seen |= 1u << at;
                     place_list[at] = slot_list[s];
                     if (slot_list[s].list >= 0) P->shared_places |= 1u << at;
-                } else if (slot_list[s].list != place_list[at].list) {
+                } else if (slot_list[s].list != place_list[at].list || slot_list[s].form != place_list[at].form) {
                     P->slot_places |= 1u << at;
                 }
             }
@@ -636,7 +639,6 @@ int prog_upload(lbm_program *P) {
         {&P->d_entry_ops, entry_ops.data(), entry_ops.size() * sizeof(int2), 0},
         {&P->d_ops, ops.data(), ops.size() * sizeof(Op), 0},
         {&P->d_form_ops, form_ops.data(), form_ops.size() * sizeof(uint32_t), 0},
-        {&P->d_sym, sym.data(), P->nsym * sizeof(uint32_t), 0},
         {&P->d_place_list, place_list.data(), place_list.size() * sizeof(lbm::NodeList), 0},
         {&P->d_list_ops, list_ops.data(), list_ops.size() * sizeof(Op), 0},
         {&P->d_slot_list, slot_list.data(), slot_list.size() * sizeof(lbm::NodeList), 0},
@@ -673,8 +675,8 @@ ProgView prog_view(const lbm_program *P) {
     v.slot_list = (const lbm::NodeList *)P->d_slot_list.p;
     v.list_ops = (const Op *)P->d_list_ops.p;
     v.form_ops = (const uint32_t *)P->d_form_ops.p;
-    v.sym = (const uint32_t *)P->d_sym.p;
-    v.nsym = P->nsym;
+    v.nsym = (int)P->sym.size();
+    for (int k = 0; k < v.nsym; ++k) v.sym[k >> 1] |= P->sym[k] << (k & 1) * 16;
     v.maxops = P->maxops;
     v.side_of_slot = P->n_smoothed > 0 ? (const int *)P->d_side_of_slot.p : nullptr;
     v.side = P->n_smoothed > 0 ? (double *)P->d_side.p : nullptr;
@@ -846,6 +848,7 @@ int collide_call(lbm_program *P, lbm_lattice *p, lbm_lattice *q, std::initialize
         cl.n_smoothed = 0;
     }
     cl.any_smooth = (P->smoothed[0] || P->smoothed[1]) ? 1 : 0;
+    P->route_smooth = !cl.any_smooth ? 0 : (cl.n_smoothed > 0 ? 2 : 1);
     if (sink) {
         if (cl.n_smoothed > 0)
             return fail(LBM_ERR_UNSUPPORTED, "a batched collide cannot run the smoothed nodes' kernel after its pass");
@@ -2176,6 +2179,14 @@ int lbm_program_equal(const lbm_program *a, const lbm_program *b) {
         if (x.node != y.node || memcmp(&x.op, &y.op, sizeof(Op))) return 0;
     }
     return 1;
+}
+int lbm_program_fused_route(const lbm_program *P, int *symbols, int *longest, int *smoothing) {
+    if (!P || !symbols || !longest || !smoothing) return fail(LBM_ERR_ARG, "null argument");
+    if (P->route_smooth < 0) return fail(LBM_ERR_STATE, "the program has run in no fused collide");
+    *symbols = (int)P->sym.size();
+    *longest = P->maxops;
+    *smoothing = P->route_smooth;
+    return LBM_OK;
 }
 int lbm_program_fusable(const lbm_program *P) { return P ? (P->ordered_ok ? 1 : 0) : fail(LBM_ERR_ARG, "null"); }
 

@@ -158,7 +158,7 @@ template <class LA, class LB>
 __device__ __forceinline__ void apply_op(const OpWord &op, const OpIn &q, double *a, double *b, const ProgView &pv,
                                          int n, const NodeFields &pre) {
     NodeFields s = pre;
-    if (!((pv.fmerged >> op.fset) & 1u)) s = load_fields(field_set(pv, (int)op.fset), n);
+    if (__builtin_expect(!((pv.fmerged >> op.fset) & 1u), 0)) s = load_fields(field_set(pv, (int)op.fset), n);
     s.has_diff = (pv.has_diff >> op.fset) & 1u;
     if (((int)op.lat ^ pv.latswap) == 0) apply_on<LA, LB>(op, q, a, b, s);
     else if constexpr (LB::nc > 0) apply_on<LB, LA>(op, q, b, a, s);
@@ -206,90 +206,81 @@ __device__ __forceinline__ void settle(double *f) {
 #pragma unroll
     for (int c = 0; c < L::nc; ++c) asm volatile("" : "+v"(f[c]));
 }
+struct NoSmooth {};  // SMOOTH operators do nothing
 // Run a node's operators in record order; smooth(kernel lattice 0 / 1) stands for a SMOOTH operator.
-// Called with the boundary lanes (and any others: form -1) active.
+// Called with the boundary lanes (and any others: no operators) active.
 //
-// What bounds it is latency and instruction fetch, not arithmetic: a wavefront of 64 consecutive
-// nodes holds one or two x-face nodes, which it all waits for, and with each lane deciding for
-// itself which operator and which face to run, the wavefront walked every branch of a decision
-// tree per operator, in four inlined copies, after three dependent memory round trips.  Here the
-// choice of operator and face is scalar branches over one copy.
-// 2D: the wavefront takes the forms its lanes have one after the other (nearly always one or two); the
-// words come with the node's list.  200x400 heat sink, FP64 forward step: 9.1 -> 7.6 us (5.9 without
-// boundaries); in the 3D manner, whose first word is a round trip of its own, 8.1 us.
-// 3D, where the program's operators fit 64 bits (ProgView::nsym; the forms are the general path): it
-// takes those its lanes have in an order that keeps every list's, each once for all lanes that have it.
-// A wavefront along an edge of the grid has up to six forms, and on grids of few workgroups the step
-// waits for it: 44x40x30 duct, forward / adjoint, 16.7 / 21.4 us by forms, 12.2 / 13.2 by operators (12.2 /
-// 13.8 with each lane deciding for itself); 113x36x43 19.7 / 22.6, 17.8 / 21.8 (18.7 / 21.0 so).
-// 96x96x48 forward 36.7 -> 34 us, 128x128x64 84 -> 78 us before the operators were merged, and
-// an evaluation of 300 + 300 steps there 52.4 -> 49.8 ms with it.
-template <class LA, class LB, class Smooth>
+// What bounds it is latency, not throughput: a wavefront of 64 consecutive nodes holds one or two
+// x-face nodes, on small grids the step waits for the wavefront with the most operators, and each of
+// them is a chain of branches, instruction fetches and divisions of some 0.15 us.  So the wavefront
+// takes the program's symbols that its lanes have one after the other, each once for all lanes that
+// have it, with scalar branches over one copy of the operators.  FP64 step, us, against each list's
+// sequence of words run by itself (and against each lane deciding for itself): 200x400 D2Q9 + D2Q5 heat
+// sink 7.7 (8.4; 7.8), smoothed 7.7 (7.9; 9.1), 101x101 6.3 (7.4; 6.8), 200x400 with six calls whose masks
+// are drawn per node 12.5 (91; 13.2); ducts forward / adjoint 44x40x30 11.0 / 11.9 (11.4 / 12.7; 11.1 /
+// 12.7), 113x36x43 17.8 / 21.1 (17.5 / 21.7; 18.0 / 20.9), 96x96x48 33.5 / 38.9 (34.2 / 39.8; 37.4 / 43.6).
+// Slower than each lane deciding for itself: 200x400 with two calls on all four faces 7.5 (8.2; 7.2) and
+// 101x101 with both bounce types, T and Q alternating along the walls 7.8 (9.7; 6.4).
+// More than kSymbols symbols (11 calls that each reach six faces): position by position of the lists, at
+// each the words that the lanes have, each once.
+template <class LA, class LB, class Smooth = NoSmooth>
 __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, int n, double *a, double *b,
-                                        Smooth &&smooth) {
+                                        Smooth &&smooth = Smooth{}) {
     const NodeList &o = no.o;
-    const bool merged = LA::nd == 3 && pv.nsym > 0;
-    unsigned long long all = 0;   // merged: the operators left; else the lanes left
+    const bool merged = pv.nsym > 0;
+    unsigned long long all = 0;  // merged: the symbols left; else the lanes whose operator at position t is left
+    int t = 0;
+    uint32_t word = (uint32_t)o.w[0] & 0xffffu, next = 0;
+    uint64_t w0 = o.w[0], w1 = o.w[1];
     if (merged) {
         for (unsigned long long left = __ballot(o.w[0] != 0); left;) {
             all |= readlane64(o.w[0], __builtin_ctzll(left));
             left = __ballot((o.w[0] & ~all) != 0);
         }
+        if (all) next = pv.sym[__builtin_ctzll(all) >> 1];
     } else {
-        all = __ballot(o.form >= 0);
+        all = __ballot(o.count > 0);
     }
-    if (all == 0) return;
-    auto symbol = [&](int bit) {
-        return ((const __attribute__((address_space(4))) uint32_t *)pv.sym)[bit];
-    };
-    uint32_t next = merged ? symbol(__builtin_ctzll(all)) : 0u;
-    int form = -1, count = 0, t = 0;
-    uint64_t w0 = 0, w1 = 0;
-    for (;;) {
+    while (all) {
         uint32_t w;
-        unsigned long long before = 0;  // merged: the operators ahead of this one
+        int bit = 0;
         bool mine;
         if (merged) {
-            if (all == 0) break;
-            const int bit = __builtin_ctzll(all);
+            bit = __builtin_ctzll(all);
             all &= all - 1;
-            w = next;
-            if (all) next = symbol(__builtin_ctzll(all));
-            before = (1ull << bit) - 1;
+            w = next >> (bit & 1) * 16;  // loaded one operator ahead
+            next = pv.sym[(all ? __builtin_ctzll(all) : bit) >> 1];
             mine = o.w[0] >> bit & 1u;
         } else {
-            if (t == count) {
-                if (all == 0) break;
-                const int lead = __builtin_ctzll(all);
-                form = __builtin_amdgcn_readlane(o.form, lead);
-                count = __builtin_amdgcn_readlane(o.count, lead);
-                w0 = readlane64(o.w[0], lead);
-                w1 = readlane64(o.w[1], lead);
-                all &= ~__ballot(o.form == form);
-                t = 0;
-            }
-            w = (uint32_t)w0 & 0xffffu;
-            w0 = w0 >> 16 | w1 << 48;
-            w1 >>= 16;
-            if (t >= kWordOps)
-                w = (uint32_t)__builtin_amdgcn_readfirstlane((int)pv.form_ops[(size_t)form * pv.maxops + t]);
-            ++t;
-            mine = o.form == form;
+            w = (uint32_t)__builtin_amdgcn_readlane((int)word, __builtin_ctzll(all));
+            mine = t < o.count && word == w;
+            all &= ~__ballot(mine);
         }
         const OpWord op = op_fields(w);
         if (mine) {
-            OpIn q{{o.vals.a[0], o.vals.a[1], o.vals.a[2], o.vals.a[3]}, {o.vals.b[0][0], o.vals.b[0][1]}};
-            if (op.src == kFromSecond) {
-                q.b[0] = o.vals.b[1][0];
-                q.b[1] = o.vals.b[1][1];
-            } else if (op.src == kFromList) {
-                const int at = merged ? __popcll(o.w[0] & before) : t - 1;
+            const bool second = op.src == kFromSecond;
+            OpIn q{{o.vals.a[0], o.vals.a[1], o.vals.a[2], o.vals.a[3]},
+                   {second ? o.vals.b[1][0] : o.vals.b[0][0], second ? o.vals.b[1][1] : o.vals.b[0][1]}};
+            if (__builtin_expect(op.src == kFromList, 0)) {
+                const int at = merged ? __popcll(o.w[0] & ((1ull << bit) - 1)) : t;
                 q = op_in(pv.list_ops[(size_t)o.list * pv.maxops + at]);
             }
-            if (op.code == OP_SMOOTH) smooth((int)op.lat ^ pv.latswap);
-            else if (op.code != OP_NONE) apply_op<LA, LB>(op, q, a, b, pv, n, no.f);
+            if constexpr (std::is_same_v<std::decay_t<Smooth>, NoSmooth>) {
+                apply_op<LA, LB>(op, q, a, b, pv, n, no.f);
+            } else {
+                if (op.code == OP_SMOOTH) smooth((int)op.lat ^ pv.latswap);
+                else apply_op<LA, LB>(op, q, a, b, pv, n, no.f);
+            }
             settle<LA>(a);
             settle<LB>(b);
+        }
+        if (!merged && all == 0) {
+            ++t;
+            all = __ballot(t < o.count);
+            w0 = w0 >> 16 | w1 << 48;
+            w1 >>= 16;
+            word = (uint32_t)w0 & 0xffffu;
+            if (t >= kWordOps && t < o.count) word = pv.form_ops[(size_t)o.form * pv.maxops + t];
         }
     }
 }
@@ -486,7 +477,7 @@ __device__ __forceinline__ void node_state(const double *sa, const double *sb, c
     coords(n, g, i, j, k);
     const NodeOps no = ops_of_node(pv, g, i, j, k, n, LA::nd, ops);
     pull_pair<LA, LB>(sa, sb, g, i, j, k, n, pv, a, b, Enc{}, Enc{});
-    run_ops<LA, LB>(pv, no, n, a, b, [](int) {});
+    run_ops<LA, LB>(pv, no, n, a, b);
 }
 template <class LA, class LB, class S, std::enable_if_t<!std::is_same_v<S, double>, int> = 0>
 __device__ __forceinline__ void node_state(const S *sa, const S *sb, const Grid &g, const ProgView &pv, int n,
@@ -500,7 +491,7 @@ __device__ __forceinline__ void node_state(const S *sa, const S *sb, const Grid 
         double xa[LA::nc], xb[LB::nc > 0 ? LB::nc : 1];
         dev_to_f64<LA>(a, xa, ea, oa);
         if constexpr (LB::nc > 0) dev_to_f64<LB>(b, xb, eb, ob);
-        run_ops<LA, LB>(pv, no, n, xa, xb, [](int) {});
+        run_ops<LA, LB>(pv, no, n, xa, xb);
         f64_to_dev<LA>(xa, a, ea, oa);
         if constexpr (LB::nc > 0) f64_to_dev<LB>(xb, b, eb, ob);
     }

@@ -55,7 +55,8 @@ constexpr size_t kXcdRemapMaxBytes = size_t(640) << 20;  // population bytes rea
 // (OpIn: a for the Navier-Stokes operators, b for the advection-diffusion ones), so that a boundary
 // node learns all it has to do with one load and has every operand with the next ones.
 enum OpSource : uint32_t { kFromFirst = 0, kFromSecond = 1, kFromList = 2 };
-constexpr int kWordOps = 8;  // operators in a NodeList without ProgView::sym; a longer list's further words sit in form_ops
+constexpr int kWordOps = 8;  // operators in a NodeList of a program without symbols; a longer list's further words sit in form_ops
+constexpr int kSymbols = 64;  // most symbols of a program (ProgView::sym)
 __host__ __device__ constexpr uint32_t op_word(uint32_t code, uint32_t face, uint32_t lat, uint32_t fset, uint32_t arg,
                                                uint32_t src) {
     return code | face << 4 | lat << 7 | fset << 8 | arg << 10 | src << 12;
@@ -80,10 +81,10 @@ struct alignas(16) ListVals {  // a list's values: one a, two b
 };
 
 // A boundary node's operators and their values.  Lists that differ in their values only share a form
-// (the sequence of words): a wavefront runs one form at a time on all lanes that have it.
+// (the sequence of words and of the calls that recorded them).
 struct alignas(16) NodeList {
     int list, form, count, pad;  // list, form: -1 without operators
-    uint64_t w[2];               // w[0]: which of ProgView::sym; without sym: the first kWordOps operators, 16 bits each
+    uint64_t w[2];               // w[0]: which of ProgView::sym; without symbols: the first kWordOps operators, 16 bits each
     ListVals vals;
 };
 // The nodes of a grid fall into 27 places: on the low side, between or on the high side of each axis
@@ -108,9 +109,11 @@ struct ProgView {
     unsigned shared, by_slot;    // bit p: place p's nodes share a list of operators / have several lists
     const Op *list_ops;         // list -> maxops operators (for values outside a NodeList)
     const uint32_t *form_ops;   // form -> maxops words
-    // The program's distinct operators (words; a list with one twice has two of them), at most 64, in an
-    // order that every list's operators are in.  nsym 0: 2D, or there are more, or no such order.
-    const uint32_t *sym;
+    // The program's symbols: its distinct (call, face, word), two words to an element, in the order of
+    // the calls and their faces, which every list is in.  They ride in the kernel's arguments: from memory
+    // their first use was a round trip of its own (101x101 D2Q9 + D2Q5 step 6.5 us against 6.3).
+    // nsym 0: more than kSymbols.
+    uint32_t sym[kSymbols / 2];
     int nsym;
     int maxops;             // operators per list (0: no operators)
     int nentry;

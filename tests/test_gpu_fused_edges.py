@@ -241,3 +241,165 @@ def test_duct_coefficients_match_numpy(ctx, dims, box, plate, have_prev):
             "dads": -am / (ly - 1.0) * qf * (1.0 + qf) / (s + qf) ** 2,
             "diff": dso + (dfl - dso) * s * (1.0 + qg) / (s + qg), "dkds": (dfl - dso) * qg * (1.0 + qg) / (s + qg) ** 2}
     _same({m: dev[m].download() for m in want}, want)
+
+
+def _route(b):
+    """(symbols, most operators at a node, smoothing) of the backend's last fused collide."""
+    import panslbm2_amd as pa
+
+    v = [ctypes.c_int(-9) for _ in range(3)]
+    pa.check(b.L.lbm_program_fused_route(b._pending, *(ctypes.byref(x) for x in v)))
+    return tuple(x.value for x in v)
+
+
+def test_route_before_a_fused_collide_is_an_error(ctx):
+    import panslbm2_amd as pa
+
+    p = pa.Lattice(ctx, pa.D2Q9, 5, 4, 1)
+    prog, v = ctypes.c_void_p(), ctypes.c_int()
+    pa.check(ctx.lib.lbm_record_begin(ctx.h))
+    pa.check(ctx.lib.lbm_stream(p.h))
+    pa.check(ctx.lib.lbm_record_end(ctx.h, ctypes.byref(prog)))
+    r = [ctypes.byref(v)] * 3
+    assert ctx.lib.lbm_program_fused_route(prog, *r) < 0
+    assert ctx.lib.lbm_program_fused_route(None, *r) < 0
+    ctx.lib.lbm_program_destroy(prog)
+
+
+@pytest.mark.parametrize("smooth,own", [("", False), ("fg", False), ("fg", True)], ids=["plain", "in-pass", "after-pass"])
+@pytest.mark.parametrize("pair", ["q9q5", "q15q7"])
+def test_route_of_a_program_in_one_order(ctx, pair, smooth, own):
+    """Two calls on every face: a symbol per call and face, and one per smoothed lattice; a corner of the
+    grid has both calls on each of its faces.  Smoothed nodes inside the pass, or after it where an
+    operator reads what the collide writes."""
+    from gpu_backend import FusedGpuBackend
+
+    kinds = tuple(getattr(_oracle, n) for n in PAIRS[pair])
+    nd = ND[kinds[0]]
+    dims = (9, 7, 1) if nd == 2 else (6, 5, 4)
+    print("route", pair, smooth, own, flush=True)
+
+    def run(b):
+        def ops(p, q, z, N, rng):
+            b.bc(p, np.ones(N, np.int32))
+            u = ("ux", "uy", z("uz")) if own else ("vx", "vy", z("vz"))
+            b.ad_set_t(q, np.ones(N, np.int32), np.full(N, 1.2), *u)
+            for h, name in ((p, "f"), (q, "g")):
+                if name in smooth:
+                    b.smooth(h)
+
+        return _run(b, kinds, dims, 5, False, 2, ops)
+
+    fb = FusedGpuBackend(ctx)
+    got = run(fb)
+    assert _route(fb) == (4 * nd + len(smooth), 2 * nd + len(smooth), 0 if not smooth else (2 if own else 1))
+    _same(got, run(OracleBackend()))
+
+
+@pytest.mark.parametrize("calls", [11, 18], ids=["11", "18"])
+@pytest.mark.parametrize("pair", ["q9q5", "q15q7"])
+def test_route_of_a_program_position_by_position(ctx, pair, calls):
+    """Programs around the limit of 64 symbols, one per call, face and type that some node of the face has:
+    `calls` bounce-back calls with types drawn per node, both of them in every other call.  Beyond it the operators are taken
+    position by position, here with lists of up to 54, most of them past the eight in a list's header."""
+    from gpu_backend import FusedGpuBackend
+
+    kinds = tuple(getattr(_oracle, n) for n in PAIRS[pair])
+    nd = ND[kinds[0]]
+    dims = (131, 9, 1) if nd == 2 else (65, 5, 7)
+    print("route", pair, calls, flush=True)
+
+    n = np.arange(dims[0] * dims[1] * dims[2])
+    at = (n % dims[0], n // dims[0] % dims[1], n // (dims[0] * dims[1]))
+    faces = [at[f // 2] == (f % 2) * (dims[f // 2] - 1) for f in range(2 * nd)]
+    symbols = set()
+
+    def run(b):
+        def ops(p, q, z, N, rng):
+            for c in range(calls):
+                t = rng.integers(0, 3, N) if c % 2 else rng.integers(0, 2, N)
+                t[:] = np.where(np.arange(N) == 0, 1, t)  # the longest list is the first corner's
+                symbols.update((c, f, x) for f, on in enumerate(faces) for x in set(t[on]) if x)
+                b.bc(q if c % 3 else p, t.astype(np.int32))
+
+        return _run(b, kinds, dims, 5, False, 2, ops)
+
+    fb = FusedGpuBackend(ctx)
+    got = run(fb)
+    assert (len(symbols) > 64) == ((calls, nd) != (11, 2))
+    assert _route(fb) == (len(symbols) if len(symbols) <= 64 else 0, calls * nd, 0)
+    _same(got, run(OracleBackend()))
+
+
+@pytest.mark.parametrize("dims", [(200, 400, 1), (65, 49, 33)], ids=["2d", "3d"])
+def test_mixed_operator_lists_cost_little_more_than_uniform_ones(ctx, dims):
+    """A step waits for the wavefront with the most operators.  With masks drawn per node a wavefront of
+    64 wall nodes has up to 64 different lists, of six calls (24 or 36 symbols) together; with the same
+    two calls everywhere it has 2 or 3 of 4 to 6 symbols.  A wavefront runs each symbol once, so the
+    ratio of the step times is below that of the symbols, 24 / 4 = 6, and of the operators' share in a
+    step, of which about half is not operators: 3."""
+    import time
+
+    import panslbm2_amd as pa
+    from panslbm2_amd import D, check, hptr
+
+    L, (lx, ly, lz) = ctx.lib, dims
+    N, d3 = lx * ly * lz, lz > 1
+    kinds = (pa.D3Q15, pa.D3Q7) if d3 else (pa.D2Q9, pa.D2Q5)
+    rng = np.random.default_rng(3)
+
+    def arr(v):
+        return ctx.array((N,), data=np.full(N, v))
+
+    one, zero, alpha, diff = arr(1.0), arr(0.0), arr(0.1), arr(0.1)
+    out = [arr(0.0) for _ in range(8)]
+    uz = zero.ptr if d3 else None
+
+    def face(a, dt=np.float64):
+        return pa.to_face(kinds[0], lx, ly, lz, np.broadcast_to(a, (N,)), dt)
+
+    def step_us(masks):
+        p, q = (pa.Lattice(ctx, k, lx, ly, lz) for k in kinds)
+        m = [face(a, np.int32) for a in masks]
+        u, r, z = face(0.01), face(1.0), face(0.0)
+        check(L.lbm_record_begin(ctx.h))
+        for h in (p, q):
+            check(L.lbm_stream(h.h))
+        check(L.lbm_bc(p.h, hptr(m[0])))
+        check(L.lbm_ns_set_u(p.h, hptr(m[1]), hptr(u), hptr(z), hptr(z)))
+        check(L.lbm_ns_set_rho(p.h, hptr(m[2]), hptr(r), hptr(z), hptr(z)))
+        check(L.lbm_ad_set_t(q.h, hptr(m[3]), hptr(u), zero.ptr, zero.ptr, uz))
+        check(L.lbm_ad_set_q(q.h, hptr(m[4]), hptr(z), zero.ptr, zero.ptr, uz, diff.ptr, D(0)))
+        check(L.lbm_bc(q.h, hptr(m[5])))
+        prog, g = ctypes.c_void_p(), ctypes.c_void_p()
+        check(L.lbm_record_end(ctx.h, ctypes.byref(prog)))
+        check(L.lbm_ns_initial_condition(p.h, one.ptr, zero.ptr, zero.ptr, uz))
+        check(L.lbm_ad_initial_condition(q.h, zero.ptr, zero.ptr, zero.ptr, uz))
+
+        def step():
+            check(L.lbm_ad_macro_brinkman_collide_force_convection_p(
+                prog, p.h, *(x.ptr for x in out[:3]), out[3].ptr, alpha.ptr, D(0.1), q.h,
+                *(x.ptr for x in out[4:7]), out[7].ptr, diff.ptr, 0, None, None))
+
+        step()
+        step()
+        check(L.lbm_graph_begin(ctx.h))
+        for _ in range(100):
+            step()
+        check(L.lbm_graph_end(ctx.h, ctypes.byref(g)))
+        best = np.inf
+        for _ in range(6):
+            ctx.sync()
+            t0 = time.perf_counter()
+            check(L.lbm_graph_launch(g))
+            ctx.sync()
+            best = min(best, time.perf_counter() - t0)
+        L.lbm_graph_destroy(g)
+        L.lbm_program_destroy(prog)
+        return 1e4 * best
+
+    uniform = step_us([np.ones(N, np.int32)] + [np.zeros(N, np.int32)] * 2 + [np.ones(N, np.int32)] +
+                      [np.zeros(N, np.int32)] * 2)
+    mixed = step_us([rng.integers(0, top + 1, N).astype(np.int32) for top in (2, 1, 1, 1, 1, 2)])
+    print("mixed lists", dims, "%.1f us, uniform %.1f us" % (mixed, uniform), flush=True)
+    assert mixed <= 3.0 * uniform
