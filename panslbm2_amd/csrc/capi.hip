@@ -466,11 +466,14 @@ int prog_upload(lbm_program *P) {
     // mostly share theirs), forms once per distinct sequence of operator words and calls
     int most = 0;
     for (const int2 &r : entry_ops) most = std::max(most, r.y);
+    if (most >= 1 << 24) return fail(LBM_ERR_UNSUPPORTED, "more than 2^24 operators at one node");
     P->maxops = most;
     std::vector<Op> list_ops;
     std::vector<uint32_t> form_ops;
     std::vector<int> form_calls;
-    std::vector<lbm::NodeList> slot_list(P->nslot, lbm::NodeList{-1, -1, 0, 0, {0, 0}, {}});
+    const lbm::NodeList no_list{~uint64_t(0), 0, {0, 0}, {}};
+    std::vector<lbm::NodeList> slot_list(P->nslot, no_list);
+    std::vector<int> slot_form(P->nslot, -1);
     std::map<std::string, int> form_of, list_of;
     std::vector<Op> one(P->maxops);
     std::vector<uint32_t> words(P->maxops);
@@ -487,6 +490,7 @@ int prog_upload(lbm_program *P) {
             if (x.y == y.y && !memcmp(&ops[x.x], &ops[y.x], y.y * sizeof(Op)) &&
                 !memcmp(&op_call[x.x], &op_call[y.x], y.y * sizeof(int))) {
                 slot_list[s] = slot_list[before];
+                slot_form[s] = slot_form[before];
                 continue;
             }
         }
@@ -506,17 +510,19 @@ int prog_upload(lbm_program *P) {
             form_ops.insert(form_ops.end(), words.begin(), words.end());
             form_calls.insert(form_calls.end(), calls.begin(), calls.end());
         }
-        lbm::NodeList so{l.first->second, f.first->second, count, 0, {0, 0}, vals};
+        slot_form[s] = f.first->second;
+        lbm::NodeList so{(uint64_t)l.first->second * P->maxops,
+                         (uint64_t)f.first->second * P->maxops << 24 | (uint64_t)count, {0, 0}, vals};
         for (int t = 0; t < std::min(count, lbm::kWordOps); ++t) so.w[t / 4] |= (uint64_t)words[t] << (16 * (t % 4));
         slot_list[s] = so;
     }
     std::vector<uint64_t> has;
     if (!make_symbols(form_ops, form_calls, P->maxops, P->sym, has)) P->sym.clear();  // see run_ops
     if (!P->sym.empty())
-        for (lbm::NodeList &so : slot_list)
-            if (so.form >= 0) so.w[0] = has[so.form];
+        for (int s = 0; s < P->nslot; ++s)
+            if (slot_form[s] >= 0) slot_list[s].w[0] = has[slot_form[s]];
     // places whose nodes share one list (or have none), and places that have several
-    std::vector<lbm::NodeList> place_list(lbm::kPlaces, lbm::NodeList{-1, -1, 0, 0, {0, 0}, {}});
+    std::vector<lbm::NodeList> place_list(lbm::kPlaces, no_list);
     unsigned seen = 0;
     P->shared_places = P->slot_places = 0;
     for (int k = 0; k < L->lz; ++k)
@@ -529,8 +535,9 @@ int prog_upload(lbm_program *P) {
                 if (!(seen >> at & 1u)) {
                     seen |= 1u << at;
                     place_list[at] = slot_list[s];
-                    if (slot_list[s].list >= 0) P->shared_places |= 1u << at;
-                } else if (slot_list[s].list != place_list[at].list || slot_list[s].form != place_list[at].form) {
+                    if (slot_form[s] >= 0) P->shared_places |= 1u << at;
+                } else if (slot_list[s].list != place_list[at].list ||
+                           slot_list[s].form_count != place_list[at].form_count) {
                     P->slot_places |= 1u << at;
                 }
             }
@@ -677,7 +684,6 @@ ProgView prog_view(const lbm_program *P) {
     v.form_ops = (const uint32_t *)P->d_form_ops.p;
     v.nsym = (int)P->sym.size();
     for (int k = 0; k < v.nsym; ++k) v.sym[k >> 1] |= P->sym[k] << (k & 1) * 16;
-    v.maxops = P->maxops;
     v.side_of_slot = P->n_smoothed > 0 ? (const int *)P->d_side_of_slot.p : nullptr;
     v.side = P->n_smoothed > 0 ? (double *)P->d_side.p : nullptr;
     v.nentry = P->nentry;

@@ -163,33 +163,45 @@ __device__ __forceinline__ void apply_op(const OpWord &op, const OpIn &q, double
     if (((int)op.lat ^ pv.latswap) == 0) apply_on<LA, LB>(op, q, a, b, s);
     else if constexpr (LB::nc > 0) apply_on<LB, LA>(op, q, b, a, s);
 }
-// What node n needs for its boundary operators: its list with the values, and the fields of the merged
-// set.  The fused kernels load it before the node's pull, so that the operators wait for no memory
-// of their own.
+// What node n needs for its boundary operators: its list (NodeList) with the values, and the fields of the
+// merged set.  The fused kernels load it before the node's pull, so that the operators wait for no
+// memory of their own.  Four things keep the pull from waiting for it: the list's header stays as it was
+// loaded (taken apart inside the boundary lanes' branch, it was waited for there) and has no unused half
+// (whose register the pull's addresses took, and waited for), run_ops begins with a scheduling
+// barrier (or the header's first use is moved up between the pull's loads), and the arguments that the
+// branch needs are read together ahead of it (one after the other inside it, each was waited for).
+// FP64 step, us, before and after: heat sink 200x400 7.73 -> 7.63, 141x161 7.09 -> 6.82; ducts forward /
+// adjoint 113x36x43 17.75 / 21.07 -> 17.44 / 20.61, 96x96x48 33.5 / 38.9 -> 32.5 / 37.9.
 struct NodeOps {
-    NodeList o;
+    uint64_t list, form_count;
+    uint64_t w[2];
+    ListVals vals;
     NodeFields f;
+    __device__ __forceinline__ int count() const { return (int)((uint32_t)form_count & 0xffffffu); }
 };
 __device__ __forceinline__ NodeOps ops_of_node(const ProgView &pv, const Grid &g, int i, int j, int k, int n, int nd,
                                                bool wanted = true) {
     const int place = place_of(i, j, k, g.nx, g.ny, g.nz, nd);
-    NodeOps no{{-1, -1, 0, 0, {0, 0}, {}}, {}};
+    NodeOps no{0, 0, {0, 0}, {}, {}};
+    const FieldSet &fm = pv.fm;
+    asm volatile("" ::"s"(fm.rho), "s"(fm.ux), "s"(fm.uy), "s"(fm.uz), "s"(fm.tem), "s"(fm.diff), "s"(pv.place_list),
+                 "s"(pv.slot_list));
+    asm volatile("" ::"s"(pv.nsym), "s"(pv.fmerged), "s"(pv.has_diff), "s"(pv.latswap), "s"(pv.pull[0]),
+                 "s"(pv.pull[1]));
     if (wanted && ((pv.shared | pv.by_slot) >> place & 1u)) {
         const NodeList *e = pv.place_list + place;
         if (pv.by_slot >> place & 1u) e = pv.slot_list + boundary_slot(i, j, k, g.nx, g.ny, g.nz, nd);
         const uint64_t *p = reinterpret_cast<const uint64_t *>(e);
-        const uint64_t lf = gat(p, 0);
-        no.o.list = (int)(uint32_t)lf;
-        no.o.form = (int)(uint32_t)(lf >> 32);
-        no.o.count = (int)(uint32_t)gat(p, 1);
-        no.o.w[0] = gat(p, 2);
-        no.o.w[1] = gat(p, 3);
+        no.list = gat(p, 0);
+        no.form_count = gat(p, 1);
+        no.w[0] = gat(p, 2);
+        no.w[1] = gat(p, 3);
         const double *v = reinterpret_cast<const double *>(e) + 4;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) no.o.vals.a[c] = gat(v, c);
+        for (int c = 0; c < 4; ++c) no.vals.a[c] = gat(v, c);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) no.o.vals.b[c >> 1][c & 1] = gat(v, 4 + c);
-        no.f = load_fields(pv.fm, n);
+        for (int c = 0; c < 4; ++c) no.vals.b[c >> 1][c & 1] = gat(v, 4 + c);
+        no.f = load_fields(fm, n);
     }
     return no;
 }
@@ -214,32 +226,32 @@ struct NoSmooth {};  // SMOOTH operators do nothing
 // x-face nodes, on small grids the step waits for the wavefront with the most operators, and each of
 // them is a chain of branches, instruction fetches and divisions of some 0.15 us.  So the wavefront
 // takes the program's symbols that its lanes have one after the other, each once for all lanes that
-// have it, with scalar branches over one copy of the operators.  FP64 step, us, against each list's
-// sequence of words run by itself (and against each lane deciding for itself): 200x400 D2Q9 + D2Q5 heat
-// sink 7.7 (8.4; 7.8), smoothed 7.7 (7.9; 9.1), 101x101 6.3 (7.4; 6.8), 200x400 with six calls whose masks
-// are drawn per node 12.5 (91; 13.2); ducts forward / adjoint 44x40x30 11.0 / 11.9 (11.4 / 12.7; 11.1 /
-// 12.7), 113x36x43 17.8 / 21.1 (17.5 / 21.7; 18.0 / 20.9), 96x96x48 33.5 / 38.9 (34.2 / 39.8; 37.4 / 43.6).
-// Slower than each lane deciding for itself: 200x400 with two calls on all four faces 7.5 (8.2; 7.2) and
-// 101x101 with both bounce types, T and Q alternating along the walls 7.8 (9.7; 6.4).
+// have it, with scalar branches over one copy of the operators.  FP64 step, us, against each lane
+// deciding for itself, which walked every branch of a decision tree per operator in four inlined copies
+// after three dependent memory round trips: 200x400 D2Q9 + D2Q5 heat sink 7.6 (7.8), smoothed 7.7 (9.1),
+// 101x101 6.4 (6.8), 200x400 with six calls whose masks are drawn per node 12.6 (13.2; 91 with each list
+// run by itself); ducts forward / adjoint 44x40x30 10.9 / 11.6 (11.2 / 12.7), 113x36x43 17.4 / 20.6
+// (18.0 / 21.0), 96x96x48 32.5 / 37.9 (36.2 / 43.3).  Slower: 200x400 with two calls on all four faces 7.5
+// (7.2), and 101x101 with both bounce types, T and Q alternating along the walls 7.9 (6.4).
 // More than kSymbols symbols (11 calls that each reach six faces): position by position of the lists, at
 // each the words that the lanes have, each once.
 template <class LA, class LB, class Smooth = NoSmooth>
 __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, int n, double *a, double *b,
                                         Smooth &&smooth = Smooth{}) {
-    const NodeList &o = no.o;
+    __builtin_amdgcn_sched_barrier(0);
     const bool merged = pv.nsym > 0;
     unsigned long long all = 0;  // merged: the symbols left; else the lanes whose operator at position t is left
     int t = 0;
-    uint32_t word = (uint32_t)o.w[0] & 0xffffu, next = 0;
-    uint64_t w0 = o.w[0], w1 = o.w[1];
+    uint32_t word = (uint32_t)no.w[0] & 0xffffu, next = 0;
+    uint64_t w0 = no.w[0], w1 = no.w[1];
     if (merged) {
-        for (unsigned long long left = __ballot(o.w[0] != 0); left;) {
-            all |= readlane64(o.w[0], __builtin_ctzll(left));
-            left = __ballot((o.w[0] & ~all) != 0);
+        for (unsigned long long left = __ballot(no.w[0] != 0); left;) {
+            all |= readlane64(no.w[0], __builtin_ctzll(left));
+            left = __ballot((no.w[0] & ~all) != 0);
         }
         if (all) next = pv.sym[__builtin_ctzll(all) >> 1];
     } else {
-        all = __ballot(o.count > 0);
+        all = __ballot(no.count() > 0);
     }
     while (all) {
         uint32_t w;
@@ -250,20 +262,20 @@ __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, i
             all &= all - 1;
             w = next >> (bit & 1) * 16;  // loaded one operator ahead
             next = pv.sym[(all ? __builtin_ctzll(all) : bit) >> 1];
-            mine = o.w[0] >> bit & 1u;
+            mine = no.w[0] >> bit & 1u;
         } else {
             w = (uint32_t)__builtin_amdgcn_readlane((int)word, __builtin_ctzll(all));
-            mine = t < o.count && word == w;
+            mine = t < no.count() && word == w;
             all &= ~__ballot(mine);
         }
         const OpWord op = op_fields(w);
         if (mine) {
             const bool second = op.src == kFromSecond;
-            OpIn q{{o.vals.a[0], o.vals.a[1], o.vals.a[2], o.vals.a[3]},
-                   {second ? o.vals.b[1][0] : o.vals.b[0][0], second ? o.vals.b[1][1] : o.vals.b[0][1]}};
+            OpIn q{{no.vals.a[0], no.vals.a[1], no.vals.a[2], no.vals.a[3]},
+                   {second ? no.vals.b[1][0] : no.vals.b[0][0], second ? no.vals.b[1][1] : no.vals.b[0][1]}};
             if (__builtin_expect(op.src == kFromList, 0)) {
-                const int at = merged ? __popcll(o.w[0] & ((1ull << bit) - 1)) : t;
-                q = op_in(pv.list_ops[(size_t)o.list * pv.maxops + at]);
+                const int at = merged ? __popcll(no.w[0] & ((1ull << bit) - 1)) : t;
+                q = op_in(pv.list_ops[no.list + at]);
             }
             if constexpr (std::is_same_v<std::decay_t<Smooth>, NoSmooth>) {
                 apply_op<LA, LB>(op, q, a, b, pv, n, no.f);
@@ -276,11 +288,11 @@ __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, i
         }
         if (!merged && all == 0) {
             ++t;
-            all = __ballot(t < o.count);
+            all = __ballot(t < no.count());
             w0 = w0 >> 16 | w1 << 48;
             w1 >>= 16;
             word = (uint32_t)w0 & 0xffffu;
-            if (t >= kWordOps && t < o.count) word = pv.form_ops[(size_t)o.form * pv.maxops + t];
+            if (t >= kWordOps && t < no.count()) word = pv.form_ops[(no.form_count >> 24) + t];
         }
     }
 }
@@ -487,7 +499,7 @@ __device__ __forceinline__ void node_state(const S *sa, const S *sb, const Grid 
     coords(n, g, i, j, k);
     const NodeOps no = ops_of_node(pv, g, i, j, k, n, LA::nd, ops);
     pull_pair<LA, LB>(sa, sb, g, i, j, k, n, pv, a, b, Enc{}, Enc{});
-    if (no.o.form >= 0) {
+    if (no.count() > 0) {
         double xa[LA::nc], xb[LB::nc > 0 ? LB::nc : 1];
         dev_to_f64<LA>(a, xa, ea, oa);
         if constexpr (LB::nc > 0) dev_to_f64<LB>(b, xb, eb, ob);

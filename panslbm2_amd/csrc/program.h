@@ -83,7 +83,8 @@ struct alignas(16) ListVals {  // a list's values: one a, two b
 // A boundary node's operators and their values.  Lists that differ in their values only share a form
 // (the sequence of words and of the calls that recorded them).
 struct alignas(16) NodeList {
-    int list, form, count, pad;  // list, form: -1 without operators
+    uint64_t list;               // its first operator in ProgView::list_ops; ~0 without operators
+    uint64_t form_count;         // its first word in ProgView::form_ops << 24 | operators; 0 without
     uint64_t w[2];               // w[0]: which of ProgView::sym; without symbols: the first kWordOps operators, 16 bits each
     ListVals vals;
 };
@@ -107,15 +108,14 @@ struct ProgView {
     const NodeList *place_list;  // place -> its nodes' list, where they share one
     const NodeList *slot_list;   // boundary slot -> its list (size nslot)
     unsigned shared, by_slot;    // bit p: place p's nodes share a list of operators / have several lists
-    const Op *list_ops;         // list -> maxops operators (for values outside a NodeList)
-    const uint32_t *form_ops;   // form -> maxops words
+    const Op *list_ops;         // the lists' operators (for values outside a NodeList)
+    const uint32_t *form_ops;   // the forms' words
     // The program's symbols: its distinct (call, face, word), two words to an element, in the order of
     // the calls and their faces, which every list is in.  They ride in the kernel's arguments: from memory
     // their first use was a round trip of its own (101x101 D2Q9 + D2Q5 step 6.5 us against 6.3).
     // nsym 0: more than kSymbols.
     uint32_t sym[kSymbols / 2];
     int nsym;
-    int maxops;             // operators per list (0: no operators)
     int nentry;
     int nslot;
     FieldSet fs[kMaxFieldSets];
