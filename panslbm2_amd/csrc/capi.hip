@@ -784,11 +784,21 @@ int collide_call(lbm_program *P, lbm_lattice *p, lbm_lattice *q, std::initialize
     cl.eb = q ? q->enc() : lbm::Enc{};
     cl.g = p->grid();
     {
-        // non-temporal pulls (3D) where the step's populations, read and written, exceed what the
-        // 256 MB Infinity Cache keeps: measured faster from 184 MB (FP32, 128x128x64) up, slower
-        // at 156 MB (FP64, 96x96x48)
-        const size_t bytes = 2 * p->esize() * (size_t)p->N * (size_t)(p->nc + (q ? q->nc : 0));
-        cl.g.nt = (p->nd == 3 && bytes > ((size_t)160 << 20)) ? 1 : 0;
+        // non-temporal accesses (3D) where the step's populations, read and written, exceed what the 256 MB
+        // Infinity Cache keeps of them.  Forward + adjoint step of a duct, us: plain / loads / loads and stores
+        //   FP64  104x104x54 (206 MB) 91.3 / 97.9 / 101.3   112x112x48 (212 MB) 99.7 / 95.9 / 99.4
+        //         126x120x66 (351 MB) 172.6 / 154.5 / 157.5   128x126x68 (386 MB) 191.6 / 172.7 / 166.3
+        //         D3Q27 112x104x56 (355 MB) 197.9 / 179.8 / 179.1
+        //   FP32  140x128x64 (202 MB) 112.7 / 115.2 / 113.4   144x128x64 (208 MB) 119.3 / 115.8 / 114.9
+        //         160x128x64 (231 MB) 136.7 / 122.4 / 122.2   160x144x80 (324 MB) 195.5 / 179.1 / 169.6
+        //   FP16  160x144x80 (162 MB) 154.7 / 148.7 / 152.8   192x160x80 (216 MB) 213.8 / 178.9 / 181.8
+        //         256x176x80 (317 MB) 307.6 / 272.7 / 263.6
+        // The lines of narrower storage are lower because its coefficient and result fields are FP64 all the
+        // same, and take more of the cache beside as many bytes of populations.
+        const size_t bytes = 2 * p->esize() * (size_t)p->N * (size_t)(p->nc + (q ? q->nc : 0)), MiB = (size_t)1 << 20;
+        const bool loads = bytes > (p->prec == LBM_F16 ? 160 : 200) * MiB;
+        const bool stores = bytes > (p->prec == LBM_F64 ? 340 : 256) * MiB;
+        cl.g.nt = p->nd == 3 ? (loads ? lbm::kNtLoads : 0) | (stores ? lbm::kNtStores : 0) : 0;
     }
     cl.stream = C->stream;
     bool fused = false;

@@ -693,7 +693,7 @@ __device__ __forceinline__ void fused_block(const S *__restrict__ sa, const S *_
         coef = body.load(n);
     }
     body(fa, fb, coef, n, nb > 0, oa, ob);
-    if (LA::nd == 3 && g.nt) {
+    if (LA::nd == 3 && (g.nt & kNtStores)) {
         store_raw<LA, true>(da, g.N, n, fa);
         store_raw<LB, true>(db, g.N, n, fb);
     } else {

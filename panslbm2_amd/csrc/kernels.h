@@ -459,17 +459,17 @@ __device__ __forceinline__ int nboundary(int i, int j, int k, const Grid &g, int
     return c;
 }
 
-// Both lattices' pulls of node n.  With g.nt (3D launches whose populations do not fit the
-// Infinity Cache, set by the host) the pulled loads and the stores are non-temporal: a step reads
-// each source population once and writes each once, in an order the next step repeats, so lines
-// kept behind only displace each other.  D3Q15 + D3Q7 FP64 forward step: 128x128x64 (369 MB) 89 us
-// with plain accesses, 82 with the loads non-temporal, 79 with the stores too; at 96x96x48 (156 MB,
-// cache-resident) non-temporal stores cost 32 -> 39 us.  In 2D a source row is reused from L2 for the
-// rows beside it (4096^2 step 773 -> 837 us with the loads non-temporal), so 2D stays plain.
+// Both lattices' pulls of node n.  With kNtLoads the pulled loads are non-temporal, with kNtStores the
+// stores (3D launches whose populations do not fit the Infinity Cache; the host's rule has the sizes):
+// a step reads each source population once and writes each once, in an order the next step repeats, so
+// lines kept behind only displace each other.  D3Q15 + D3Q7 FP64 forward step: 128x128x64 (369 MB) 92 us
+// with plain accesses, 78 to 82 with the loads non-temporal, 76 to 80 with the stores too; 104x100x50
+// (183 MB, half of it cached from step to step) 36, 43 and 51 us.  In 2D a source row is reused from L2
+// for the rows beside it (4096^2 step 773 -> 837 us with the loads non-temporal), so 2D stays plain.
 template <class LA, class LB, class S, class R>
 __device__ __forceinline__ void pull_pair(const S *sa, const S *sb, const Grid &g, int i, int j, int k, int n,
                                           const ProgView &pv, R *a, R *b, const Enc &, const Enc &) {
-    if (LA::nd == 3 && g.nt) {
+    if (LA::nd == 3 && (g.nt & kNtLoads)) {
         load_pull<LA, true>(sa, g, i, j, k, n, pv.pull[0], a);
         load_pull<LB, true>(sb, g, i, j, k, n, pv.pull[1], b);
     } else {

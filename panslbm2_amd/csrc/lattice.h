@@ -180,9 +180,10 @@ __host__ __device__ __forceinline__ uint32_t div_by(uint32_t n, const FastDiv &f
     return (uint32_t((uint64_t(f.m) * n) >> 32) + n) >> f.s;
 }
 
+constexpr int kNtLoads = 1, kNtStores = 2;
 struct Grid {
     int nx, ny, nz, N;
-    int nt;  // 1: the fused kernels load the pulled populations non-temporal (set per launch)
+    int nt;  // kNtLoads, kNtStores: the fused 3D kernels' accesses that are non-temporal (set per launch)
     FastDiv by_nx, by_ny;
 };
 inline Grid make_grid(int nx, int ny, int nz, int N) {

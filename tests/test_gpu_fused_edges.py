@@ -195,6 +195,24 @@ def test_grid_beyond_the_cache_matches_eager(ctx):
     _same(run(FusedGpuBackend(ctx)), run(GpuBackend(ctx)))
 
 
+@pytest.mark.parametrize("dims", [(97, 89, 67), (101, 97, 73), (129, 101, 79)], ids=["plain", "loads", "loads-stores"])
+def test_grids_on_each_side_of_the_non_temporal_lines_match_eager(ctx, dims):
+    """204 MB of populations (plain accesses), 252 MB (loads non-temporal) and 362 MB (stores too)."""
+    from gpu_backend import FusedGpuBackend, GpuBackend
+
+    kinds = (_oracle.D3Q15, _oracle.D3Q7)
+
+    def run(b):
+        def ops(p, q, z, N, rng):
+            b.bc(p, np.ones(N, np.int32))
+            b.ad_set_t(q, np.ones(N, np.int32), np.full(N, 1.2), "vx", "vy", "vz")
+
+        return _run(b, kinds, dims, 8, False, 2, ops)
+
+    print("non-temporal lines", dims, flush=True)
+    _same(run(FusedGpuBackend(ctx)), run(GpuBackend(ctx)))
+
+
 @pytest.mark.parametrize("count", [0, 1, 1023, 1024, 1025, 5000])
 def test_gather_sum_is_the_serial_sum(ctx, count):
     """The sum in the order of the list, one addition after the other, over chunks in LDS."""
