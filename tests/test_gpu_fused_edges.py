@@ -421,3 +421,48 @@ def test_mixed_operator_lists_cost_little_more_than_uniform_ones(ctx, dims):
     mixed = step_us([rng.integers(0, top + 1, N).astype(np.int32) for top in (2, 1, 1, 1, 1, 2)])
     print("mixed lists", dims, "%.1f us, uniform %.1f us" % (mixed, uniform), flush=True)
     assert mixed <= 3.0 * uniform
+
+
+def test_eager_call_does_not_pay_for_the_fused_kernels_tables(ctx):
+    """An eager boundary call uploads its operators and 4 bytes per boundary slot; recording the same call
+    also builds what a fused collide reads, some 100 bytes per slot.  So the eager call, its kernel and
+    its wait included, takes less than three quarters of the recording's time (best of 15 each)."""
+    import time
+
+    import panslbm2_amd as pa
+    from panslbm2_amd import check, hptr
+
+    L, (lx, ly, lz) = ctx.lib, (96, 96, 48)
+    N = lx * ly * lz
+    p = pa.Lattice(ctx, pa.D3Q15, lx, ly, lz)
+    one, zero = ctx.array((N,), fill=1.0), ctx.array((N,), fill=0.0)
+    check(L.lbm_ns_initial_condition(p.h, one.ptr, zero.ptr, zero.ptr, zero.ptr))
+
+    def face(a, dt=np.float64):
+        return pa.to_face(pa.D3Q15, lx, ly, lz, a, dt)
+
+    inlet, u, z = face(np.arange(N) % lx == 0, np.int32), face(np.full(N, 0.03)), face(np.zeros(N))
+
+    def eager():
+        check(L.lbm_ns_set_u(p.h, hptr(inlet), hptr(u), hptr(z), hptr(z)))
+
+    def record():
+        prog = ctypes.c_void_p()
+        check(L.lbm_record_begin(ctx.h))
+        eager()
+        check(L.lbm_record_end(ctx.h, ctypes.byref(prog)))
+        L.lbm_program_destroy(prog)
+
+    def best(call):
+        b = np.inf
+        for _ in range(15):
+            ctx.sync()
+            t0 = time.perf_counter()
+            call()
+            ctx.sync()
+            b = min(b, time.perf_counter() - t0)
+        return 1e6 * b
+
+    e, r = best(eager), best(record)
+    print("eager call %.0f us, recorded %.0f us" % (e, r), flush=True)
+    assert e < 0.75 * r
