@@ -585,10 +585,9 @@ int build_fused(lbm_program *P, const std::vector<int2> &entry_ops, const std::v
         }
         P->smooth_in_pass_ok = true;
     } else if (any_smoothed && L->nd == 2) {
-        const int smoothed_bits = (P->smoothed[0] ? 1 : 0) | (P->smoothed[1] ? 2 : 0);
         for (const int4 &e : L->sm_corner) {
             int a = side_id(e.y), b = side_id(e.z);
-            sm_ents.push_back(make_int4(e.x, a, b, smoothed_bits));
+            sm_ents.push_back(make_int4(e.x, a, b, -1));
         }
         // A smoothing lane gives a corner, per lattice, either the neighbours' mean (smoothed) or its
         // own pull + operators: exact when no operator at a corner reads the other lattice.

@@ -614,10 +614,10 @@ __global__ void __launch_bounds__(kBlock) k_collide_inplace(S *a, S *b, Grid g, 
 // pass's own node_state: of a group of 4 (2D corner, 3D edge node) or 8 (3D corner) lanes those of
 // the face neighbours, and the smoothed node's own; the means then go across the group's lanes
 // (smooth_lanes_mean) and the own lane collides and stores.  A corner has a wavefront of its own, and
-// the 3D edge nodes are sorted by edge line, because a wavefront runs the operator lists of its lanes
-// one after the other (run_ops).  So no lane chains more than one state,
-// and a smoothed step needs no second stream (fork and join of one cost about 10 us of a step, and
-// its lanes chained up to three states: 128x128x64 FP64 step 104.0 us smoothed against 83.7 plain; 79 us now).
+// the 3D edge nodes are sorted by edge line, because a wavefront runs every operator that one of its
+// lanes has (run_ops).  So no lane chains more than one state, and a smoothed step needs no second stream
+// (fork and join of one cost about 10 us of a step, and its lanes chained up to three states: 128x128x64
+// FP64 step 104.0 us smoothed against 83.7 plain; 79 us now).
 // Exact because no smoothed node reads another: an edge node is the mean of two face nodes, and a
 // corner the mean of the three edge means beside it.
 template <class LA, class LB, class Body, class S>

@@ -92,7 +92,7 @@ struct alignas(16) NodeList {
 // (2D: always between in z); 13 is the interior.  Where all nodes of a place share one list, as those
 // of a wall or of a uniform inlet do, the fused kernels take it from a table of places, which stays
 // in the nearest cache; the nodes of other places look theirs up by slot.
-constexpr int kPlaces = 27, kInterior = 13;
+constexpr int kPlaces = 27;
 __host__ __device__ inline int place_of(int i, int j, int k, int nx, int ny, int nz, int nd) {
     const int x = i == 0 ? 0 : (i == nx - 1 ? 2 : 1), y = j == 0 ? 0 : (j == ny - 1 ? 2 : 1);
     const int z = nd == 2 ? 1 : (k == 0 ? 0 : (k == nz - 1 ? 2 : 1));

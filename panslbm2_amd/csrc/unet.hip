@@ -11,10 +11,10 @@
 //     the matrix core (8 channels of one tap) are one 16-byte load, of a brick staged in LDS;
 //   * the input gradient of a convolution is the same kernel run on the output gradient with the
 //     weights transposed and the taps mirrored;
-//   * the weight gradient reduces over voxels: tiles of the output gradient and of the shifted input
-//     are staged through LDS in [channel][voxel] order, so the matrix-core operands are again
-//     16-byte reads; partial sums per voxel range are reduced in a fixed order, so the gradient is
-//     deterministic;
+//   * the weight gradient reduces over voxels: tiles of the output gradient and of the input are
+//     staged through LDS as they lie in memory ([voxel][channel]), and the matrix core's operands
+//     (eight voxels of one channel) come from transposing LDS reads; partial sums per voxel range are
+//     reduced in a fixed order, so the gradient is deterministic;
 //   * Adam keeps FP32 master weights and repacks the bfloat16 copies after each update.
 //
 // The fields the solver uses are FP64 arrays; the network reads and writes them directly
@@ -60,10 +60,6 @@ __host__ __device__ inline float bf2f(bf16_t h) {
     return f;
 }
 __device__ inline bf16x8 ld8(const bf16_t *p) { return __builtin_bit_cast(bf16x8, *(const uint4 *)p); }
-
-__host__ __device__ inline int tap_dx(int t, int taps) { return taps == 27 ? t % 3 - 1 : 0; }
-__host__ __device__ inline int tap_dy(int t, int taps) { return taps == 27 ? (t / 3) % 3 - 1 : 0; }
-__host__ __device__ inline int tap_dz(int t, int taps) { return taps == 27 ? t / 9 - 1 : 0; }
 
 // ---- convolution (forward, and input gradient with transposed weights) ----------------------------
 // y[v][o] = bias[o] + sum_k w[o][k] x[v + off(tap)][ci], k = tap cin + ci.

@@ -257,7 +257,7 @@ class Heatsink3D(Heatsink2D):
         calls()
         prog = VP()
         check(self.L.lbm_record_end(self.ctx.h, ctypes.byref(prog)))
-        # every program here fuses (with SmoothCorner too: the edges and corners run after the pass)
+        # every program here fuses (with SmoothCorner too: the pass's first workgroups do the edges and corners)
         assert self.L.lbm_program_fusable(prog) == 1
         return prog
 

@@ -75,7 +75,7 @@ def test_heatsink3d_driver_matches_oracle(ctx, graphs, smooth, rho_in):
     """The 3D heat-sink driver (fused steps, graphs, field rebinding, boundary-only saves) against its
     CPU-oracle replica (tests/heatsink_oracle.py run3d): populations, fields and the objective
     value-identical, the sensitivity (pow-based in the reference) within 1e-12 relative.  Smoothed:
-    the edges and corners concurrently with the pass (second stream, inside the step graphs), and
+    the edges and corners inside the pass (its first workgroups), and
     after it from the pass's side states ("after")."""
     import heatsink_oracle
     import panslbm2_amd as pa
@@ -188,8 +188,8 @@ def test_design_loop_matches_oracle_loop(ctx):
 
 @pytest.mark.parametrize("prec_name", ["F32", "F16"])
 def test_smoothed_concurrent_equals_after_pass_reduced_precision(ctx, prec_name):
-    """With FP32 / FP16 population storage, the smoothed 3D steps in the concurrent form (second
-    stream, each lane rebuilding its face neighbours' states) and in the after-pass form (the states
+    """With FP32 / FP16 population storage, the smoothed 3D steps in the concurrent form (inside
+    the pass, each lane rebuilding one node's state) and in the after-pass form (the states
     the pass saved) give identical populations, fields and objective: both take the same FP64 means
     of the same face states."""
     import panslbm2_amd as pa
