@@ -164,7 +164,7 @@ struct lbm_program {
     struct Table {
         void *p = nullptr;
     };
-    Table d_slot_entry, d_entry_node, d_entry_ops, d_ops, d_form_ops, d_list_ops, d_slot_list, d_place_list;
+    Table d_slot_entry, d_entry_node, d_entry_ops, d_ops, d_list_words, d_list_ops, d_slot_list, d_place_list;
     unsigned shared_places = 0, slot_places = 0;  // ProgView::shared, by_slot
     DevBuf d_side;                      // smoothing after the pass, from side states
     Table d_side_of_slot, d_smoothed;
@@ -428,7 +428,7 @@ bool make_symbols(const std::vector<uint32_t> &form_ops, const std::vector<int> 
 // What the fused kernels read of a program, beside its entries.
 struct FusedTables {
     std::vector<Op> list_ops;
-    std::vector<uint32_t> form_ops;
+    std::vector<uint32_t> list_words;
     std::vector<lbm::NodeList> slot_list, place_list;
     std::vector<int> side_of_slot;
     std::vector<int4> sm_ents;
@@ -438,15 +438,15 @@ int build_fused(lbm_program *P, const std::vector<int2> &entry_ops, const std::v
                 const std::vector<int> &op_call, const std::vector<int> &slot_entry, FusedTables &f) {
     lbm_lattice *L = P->lat[0];
     // operator lists for the fused kernels: lists are stored once per distinct one (a face's nodes
-    // mostly share theirs), forms once per distinct sequence of operator words and calls
+    // mostly share theirs), forms (for the symbols) once per distinct sequence of operator words and calls
     int most = 0;
     for (const int2 &r : entry_ops) most = std::max(most, r.y);
     if (most >= 1 << 24) return fail(LBM_ERR_UNSUPPORTED, "more than 2^24 operators at one node");
     P->maxops = most;
     std::vector<Op> &list_ops = f.list_ops;
-    std::vector<uint32_t> &form_ops = f.form_ops;
+    std::vector<uint32_t> form_ops;
     std::vector<int> form_calls;
-    const lbm::NodeList no_list{~uint64_t(0), 0, {0, 0}, {}};
+    const lbm::NodeList no_list{0, {0, 0}, {}};
     std::vector<lbm::NodeList> &slot_list = f.slot_list, &place_list = f.place_list;
     slot_list.assign(P->nslot, no_list);
     place_list.assign(lbm::kPlaces, no_list);
@@ -481,15 +481,17 @@ int build_fused(lbm_program *P, const std::vector<int2> &entry_ops, const std::v
         }
         const lbm::ListVals vals = pack_list(one.data(), count, words.data());
         auto l = list_of.emplace(key_of(one), (int)list_of.size());
-        if (l.second) list_ops.insert(list_ops.end(), one.begin(), one.end());
-        auto f = form_of.emplace(key_of(words) + key_of(calls), (int)form_of.size());
-        if (f.second) {
+        if (l.second) {
+            list_ops.insert(list_ops.end(), one.begin(), one.end());
+            f.list_words.insert(f.list_words.end(), words.begin(), words.end());
+        }
+        auto form = form_of.emplace(key_of(words) + key_of(calls), (int)form_of.size());
+        if (form.second) {
             form_ops.insert(form_ops.end(), words.begin(), words.end());
             form_calls.insert(form_calls.end(), calls.begin(), calls.end());
         }
-        slot_form[s] = f.first->second;
-        lbm::NodeList so{(uint64_t)l.first->second * P->maxops,
-                         (uint64_t)f.first->second * P->maxops << 24 | (uint64_t)count, {0, 0}, vals};
+        slot_form[s] = form.first->second;
+        lbm::NodeList so{(uint64_t)l.first->second * P->maxops << 24 | (uint64_t)count, {0, 0}, vals};
         for (int t = 0; t < std::min(count, lbm::kWordOps); ++t) so.w[t / 4] |= (uint64_t)words[t] << (16 * (t % 4));
         slot_list[s] = so;
     }
@@ -512,8 +514,8 @@ int build_fused(lbm_program *P, const std::vector<int2> &entry_ops, const std::v
                     seen |= 1u << at;
                     place_list[at] = slot_list[s];
                     if (slot_form[s] >= 0) P->shared_places |= 1u << at;
-                } else if (slot_list[s].list != place_list[at].list ||
-                           slot_list[s].form_count != place_list[at].form_count) {
+                } else if (slot_list[s].list_count != place_list[at].list_count ||
+                           slot_list[s].w[0] != place_list[at].w[0]) {
                     P->slot_places |= 1u << at;
                 }
             }
@@ -667,7 +669,7 @@ int prog_upload(lbm_program *P) {
         {&P->d_entry_node, entry_node.data(), entry_node.size() * sizeof(int), 0},
         {&P->d_entry_ops, entry_ops.data(), entry_ops.size() * sizeof(int2), 0},
         {&P->d_ops, ops.data(), ops.size() * sizeof(Op), 0},
-        {&P->d_form_ops, f.form_ops.data(), f.form_ops.size() * sizeof(uint32_t), 0},
+        {&P->d_list_words, f.list_words.data(), f.list_words.size() * sizeof(uint32_t), 0},
         {&P->d_place_list, f.place_list.data(), f.place_list.size() * sizeof(lbm::NodeList), 0},
         {&P->d_list_ops, f.list_ops.data(), f.list_ops.size() * sizeof(Op), 0},
         {&P->d_slot_list, f.slot_list.data(), f.slot_list.size() * sizeof(lbm::NodeList), 0},
@@ -702,7 +704,7 @@ ProgView prog_view(const lbm_program *P) {
     v.by_slot = P->slot_places;
     v.slot_list = (const lbm::NodeList *)P->d_slot_list.p;
     v.list_ops = (const Op *)P->d_list_ops.p;
-    v.form_ops = (const uint32_t *)P->d_form_ops.p;
+    v.list_words = (const uint32_t *)P->d_list_words.p;
     v.nsym = (int)P->sym.size();
     for (int k = 0; k < v.nsym; ++k) v.sym[k >> 1] |= P->sym[k] << (k & 1) * 16;
     v.side_of_slot = P->n_smoothed > 0 ? (const int *)P->d_side_of_slot.p : nullptr;

@@ -173,16 +173,17 @@ __device__ __forceinline__ void apply_op(const OpWord &op, const OpIn &q, double
 // FP64 step, us, before and after: heat sink 200x400 7.73 -> 7.63, 141x161 7.09 -> 6.82; ducts forward /
 // adjoint 113x36x43 17.75 / 21.07 -> 17.44 / 20.61, 96x96x48 33.5 / 38.9 -> 32.5 / 37.9.
 struct NodeOps {
-    uint64_t list, form_count;
+    uint64_t list_count;
     uint64_t w[2];
     ListVals vals;
     NodeFields f;
-    __device__ __forceinline__ int count() const { return (int)((uint32_t)form_count & 0xffffffu); }
+    __device__ __forceinline__ size_t list() const { return list_count >> 24; }
+    __device__ __forceinline__ int count() const { return (int)((uint32_t)list_count & 0xffffffu); }
 };
 __device__ __forceinline__ NodeOps ops_of_node(const ProgView &pv, const Grid &g, int i, int j, int k, int n, int nd,
                                                bool wanted = true) {
     const int place = place_of(i, j, k, g.nx, g.ny, g.nz, nd);
-    NodeOps no{0, 0, {0, 0}, {}, {}};
+    NodeOps no{0, {0, 0}, {}, {}};
     const FieldSet &fm = pv.fm;
     asm volatile("" ::"s"(fm.rho), "s"(fm.ux), "s"(fm.uy), "s"(fm.uz), "s"(fm.tem), "s"(fm.diff), "s"(pv.place_list),
                  "s"(pv.slot_list));
@@ -192,11 +193,10 @@ __device__ __forceinline__ NodeOps ops_of_node(const ProgView &pv, const Grid &g
         const NodeList *e = pv.place_list + place;
         if (pv.by_slot >> place & 1u) e = pv.slot_list + boundary_slot(i, j, k, g.nx, g.ny, g.nz, nd);
         const uint64_t *p = reinterpret_cast<const uint64_t *>(e);
-        no.list = gat(p, 0);
-        no.form_count = gat(p, 1);
-        no.w[0] = gat(p, 2);
-        no.w[1] = gat(p, 3);
-        const double *v = reinterpret_cast<const double *>(e) + 4;
+        no.list_count = gat(p, 0);
+        no.w[0] = gat(p, 1);
+        no.w[1] = gat(p, 2);
+        const double *v = reinterpret_cast<const double *>(e) + offsetof(NodeList, vals) / sizeof(double);
 #pragma unroll
         for (int c = 0; c < 4; ++c) no.vals.a[c] = gat(v, c);
 #pragma unroll
@@ -243,7 +243,6 @@ __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, i
     unsigned long long all = 0;  // merged: the symbols left; else the lanes whose operator at position t is left
     int t = 0;
     uint32_t word = (uint32_t)no.w[0] & 0xffffu, next = 0;
-    uint64_t w0 = no.w[0], w1 = no.w[1];
     if (merged) {
         for (unsigned long long left = __ballot(no.w[0] != 0); left;) {
             all |= readlane64(no.w[0], __builtin_ctzll(left));
@@ -275,7 +274,7 @@ __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, i
                    {second ? no.vals.b[1][0] : no.vals.b[0][0], second ? no.vals.b[1][1] : no.vals.b[0][1]}};
             if (__builtin_expect(op.src == kFromList, 0)) {
                 const int at = merged ? __popcll(no.w[0] & ((1ull << bit) - 1)) : t;
-                q = op_in(pv.list_ops[no.list + at]);
+                q = op_in(pv.list_ops[no.list() + at]);
             }
             if constexpr (std::is_same_v<std::decay_t<Smooth>, NoSmooth>) {
                 apply_op<LA, LB>(op, q, a, b, pv, n, no.f);
@@ -289,10 +288,8 @@ __device__ __forceinline__ void run_ops(const ProgView &pv, const NodeOps &no, i
         if (!merged && all == 0) {
             ++t;
             all = __ballot(t < no.count());
-            w0 = w0 >> 16 | w1 << 48;
-            w1 >>= 16;
-            word = (uint32_t)w0 & 0xffffu;
-            if (t >= kWordOps && t < no.count()) word = pv.form_ops[(no.form_count >> 24) + t];
+            word = (uint32_t)((t < 4 ? no.w[0] : no.w[1]) >> 16 * (t & 3)) & 0xffffu;
+            if (t >= kWordOps && t < no.count()) word = pv.list_words[no.list() + t];
         }
     }
 }

@@ -55,7 +55,7 @@ constexpr size_t kXcdRemapMaxBytes = size_t(640) << 20;  // population bytes rea
 // (OpIn: a for the Navier-Stokes operators, b for the advection-diffusion ones), so that a boundary
 // node learns all it has to do with one load and has every operand with the next ones.
 enum OpSource : uint32_t { kFromFirst = 0, kFromSecond = 1, kFromList = 2 };
-constexpr int kWordOps = 8;  // operators in a NodeList of a program without symbols; a longer list's further words sit in form_ops
+constexpr int kWordOps = 8;  // operators in a NodeList of a program without symbols; a longer list's further words sit in list_words
 constexpr int kSymbols = 64;  // most symbols of a program (ProgView::sym)
 __host__ __device__ constexpr uint32_t op_word(uint32_t code, uint32_t face, uint32_t lat, uint32_t fset, uint32_t arg,
                                                uint32_t src) {
@@ -80,11 +80,9 @@ struct alignas(16) ListVals {  // a list's values: one a, two b
     double a[4], b[2][2];
 };
 
-// A boundary node's operators and their values.  Lists that differ in their values only share a form
-// (the sequence of words and of the calls that recorded them).
+// A boundary node's operators and their values.
 struct alignas(16) NodeList {
-    uint64_t list;               // its first operator in ProgView::list_ops; ~0 without operators
-    uint64_t form_count;         // its first word in ProgView::form_ops << 24 | operators; 0 without
+    uint64_t list_count;         // its first operator in ProgView::list_ops << 24 | operators; 0 without
     uint64_t w[2];               // w[0]: which of ProgView::sym; without symbols: the first kWordOps operators, 16 bits each
     ListVals vals;
 };
@@ -109,7 +107,7 @@ struct ProgView {
     const NodeList *slot_list;   // boundary slot -> its list (size nslot)
     unsigned shared, by_slot;    // bit p: place p's nodes share a list of operators / have several lists
     const Op *list_ops;         // the lists' operators (for values outside a NodeList)
-    const uint32_t *form_ops;   // the forms' words
+    const uint32_t *list_words; // their words
     // The program's symbols: its distinct (call, face, word), two words to an element, in the order of
     // the calls and their faces, which every list is in.  They ride in the kernel's arguments: from memory
     // their first use was a round trip of its own (101x101 D2Q9 + D2Q5 step 6.5 us against 6.3).
